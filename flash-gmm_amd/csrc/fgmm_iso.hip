@@ -16,6 +16,11 @@
 //               8-wave workgroup whose two waves per SIMD run a block's contraction
 //               and the previous block's epilogue in opposite orders (ping-pong), so
 //               one wave's VALU work runs under the other's matrix steps.
+//   iso_screen  the screened pass 1 of large calls, where the probe finds that most rows
+//               are near one component block: one bf16 step per chunk with a proven
+//               error bound tells near, faint and zero pairs apart; the gathering pass 2
+//               then forms logZ of a row near one block itself, and iso_lse_pipe runs
+//               the listed others.
 //   iso_lse     pass 1 of the stored plan up to D = 128 (two waves per SIMD), and at
 //               D = 192 and 256 on the default plan (one wave per SIMD, four chains in
 //               iso_lse_ctile's order), grid over row tiles.  Each wave keeps 32 rows
@@ -128,6 +133,8 @@ struct IsoPlan {
   int cpg;      // component blocks per pass-2 workgroup
   int ncg;      // groups of cpg component blocks (pass 2)
   int nslab;    // row slabs (pass 2)
+  int nslab_lj; // row slabs of the automatic stored branch's pass 2
+  int64_t rows_per_slab_lj;
   int rgroups;  // row groups per slab (partials per slab)
   int npart;    // nslab * rgroups
   int64_t rows_per_slab;
@@ -144,9 +151,70 @@ struct IsoPlan {
   bool bfw;     // bf16 contract above D = 256: stored log-joint, iso_bf16_*_wide
   bool bfneed;  // bf16 contract up to D = 128: need masks from pass 1, iso_bf16_gather in pass 2
                 // (or iso_bf16_accum where most pairs are needed)
+  bool screen;  // default plan up to D = 128, large calls: a probe selects the screened pass 1
+                // (iso_screen) on the device where most rows need one component block only
   size_t off_musw, off_mu3, off_kcblk, off_kclin, off_kcgat, off_rowstat, off_part_mu, off_part_nk,
-      off_part_sig, off_lj, off_ljmax, off_ljmask, off_ljcount, off_xsplit, off_zpair, off_probe, total;
+      off_part_sig, off_lj, off_ljmax, off_ljmask, off_ljcount, off_xsplit, off_zpair, off_probe, off_scop,
+      off_sce, off_list, off_single, off_faint, off_nearnk, total;
 };
+
+// The screened pass 1 (iso_screen): 16-dimension chunks of its approximate contraction
+// (the constants' chunk included), its LDS, and the calls it may take.
+constexpr int kScreenWaves = 4;     // waves per workgroup, 64 rows (two 32-row tiles) each
+constexpr int kScreenBlocks = 2;    // component blocks per LDS stage
+__host__ __device__ constexpr int screen_chunks(int DP) { return DP / 16 + 1; }
+__host__ __device__ constexpr int screen_rs(int DP) { return DP / 2 + 8; }   // bf16 row stride of the staging tile
+__host__ __device__ constexpr size_t screen_stage_bytes(int DP) {
+  return (size_t)kScreenBlocks * screen_chunks(DP) * 64 * 16;
+}
+// Per wave: half of a 32-row tile's columns in bf16 and their partial sums of squares.
+__host__ __device__ constexpr size_t screen_tile_bytes(int DP) {
+  return (size_t)32 * screen_rs(DP) * 2 + (size_t)32 * (DP / 8 + 1) * 4;
+}
+// The first stage's operands, then the staging tiles, which the second stage and the
+// rows' block bounds (bf16, 64 rows per wave) overlay once the rows are in registers.
+__host__ __device__ constexpr size_t screen_lds_bytes(int DP, int KB) {
+  const size_t a = kScreenWaves * screen_tile_bytes(DP);
+  const size_t b = screen_stage_bytes(DP) + (size_t)kScreenWaves * 64 * round_up(KB, 8) * 2;
+  return screen_stage_bytes(DP) + (a > b ? a : b);
+}
+// Calls whose pass 1 is worth screening: at least kScreenMinWork (32-row tile, block,
+// chunk) steps, below which the further launches cost more than the screening saves,
+// and at least 4 blocks (with one needed block a row, screening B blocks leaves 1/B of
+// the exact contraction); two workgroups per compute unit.
+constexpr int64_t kScreenMinWork = 500000;
+constexpr int64_t kMaxScreenLdx = (int64_t)4 << 20;   // 64 rows within 32-bit buffer offsets
+__host__ inline bool use_screen(int64_t N, int DP, int KB) {
+  return DP <= 128 && KB >= 4 && KB <= kProbeMaxKB && N < ((int64_t)1 << 31) - 256 &&
+         cdiv(N, 32) * KB * (DP / 16) >= kScreenMinWork && screen_lds_bytes(DP, KB) <= kMaxLds / 2;
+}
+
+// The screened pass 1 tells near pairs from faint ones.  A pair is near unless its
+// responsibility r provably has r, r ||x||, r ||x||^2 <= 2^-kNearGap; the faint pairs of
+// a component with Nk >= kNearNk then change none of its sums by a rounding (at most
+// N 2^-72 <= 2^-41, against 2^-24 of 2^-10), and a row's terms outside its near blocks
+// change no bit of its fp32 log-sum-exp (at most K 2^-72 of it).  So pass 2 takes the
+// near pairs, and then the faint ones of those blocks that hold a component with less.
+constexpr float kNearGap = 72.0f;
+constexpr float kNearNk = 0x1p-10f;
+
+// How a call's passes run.  The probe's last workgroup sums its counts and writes the
+// choice as one word, which every later kernel of the call reads with one scalar load
+// (each summing the counts for itself cost 0.5 us a kernel).
+enum IsoMode { kModeDefault = 0, kModeStored = 1, kModeScreen = 2 };
+__device__ __forceinline__ int iso_mode(const int* __restrict__ sel) { return sel ? *sel : kModeDefault; }
+// What the probe chooses from: up to max_multi sampled rows near several blocks, the
+// screened pass 1 (-1: never); else, from min_pairs needed pairs on, the stored branch if
+// the call has one.
+struct IsoRule {
+  int64_t max_multi, min_pairs;
+  int stored;
+};
+// The probe's part of the workspace: per sampled tile the needed pairs, then (from
+// kProbeTiles on) the rows near several blocks; then the choice and the count of
+// finished workgroups (zeroed by the prologue).
+constexpr int kProbeMode = 2 * kProbeTiles, kProbeDone = 2 * kProbeTiles + 1;
+constexpr size_t kIsoProbeBytes = (2 * kProbeTiles + 2) * sizeof(unsigned);
 
 // Pass 1 with need masks keeps a bf16 bound of each row's block maximum in LDS,
 // 2 bytes per (row, block) for its 4 waves, while the workgroup still fits twice in
@@ -199,7 +267,7 @@ __host__ __device__ constexpr int bf16_halves(int DP);
 __host__ inline int bf16_blocks_per_group(int DP, int KB);
 
 IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool bf16 = false,
-                  bool auto_lj = false) {
+                  bool auto_lj = false, bool allow_screen = true) {
   IsoPlan p{};
   p.N = N; p.K = K; p.D = D;
   p.DP = iso_padded_dim(D);
@@ -210,7 +278,8 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   p.need = !bf16 && !p.lj;
   p.autolj = p.need && auto_lj && p.DP <= 128 && N > 0 && p.KB > 0 && p.KB <= kProbeMaxKB &&
              (size_t)round_up(cdiv(N, 32), 8) * (size_t)p.KB * kLjTile * sizeof(float) <= kMaxLjBytes;
-  p.nprobe = p.autolj ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
+  p.screen = p.need && allow_screen && use_screen(N, p.DP, p.KB);
+  p.nprobe = (p.autolj || p.screen) ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
   p.ctile = p.need && p.DP > 128;
   p.rexact = (p.need || (p.lj && p.DP <= 128)) &&
              p.KB <= ((p.ctile && !lse_in_regs(p.DP)) ? ctile_need_exact_cap(ctile_blocks(p.DP))
@@ -257,11 +326,18 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double2));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
   } else if (p.need && N > 0 && p.KB > 0) {
-    // The gathering pass 2: eight waves per compute unit, two rounds at one wave per
-    // SIMD (one round where two fit).
-    const int64_t want = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
+    // The gathering pass 2: one round of waves, two per SIMD up to D = 64, one above
+    // (there, 64 slabs in two rounds took 0.266 ms at N=1M K=1024 D=128, 32 slabs take
+    // 0.247 ms).  The stored branch's pass 2 takes eight blocks per compute unit.
+    const int64_t rounds = p.DP <= 64 ? 8 : 4;
+    const int64_t want = gather_slab_count(cdiv(rounds * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double2));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
+    if (p.autolj) {
+      const int64_t wl = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
+      p.rows_per_slab_lj = cap_slab_rows(round_up(cdiv(N, wl), 32), sizeof(double2));
+      p.nslab_lj = (int)cdiv(N, p.rows_per_slab_lj);
+    }
   } else if (N > 0 && p.ncg > 0) {
     // One 8-wave workgroup per compute unit; the stored pass 2 up to D = 128 runs two
     // 4-wave workgroups on each.
@@ -277,7 +353,7 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     p.rows_per_slab = tile_rows;
     p.nslab = 0;
   }
-  p.npart = p.nslab * p.rgroups;
+  p.npart = std::max(p.nslab, p.nslab_lj) * p.rgroups;
   // The bf16 contract's need masks: each row's block maxima (bf16, 2 bytes per row and
   // block for the 4 waves of a pass-1 workgroup) must fit in LDS beside the stages.
   p.bfneed = bf16 && !p.bfw && p.DP <= 128 && p.KB > 0 &&
@@ -290,7 +366,18 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   p.off_kclin = off;   off = align256(off + (size_t)p.KP * 4 * sizeof(double));
   p.off_kcgat = off;   off = align256(off + (size_t)p.KP * 4 * sizeof(double));
   p.off_rowstat = off; off = align256(off + (size_t)(N > 0 ? N : 0) * 2 * sizeof(double));
-  p.off_part_mu = off; off = align256(off + (size_t)p.npart * p.KP * p.DP * sizeof(float));
+  p.off_part_mu = off;
+  if (p.screen) {
+    // Read by pass 1 only, so they share the space of the slab partials pass 2 writes
+    // after it: the screening operands and error bounds, and the list of rows that need
+    // several blocks (its length first).
+    size_t so = off;
+    p.off_scop = so; so = align256(so + (size_t)p.KB * screen_chunks(p.DP) * 64 * 16);
+    p.off_sce = so;  so = align256(so + (size_t)p.KB * sizeof(float4));
+    p.off_list = so; so = align256(so + 256 + (size_t)N * sizeof(int));
+    off = so;
+  }
+  off = std::max(off, align256(p.off_part_mu + (size_t)p.npart * p.KP * p.DP * sizeof(float)));
   p.off_part_nk = off; off = align256(off + (size_t)p.npart * p.KP * sizeof(float));
   p.off_part_sig = off; off = align256(off + (size_t)p.npart * p.KP * sizeof(float));
   // One log-joint tile per pass-1 wave (the grid's 32-row tiles, rounded up to 4),
@@ -308,105 +395,153 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   p.off_xsplit = off; off = align256(off + ptiles * ljt_xsplit_bytes(p.DP));
   p.off_zpair = off;  off = align256(off + ptiles * 32 * sizeof(float2));
   // The probe: sampled rows' block maxima, its counters and the selector word.
-  p.off_probe = off;  off = align256(off + (p.autolj ? probe_bytes() : 0));
+  p.off_probe = off;  off = align256(off + (p.nprobe > 0 ? kIsoProbeBytes : 0));
+  // The screened pass 1: one bit per row, set where the row is near one block only; the
+  // faint pairs' words; and pass 2's Nk partials before it adds faint pairs.
+  p.off_single = off; off = align256(off + (p.screen ? (size_t)cdiv(N, 64) * 2 * sizeof(unsigned) : 0));
+  p.off_faint = off;  off = align256(off + (p.screen ? ntile * sizeof(unsigned) : 0));
+  p.off_nearnk = off; off = align256(off + (p.screen ? (size_t)p.nslab * p.KP * sizeof(float) : 0));
   p.total = off;
   return p;
 }
 
 // ---------------------------------------------------------------------------
-// Prologue: one 64-thread block per 32-component block.
+// Prologue: one workgroup of kPrepWaves waves per 32-component block, the 16-dimension
+// chunks dealt to the waves (latency bound: with one wave walking all chunks it took
+// 16 us at K = 1024, D = 128).  Each chunk's squared norms stay in LDS for the
+// constants, which add them in chunk order.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void iso_prep(const float* __restrict__ mu, int64_t ldmu, int64_t K,
+constexpr int kPrepWaves = 8;
+constexpr int kPrepChunks = 16;   // chunks whose squared norms are kept at a time
+__global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restrict__ mu, int64_t ldmu, int64_t K,
                                                int D, int DP, const float* __restrict__ lss,
                                                const float* __restrict__ lpi, double2* __restrict__ kc_blk, double4* __restrict__ kc_lin,
                                                double4* __restrict__ kc_gat, bf16x8* __restrict__ mu3,
-                                               unsigned* __restrict__ ljcount) {
-  __shared__ double sC[32], sB[32];
+                                               unsigned* __restrict__ ljcount, bf16x8* __restrict__ sc_op,
+                                               float4* __restrict__ sc_e, unsigned* __restrict__ list_count,
+                                               unsigned* __restrict__ probe) {
+  __shared__ double sC[32], sB[32], sL[32], sO[kPrepChunks][32];
   const int kb = blockIdx.x;
-  const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Pass 1 counts the needed row pairs of the stored log-joint into these.
-  if (ljcount && kb == 0) ljcount[lane] = 0u;
+  if (ljcount && kb == 0 && wave == 0) ljcount[lane] = 0u;
+  if (list_count && kb == 0 && tid == 0) *list_count = 0u;
+  if (probe && kb == 0 && tid == 0) probe[kProbeDone] = 0u;
   const int64_t comp = (int64_t)kb * 32 + c;
   const bool valid = comp < K;
   const int NQ = DP / 16;
-  if (g == 0) {
-    double C = -INFINITY, b = 0.0, musq = 0.0, osum = 0.0;
-    if (valid) {
-      // ||mu||^2 as the sum of the chunks' squared norms, and the centring offsets
-      // of the bf16x6 pass 1, o_q = fp32(||mu chunk q||^2).  Each chunk's 16 loads
-      // are unrolled so they are in flight together (this kernel runs K / 32 blocks
-      // and is latency bound).
-      // Loads from clamped addresses with the value selected after, so no load waits
-      // behind a branch.
-#pragma unroll 2
-      for (int q = 0; q < NQ; ++q) {
-        double o = 0.0;
+  const float* mrow = mu + (valid ? comp : 0) * ldmu;
+  const double l = valid ? (double)lss[comp] : 0.0, lp = valid ? (double)lpi[comp] : 0.0;
+  const double b = valid ? 0.5 * exp(-l) * kLog2e : 0.0;
+  const float w2 = (float)(2.0 * b);
+  double musq = 0.0, osum = 0.0;
+  for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
+    // Three-way bf16 splits for the split-bf16 contraction, mu3[kb][q][s][lane] = split s
+    // of mu[comp][16q + 8g .. 16q + 8g + 7] (s < 3), and slot 3 = the splits of the
+    // centring offset -o_q, o_q = fp32(||mu chunk q||^2), in k slots 0..2 (lane-half 0,
+    // elements 0..2).  Loads from clamped addresses with the value selected after, so no
+    // load waits behind a branch.
+    const int q1 = q0 + kPrepChunks < NQ ? q0 + kPrepChunks : NQ;
+    for (int q = q0 + wave; q < q1; q += kPrepWaves) {
+      f32x4 v[4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int d = 16 * q + e;
-          const float f = mu[comp * ldmu + (d < D ? d : D - 1)];
-          const double v = d < D ? (double)f : 0.0;
-          o = fma(v, v, o);
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int d = 16 * q + 4 * j + e;
+          const float f = mrow[d < D ? d : D - 1];
+          v[j][e] = valid && d < D ? f : 0.0f;
         }
+      }
+      double o = 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = fma((double)v[j][e], (double)v[j][e], o);
+      }
+      const f32x4 lo = g == 0 ? v[0] : v[2], hi = g == 0 ? v[1] : v[3];
+      bf16x8 sp[3];
+      split3_bf16(lo, hi, sp);
+#pragma unroll
+      for (int t = 0; t < 3; ++t) mu3[(((int64_t)kb * NQ + q) * 4 + t) * 64 + lane] = sp[t];
+      if (sc_op) sc_op[((int64_t)kb * (NQ + 1) + q) * 64 + lane] = to_bf16x8(lo * w2, hi * w2);
+      f32x4 olo = zero4();
+      if (g == 0) olo.x = -(float)o;
+      bf16x8 so[3];
+      split3_bf16(olo, zero4(), so);
+      bf16x8 ov;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ov[e] = (__bf16)0.0f;
+      ov[0] = so[0][0];
+      ov[1] = so[1][0];
+      ov[2] = so[2][0];
+      mu3[(((int64_t)kb * NQ + q) * 4 + 3) * 64 + lane] = ov;
+      if (g == 0) sO[q - q0][c] = o;
+    }
+    __syncthreads();
+    if (tid < 32) {
+      // ||mu||^2 as the sum of the chunks' squared norms.
+      for (int q = q0; q < q1; ++q) {
+        const double o = sO[q - q0][c];
         musq += o;
         osum += (double)(float)o;
       }
-      const double l = (double)lss[comp];
-      const double lp = (double)lpi[comp];
-      b = 0.5 * exp(-l) * kLog2e;
-      C = (lp - 0.5 * (double)D * (kLog2Pi + l)) * kLog2e - b * musq;
     }
+    if (q1 < NQ) __syncthreads();
+  }
+  if (wave != 0) return;
+  double eW = 0.0, eB = 0.0, eC = 0.0;   // the component's part of the screening's error bound
+  if (g == 0) {
+    const double C = valid ? (lp - 0.5 * (double)D * (kLog2Pi + l)) * kLog2e - b * musq : -INFINITY;
     // The split-bf16 passes contract the centred cross term x.mu - sum_q o_q, so
     // their constant carries + 2 b sum_q o_q.
     sC[c] = valid ? C + 2.0 * b * osum : C;
     sB[c] = b;
+    sL[c] = C;
     kc_lin[comp] = make_double4(C, b, musq, 0.0);
     // The gathering passes 2 take the centred constant and, for
     // ||x - mu||^2 = ||x||^2 - 2 (x.mu - sum_q o_q) + (||mu||^2 - 2 sum_q o_q), the last term.
     kc_gat[comp] = make_double4(sC[c], b, musq - 2.0 * osum, 0.0);
-  }
-  // The same chunks as three-way bf16 splits for the bf16x6 pass 1,
-  // mu3[kb][q][s][lane] = split s of mu[comp][16q + 8g .. 16q + 8g + 7] (s < 3), and
-  // slot 3 = the splits of -o_q in k slots 0..2 (lane-half 0, elements 0..2).
-  for (int q = 0; q < NQ; ++q) {
-    f32x4 lo = zero4(), hi = zero4();
-    const int d0 = 16 * q + 8 * g;
     if (valid) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float a = mu[comp * ldmu + (d0 + e < D ? d0 + e : D - 1)];
-        const float b = mu[comp * ldmu + (d0 + 4 + e < D ? d0 + 4 + e : D - 1)];
-        lo[e] = d0 + e < D ? a : 0.0f;
-        hi[e] = d0 + 4 + e < D ? b : 0.0f;
-      }
+      eW = 2.0 * b * sqrt(musq);
+      eB = b;
+      eC = C == -INFINITY ? 0.0 : fabs(C);
+      // A component whose constants are not ordinary numbers gets no finite bound: every
+      // row then needs its block, and the exact passes see it.
+      if (!(eW < 1e30) || !(eB < 1e30) || !(eC < 1e30)) eC = INFINITY;
     }
-    bf16x8 sp[3];
-    split3_bf16(lo, hi, sp);
-#pragma unroll
-    for (int t = 0; t < 3; ++t) mu3[(((int64_t)kb * NQ + q) * 4 + t) * 64 + lane] = sp[t];
-    f32x4 olo = zero4();
-    if (valid && g == 0) {
-      double o = 0.0;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int d = 16 * q + e;
-        const float f = mu[comp * ldmu + (d < D ? d : D - 1)];
-        const double v = d < D ? (double)f : 0.0;
-        o = fma(v, v, o);
-      }
-      olo.x = -(float)o;
-    }
-    bf16x8 so[3];
-    split3_bf16(olo, zero4(), so);
-    bf16x8 ov;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ov[e] = (__bf16)0.0f;
-    ov[0] = so[0][0];
-    ov[1] = so[1][0];
-    ov[2] = so[2][0];
-    mu3[(((int64_t)kb * NQ + q) * 4 + 3) * 64 + lane] = ov;
   }
-  __syncthreads();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
+  if (sc_op) {
+    // The screening's constants chunk, -b ||x||^2 + C as products of three-way bf16
+    // splits (iso_screen's row operand holds the matching splits of ||x||^2 and ones),
+    // and the block's error bound |approximate - exact log-joint| <=
+    // sc_e.x ||x|| + sc_e.y ||x||^2 + sc_e.z (iso_screen).
+    f32x4 lo = zero4();
+    const double C = sL[c];
+    lo.x = -(float)sB[c];
+    lo.y = !valid || C == -INFINITY ? -1e30f : (float)C;
+    bf16x8 sp[3], a;
+    split3_bf16(lo, zero4(), sp);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = (__bf16)0.0f;
+    if (g == 0) {   // with ||x||^2's s1, s2, s3, s1, s2, s1
+      a[0] = sp[0][0]; a[1] = sp[0][0]; a[2] = sp[0][0];
+      a[3] = sp[1][0]; a[4] = sp[1][0]; a[5] = sp[2][0];
+    } else {
+      a[0] = sp[0][1]; a[1] = sp[1][1]; a[2] = sp[2][1];
+    }
+    sc_op[((int64_t)kb * (NQ + 1) + NQ) * 64 + lane] = a;
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) {
+      eW = fmax(eW, __shfl_xor(eW, o));
+      eB = fmax(eB, __shfl_xor(eB, o));
+      eC = fmax(eC, __shfl_xor(eC, o));
+    }
+    if (lane == 0)
+      sc_e[kb] = make_float4((float)(eW * 0x1.06p-8), (float)(eB * 0x1p-14), (float)(eC * 0x1p-14 + 1.0), 0.0f);
+  }
   // Constants in accumulator-register order: entry (g, i) is component acc_row(i, g).
   {
     const int i = lane & 15, gg = (lane >> 4) & 1;
@@ -626,6 +761,10 @@ void iso_lse(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
 // ---------------------------------------------------------------------------
 constexpr int kPipeWaves = 8;
 constexpr int kPipeThreads = 64 * kPipeWaves;
+constexpr int kListBase = 64;   // ints before the first row of iso_screen's list (entry 0: its length)
+// Lists of up to this many 32-row workgroups per compute unit run one tile per workgroup
+// (a round of them takes about a quarter of a round of 256-row workgroups).
+constexpr int kFewRounds = 3;
 
 // iso_lse_pipe's grid: whole rounds of 8-tile workgroups (one per compute unit),
 // then the tiles left in groups of `small`, one group per compute unit.
@@ -657,8 +796,8 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
                   const bf16x8* __restrict__ mu3, const double2* __restrict__ kc_blk, int KB,
                   float* __restrict__ logZ, double2* __restrict__ rowstat, unsigned* __restrict__ ljmask,
                   unsigned* __restrict__ ljcount, int dense, float* __restrict__ lj,
-                  ProbeSel probe, __bf16* __restrict__ xsplit, float2* __restrict__ zpair, int64_t full,
-                  int small) {
+                  const int* __restrict__ sel, __bf16* __restrict__ xsplit, float2* __restrict__ zpair, int64_t full,
+                  int small, const int* __restrict__ list, int64_t few) {
   static_assert(DP <= 128, "pipelined pass 1 keeps all of a row's splits in registers");
   constexpr int NQ = DP / 16;
   constexpr int BLK = NQ * 4 * 64;        // bf16x8 per 32-component block
@@ -676,15 +815,95 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
-  const bool tail = (int64_t)blockIdx.x >= full;
+  const int mode = iso_mode(sel);
+  // After the screening (iso_screen) only the rows on its list are left, the listed rows
+  // taking the place of rows 0 .. n - 1; it has written the need masks.
+  const bool listed = mode == kModeScreen;
+  const int64_t nrow = listed ? (int64_t)(unsigned)list[0] : N;
+  const bool tail = !listed && (int64_t)blockIdx.x >= full;
   const int64_t tile = tail ? full * kPipeWaves + ((int64_t)blockIdx.x - full) * small + wave
                             : (int64_t)blockIdx.x * kPipeWaves + wave;
-  const bool idle = tail && (wave >= small || tile * 32 >= N);
-  const int64_t row = tile * 32 + c;
-  const bool valid = !idle && row < N;
+  if (listed && nrow <= few) {
+    // A short list: a workgroup per 32 rows, whose waves contract eight blocks at a time
+    // and then take turns to add theirs to the row's running (max, sum), in block order:
+    // the same operations on the same values, so the same bits.  (117 listed rows of
+    // N=1M K=1024 D=128 took 60 us as one workgroup of 256 rows, 8 us here.)
+    if ((int64_t)blockIdx.x * 32 >= nrow) return;   // uniform over the workgroup
+    double* smx = reinterpret_cast<double*>(lds_raw);          // [64] the lane's running max
+    float* ssm = reinterpret_cast<float*>(smx + 64);           // [64] and sum
+    const bool ok = (int64_t)blockIdx.x * 32 + c < nrow;
+    const int64_t r = ok ? (int64_t)list[kListBase + (int64_t)blockIdx.x * 32 + c] : 0;
+    bf16x8 xb[NQ][3];
+    double xsq = 0.0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int d0 = 16 * q + 8 * g;
+      const f32x4 lo = load_row4(X, ldx, r, d0, D, ok), hi = load_row4(X, ldx, r, d0 + 4, D, ok);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xsq = fma((double)lo[e], (double)lo[e], xsq);
+        xsq = fma((double)hi[e], (double)hi[e], xsq);
+      }
+      split3_bf16(lo, hi, xb[q]);
+    }
+    xsq += __shfl_xor(xsq, 32);
+    const bf16x8 ones = x6c_ones(lane);
+    double mx = -INFINITY;
+    float sm = 0.0f;
+    for (int kb0 = 0; kb0 < KB; kb0 += kPipeWaves) {
+      const int kb = kb0 + wave;
+      double ll[16], bm = -INFINITY;
+      if (kb < KB) {
+        const bf16x8* mp = mu3 + (int64_t)kb * BLK + lane;
+        const f32x16 xm = x6c_tile<NQ, kIsoChains>([&](int q, int t) { return mp[(q * 4 + t) * 64]; }, xb, ones);
+        const double2* kp = kc_blk + (int64_t)kb * 32 + g * 16;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const double2 cb = kp[i];
+          ll[i] = fma(-cb.y, fma(-2.0, (double)xm[i], xsq), cb.x);
+          bm = fmax(bm, ll[i]);
+        }
+      }
+      for (int w = 0; w < kPipeWaves && kb0 + w < KB; ++w) {
+        if (w == wave) {
+          if (kb > 0) {
+            mx = smx[lane];
+            sm = ssm[lane];
+          }
+          const double mn = fmax(mx, bm);
+          const double ms = (mn == -INFINITY) ? 0.0 : mn;
+          float acc = sm * fast_exp2((float)(mx - ms));
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc += fast_exp2((float)(ll[i] - ms));
+          smx[lane] = mn;
+          ssm[lane] = acc;
+        }
+        lds_barrier();
+      }
+    }
+    if (wave == 0) {
+      mx = smx[lane];
+      sm = ssm[lane];
+      const double mo = __shfl_xor(mx, 32);
+      const float so = __shfl_xor(sm, 32);
+      const double mn = fmax(mx, mo);
+      const double ms = (mn == -INFINITY) ? 0.0 : mn;
+      const float tot = sm * fast_exp2((float)(mx - ms)) + so * fast_exp2((float)(mo - ms));
+      const double lz2 = mn + (double)log2f(tot);
+      if (ok && g == 0) {
+        rowstat[r] = make_double2(xsq, lz2);
+        if (logZ) logZ[r] = (float)(lz2 * kLn2);
+      }
+    }
+    return;
+  }
+  if (listed && (int64_t)blockIdx.x * kPipeWaves * 32 >= nrow) return;   // uniform over the workgroup
+  const bool idle = (tail && wave >= small) || ((tail || listed) && tile * 32 >= nrow);
+  const bool valid = !idle && tile * 32 + c < nrow;
+  const int64_t row = (listed && valid) ? (int64_t)list[kListBase + tile * 32 + c] : tile * 32 + c;
   // Whether this call stores the log-joint: never without lj, always without a
   // probe, else as the probe's counts (written before this kernel) say.
-  const bool store = lj != nullptr && (probe.count == nullptr || probe_selects(probe));
+  const bool store = lj != nullptr && (sel == nullptr || mode == kModeStored);
 
   // Block kb's operands into mu buffer kb & 1, its constants into kc buffer kb % 3.
   // A lane whose piece lies past the block (BLK not a multiple of the workgroup's
@@ -790,7 +1009,7 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   // The need bound of block kb: kept in LDS (REXACT) or tested against the running
   // max.  Both half-waves store the row's bound (the same value); the mask word goes
   // out through a buffer store whose offset is out of range on every lane but 0.
-  const buf_rsrc mask_r = make_rsrc(ljmask + tile * KB, (uint32_t)(KB * sizeof(unsigned)));
+  const buf_rsrc mask_r = make_rsrc(ljmask + tile * KB, listed ? 0u : (uint32_t)(KB * sizeof(unsigned)));
   const int mask_off = buf_off(lane == 0 ? 0 : kBufOob);
   auto put_need = [&](int kb, float R) {
     if constexpr (REXACT) {
@@ -875,6 +1094,7 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
       zpair[tile * 32 + c] = make_float2(zh, zl);
     }
   }
+  if (listed) return;
   if constexpr (REXACT) {
     // Each lane reads back the bounds it wrote itself.
     const unsigned short* rm = rmax_l + wave * KB * 32 + c;
@@ -908,11 +1128,15 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
                                                                     int64_t N, int D,
                                                                     const bf16x8* __restrict__ mu3,
                                                                     const double2* __restrict__ kc_blk, int KB,
-                                                                    int ntile, unsigned* __restrict__ count) {
+                                                                    const float4* __restrict__ sc_e, int ntile,
+                                                                    IsoRule rule, unsigned* __restrict__ count) {
   constexpr int NQ = DP / 16;
   constexpr int BLK = NQ * 4 * 64;
-  __shared__ float rmax[kProbeMaxKB * 32];
-  __shared__ unsigned part[kProbeWaves];
+  // The rows' block maxima and the screening's error bounds, the rows' maxima over the
+  // blocks (R, and R less its bound) by 32 threads each, and their kept blocks.
+  __shared__ float rmax[kProbeMaxKB * 32], rerr[kProbeMaxKB * 32];
+  __shared__ float rowR[32][33], rowL[32][33];
+  __shared__ unsigned part[kProbeWaves], blocks[32];
   const int s = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -921,22 +1145,31 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
   const int64_t row = tile * 32 + c;
   const bool valid = row < N;
 
-  bf16x8 xh[NQ];
-  double xsq = 0.0;
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int d0 = 16 * q + 8 * g;
-    const f32x4 lo = load_row4(X, ldx, row, d0, D, valid), hi = load_row4(X, ldx, row, d0 + 4, D, valid);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      xsq = fma((double)lo[e], (double)lo[e], xsq);
-      xsq = fma((double)hi[e], (double)hi[e], xsq);
-    }
-    xh[q] = to_bf16x8(lo, hi);
+  // The tile's rows, loaded once by all waves (each loading them in operand order took
+  // most of this kernel's time) and passed through LDS in bf16.
+  constexpr int V4 = DP / 4, XRS = DP + 8;
+  __shared__ __align__(16) __bf16 xt[32 * XRS];
+  __shared__ float sq[32][V4 + 1];
+  for (int idx = tid; idx < 32 * V4; idx += 64 * kProbeWaves) {
+    const int rr = idx / V4, v = idx % V4;
+    const int64_t xr = tile * 32 + rr;
+    const f32x4 x = load_row4(X, ldx, xr, 4 * v, D, xr < N);
+    const uint2 w = {bf16_pair(f32x2{x.x, x.y}), bf16_pair(f32x2{x.z, x.w})};
+    *reinterpret_cast<uint2*>(xt + rr * XRS + 4 * v) = w;
+    sq[rr][v] = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w)));
   }
-  xsq += __shfl_xor(xsq, 32);
+  __syncthreads();
+  bf16x8 xh[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) xh[q] = *reinterpret_cast<const bf16x8*>(xt + c * XRS + 16 * q + 8 * g);
+  float xs = 0.0f;
+#pragma unroll
+  for (int v = 0; v < V4; ++v) xs += sq[c][v];
+  const double xsq = (double)xs;
+  const float nx = sqrtf(xs);
   const bf16x8 ones = x6c_ones(lane);
   for (int kb = wave; kb < KB; kb += kProbeWaves) {
+    const float4 e = sc_e ? sc_e[kb] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const bf16x8* mp = mu3 + (int64_t)kb * BLK + lane;
     bf16x8 a0[NQ], a3[NQ];
 #pragma unroll
@@ -959,15 +1192,38 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
       bm = fmax(bm, fma(-cb.y, fma(-2.0, (double)xm, xsq), cb.x));
     }
     const float R = lj_row_max(bm);
-    if (g == 0) rmax[kb * 32 + c] = R;
+    if (g == 0) {
+      rmax[kb * 32 + c] = R;
+      rerr[kb * 32 + c] = sc_e ? fmaf(e.x, nx, fmaf(e.y, xs, e.z)) : 0.0f;
+    }
   }
+  if (tid < 32) blocks[tid] = 0u;
   __syncthreads();
-  // Row c's maximum and needed blocks; the waves split the blocks again.
-  unsigned need = 0;
-  if (g == 0 && valid) {
-    float M = -INFINITY;
-    for (int kb = 0; kb < KB; ++kb) M = fmaxf(M, rmax[kb * 32 + c]);
-    for (int kb = wave; kb < KB; kb += kProbeWaves) need += (rmax[kb * 32 + c] - M >= -kLjNeedGap) ? 1u : 0u;
+  // Each row's largest maximum R and largest lower bound L: 32 threads a row.
+  const int t32 = tid >> 5;
+  float R = -INFINITY, L = -INFINITY;
+  for (int kb = t32; kb < KB; kb += 32) {
+    const float r = rmax[kb * 32 + c];
+    R = fmaxf(R, r);
+    L = fmaxf(L, r - rerr[kb * 32 + c]);
+  }
+  rowR[t32][c] = R;
+  rowL[t32][c] = L;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 32; ++j) {
+    R = fmaxf(R, rowR[j][c]);
+    L = fmaxf(L, rowL[j][c]);
+  }
+  unsigned need = 0, kept = 0;
+  if (valid) {
+    const float near_gap = fminf(kLjNeedGap, kNearGap + 2.0f * log2f(1.0f + nx));
+    for (int kb = t32; kb < KB; kb += 32) {
+      const float r = rmax[kb * 32 + c];
+      need += (r - R >= -kLjNeedGap) ? 1u : 0u;
+      kept += !(r + rerr[kb * 32 + c] - L < -near_gap) ? 1u : 0u;   // iso_screen's near blocks
+    }
+    if (sc_e && kept != 0) atomicAdd(blocks + c, kept);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) need += __shfl_xor(need, o);
@@ -978,8 +1234,276 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
     for (int w = 0; w < kProbeWaves; ++w) tot += part[w];
     count[s] = tot;
   }
+  if (wave != 0) return;
+  const uint64_t multi = __builtin_amdgcn_ballot_w64(sc_e != nullptr && lane < 32 && blocks[c] > 1u);
+  unsigned done = 0;
+  if (lane == 0) {
+    count[kProbeTiles + s] = (unsigned)__builtin_popcountll(multi);
+    __threadfence();
+    done = atomicAdd(count + kProbeDone, 1u);
+  }
+  if (__builtin_amdgcn_readfirstlane(done) != (unsigned)ntile - 1u) return;
+  // The last workgroup to finish: every count is visible to device-scope loads.
+  __threadfence();
+  uint64_t t = 0;
+  if (lane < ntile)
+    t = ((uint64_t)__hip_atomic_load(count + kProbeTiles + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) << 32) |
+        __hip_atomic_load(count + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);   // at most 2^20 pairs and 2^11 rows
+  if (lane == 0)
+    count[kProbeMode] = (int64_t)(t >> 32) <= rule.max_multi ? kModeScreen
+                        : rule.stored && (int64_t)(t & 0xffffffffu) >= rule.min_pairs ? kModeStored : kModeDefault;
 }
 
+
+// ---------------------------------------------------------------------------
+// The screened pass 1 (default plan up to D = 128, large calls, selected by the probe).
+//
+// Where clusters are separated, the exact contraction (seven bf16 steps per 16
+// dimensions) of nearly every (row, block) pair only proves that its responsibilities
+// are zero.  This kernel proves it with one step: the approximate log-joint
+//   a_nk = sum_d bf16(x_d) bf16(2 b_k mu_kd) - b_k ||x||^2 + C_k
+// comes straight out of the matrix cores (the constants are one more chunk of three-way
+// splits), a row's block maximum is a maximum of accumulators, and
+//   |a_nk - ll2_nk| <= E = sc_e.x ||x|| + sc_e.y ||x||^2 + sc_e.z   (iso_prep, per block):
+// each operand is rounded by at most 2^-9 of itself, so the products err by 2^-8 ||x||
+// ||2 b mu|| (Cauchy-Schwarz; 0x1.06p-8 with the second-order and accumulation terms),
+// the constants' dropped split products and fp32 sums by under 2^-14 (b ||x||^2 + |C|).
+// With L the largest a - E over all blocks (logZ2 >= L), a block with a + E < L -
+// kLjNeedGap holds only responsibilities that are exactly zero, as the need masks of the
+// exact pass 1 state; the other blocks get their need bit.  Not-finite values make E
+// or a infinite or NaN, and the comparison then keeps the block.
+// A row with one needed block needs no other block for logZ either: the gathering pass
+// 2 forms its log-sum-exp there (`single` bit).  The rest go on a list, which
+// iso_lse_pipe runs through the exact pass 1.
+//
+// Bound: matrix steps and VALU, which mostly add up on a SIMD: at D = 128, 9 matrix
+// steps (288 cycles) and about 25 VALU instructions per (32 rows, block); matrix steps
+// alone 51% of its cycles.  Each operand read from LDS serves two 32-row tiles.  Rows
+// are read in whole lines and transposed through LDS (the exact pass reads 16-byte
+// pieces of 32 rows per instruction, which at this kernel's length would bound it).
+// N=1M K=1024 D=128 clustered: 0.27 ms, and pass 1 and 2 with it 0.55 ms instead of
+// 1.73 ms (drop-in call 1.73 -> 0.58 ms); N=400K K=300 D=50: call 0.51 -> 0.28 ms.
+// ---------------------------------------------------------------------------
+template <int DP>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * kScreenWaves, 64 * kScreenWaves),
+                          amdgpu_waves_per_eu(3, 3)))
+void iso_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ sc_op,
+                const float4* __restrict__ sc_e, int KB, unsigned* __restrict__ need,
+                unsigned* __restrict__ faint, unsigned* __restrict__ single, int* __restrict__ list, const int* __restrict__ sel) {
+  constexpr int NC = screen_chunks(DP), NQ = DP / 16;
+  constexpr int BLK = NC * 64;                    // bf16x8 per block
+  constexpr int STG = kScreenBlocks * BLK;        // bf16x8 per stage
+  constexpr int RS = screen_rs(DP), V4 = DP / 8;  // float4 per half row
+  constexpr int LPT = 32 * V4 / 64;               // float4 per lane and half tile
+  if (iso_mode(sel) != kModeScreen) return;
+
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  bf16x8* const op0 = reinterpret_cast<bf16x8*>(lds_raw);
+  unsigned char* const rest = lds_raw + screen_stage_bytes(DP);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, g = lane >> 5;
+  unsigned short* const ub_l = reinterpret_cast<unsigned short*>(rest + screen_stage_bytes(DP)) +
+                               wave * 64 * ((KB + 7) & ~7) + lane;
+
+  // Stage st (blocks kScreenBlocks st ..) into operand buffer st & 1, in 1 KB pieces.
+  auto fetch = [&](int st) {
+    const int nb = KB - st * kScreenBlocks < kScreenBlocks ? KB - st * kScreenBlocks : kScreenBlocks;
+    const DmaSrc r = dma_src(sc_op + (int64_t)st * STG, (uint32_t)(nb * BLK * (int)sizeof(bf16x8)));
+    bf16x8* dst = (st & 1) ? reinterpret_cast<bf16x8*>(rest) : op0;
+    for (int p = wave; p < nb * NC; p += kScreenWaves)
+      lds_dma16(r, dst + p * 64, lane * (int)sizeof(bf16x8), p * 64 * (int)sizeof(bf16x8));
+  };
+  const int64_t row0 = (int64_t)blockIdx.x * (64 * kScreenWaves) + wave * 64;
+  const int64_t row = row0 + lane;
+  fetch(0);
+
+  // The wave's two 32-row tiles in halves of the columns: whole 128-byte lines per load,
+  // rounded to bf16 into the wave's staging tile and read back as B operands; ||x||^2
+  // from the fp32 values.  The next half's loads are in flight meanwhile.
+  __bf16* const xt = reinterpret_cast<__bf16*>(rest + wave * screen_tile_bytes(DP));
+  float* const sq = reinterpret_cast<float*>(xt + 32 * RS);
+  bf16x8 xb[2][NC];
+  float xs = 0.0f;   // of the lane's own row, row0 + lane
+  f32x4 raw[2][LPT];
+  // Rows past N lie past the resource and read zeros, as do columns from D on.
+  const int64_t rows = N - row0 < 64 ? (N - row0 > 0 ? N - row0 : 0) : 64;
+  const buf_rsrc xr = make_rsrc(X + (rows > 0 ? row0 * ldx : 0), (uint32_t)(rows * ldx * (int64_t)sizeof(float)));
+  const int rbytes = (int)ldx * (int)sizeof(float);
+  auto load = [&](int u, f32x4 (&r)[LPT]) __attribute__((always_inline)) {
+    if constexpr (64 % V4 == 0) {   // a lane's column is the same in every load
+      const int d0 = (u & 1) * (DP / 2) + 4 * (lane % V4);
+      int off = d0 < D ? (32 * (u >> 1) + lane / V4) * rbytes + d0 * 4 : kBufOob;
+#pragma unroll
+      for (int i = 0; i < LPT; ++i) {
+        r[i] = buf_load_f32x4(xr, buf_off(off));
+        off += (64 / V4) * rbytes;
+        if (d0 >= D) off = kBufOob;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < LPT; ++i) {
+        const int idx = i * 64 + lane, d0 = (u & 1) * (DP / 2) + 4 * (idx % V4);
+        r[i] = buf_load_f32x4(xr, buf_off(d0 < D ? (32 * (u >> 1) + idx / V4) * rbytes + d0 * 4 : kBufOob));
+      }
+    }
+    if (D & 3) {   // uniform: the columns past D inside the last vector
+#pragma unroll
+      for (int i = 0; i < LPT; ++i) {
+        const int d0 = (u & 1) * (DP / 2) + 4 * ((i * 64 + lane) % V4);
+        if (d0 + 1 >= D) r[i].y = 0.0f;
+        if (d0 + 2 >= D) r[i].z = 0.0f;
+        if (d0 + 3 >= D) r[i].w = 0.0f;
+      }
+    }
+  };
+  load(0, raw[0]);
+  float s = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int t = u >> 1, h = u & 1;
+    if (u < 3) load(u + 1, raw[(u + 1) & 1]);
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int idx = i * 64 + lane, rr = idx / V4, v = idx % V4;
+      const f32x4 x = raw[u & 1][i];
+      const uint2 w = {bf16_pair(f32x2{x.x, x.y}), bf16_pair(f32x2{x.z, x.w})};
+      *reinterpret_cast<uint2*>(xt + rr * RS + 4 * v) = w;
+      sq[rr * (V4 + 1) + v] = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w)));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (h == 0) s = 0.0f;
+#pragma unroll
+    for (int v = 0; v < V4; ++v) s += sq[c * (V4 + 1) + v];
+#pragma unroll
+    for (int q = 0; q < NQ / 2; ++q)
+      xb[t][h * (NQ / 2) + q] = *reinterpret_cast<const bf16x8*>(xt + c * RS + 16 * q + 8 * g);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (h == 1) {
+      if (g == t) xs = s;
+      // The constants' chunk: ||x||^2's splits in the first half, ones in the second.
+      f32x4 lo = zero4();
+      lo.x = s;
+      bf16x8 sp[3], a;
+      split3_bf16(lo, zero4(), sp);
+      const __bf16 one = (__bf16)1.0f, zero = (__bf16)0.0f;
+      a[0] = g == 0 ? sp[0][0] : one;
+      a[1] = g == 0 ? sp[1][0] : one;
+      a[2] = g == 0 ? sp[2][0] : one;
+      a[3] = g == 0 ? sp[0][0] : zero;
+      a[4] = g == 0 ? sp[1][0] : zero;
+      a[5] = g == 0 ? sp[0][0] : zero;
+      a[6] = zero;
+      a[7] = zero;
+      xb[t][NQ] = a;
+    }
+  }
+  const float nx = sqrtf(xs);
+  lds_barrier();   // every wave has read its staging tile: the second stage and the bounds may overwrite it
+
+  for (int kb = KB; kb < ((KB + 7) & ~7); ++kb) ub_l[kb * 64] = 0xff7f;   // the least finite bound
+
+  float L = -INFINITY;
+  const int nst = (KB + kScreenBlocks - 1) / kScreenBlocks;
+  for (int st = 0; st < nst; ++st) {
+    dma_barrier();   // stage st has landed, and every wave is done with stage st - 1
+    if (st + 1 < nst) fetch(st + 1);
+    const bf16x8* op = ((st & 1) ? reinterpret_cast<const bf16x8*>(rest) : op0) + lane;
+#pragma unroll
+    for (int j = 0; j < kScreenBlocks; ++j) {
+      const int kb = st * kScreenBlocks + j;
+      if (kb >= KB) break;
+      const float4 e = sc_e[kb];
+      // All of the block's operand reads in flight before the first is used.
+      bf16x8 a[NC];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) a[q] = op[(j * NC + q) * 64];
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16 acc[2] = {zero16(), zero16()};
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int q = 0; q < NC; ++q) acc[t] = mfma_bf16(a[q], xb[t][q], acc[t]);
+      }
+      float m[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        m[t] = acc[t][0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) m[t] = fmaxf(m[t], acc[t][i]);
+      }
+      // Lane l's own row is row l % 32 of tile l / 32; the other half-wave holds half of
+      // its block maximum.
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[0]), __float_as_uint(m[1]), false, false);
+      const float am = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      const float E = fmaf(e.x, nx, fmaf(e.y, xs, e.z));
+      // The bound rounded up to bf16: truncation does it for negative values, and for
+      // positive ones after adding 2^-7 of them (one bf16 step or more).
+      const float ub = am + E;
+      ub_l[kb * 64] = (unsigned short)(__float_as_uint(fmaf(fmaxf(ub, 0.0f), 0x1p-7f, ub)) >> 16);
+      L = fmaxf(L, am - E);
+    }
+  }
+
+  // Need words of the two tiles (each lane reads back the bounds it wrote itself), 32
+  // blocks at a time, lane c of half g keeping block kb0 + c of tile g.
+  const bool valid = row < N;
+  if (!valid) L = INFINITY;   // a row past N (zeros: finite bounds) gets no bit
+  const float near_gap = fminf(kLjNeedGap, kNearGap + 2.0f * log2f(1.0f + nx));   // kLjNeedGap if nx is NaN
+  uint64_t once = 0, twice = 0;   // rows with at least one, two near blocks
+  const int64_t tile = (row0 >> 5) + g;
+  for (int kb0 = 0; kb0 < KB; kb0 += 32) {
+    unsigned w = 0, wf = 0;
+#pragma unroll 1
+    for (int j0 = 0; j0 < 32 && kb0 + j0 < KB; j0 += 8) {
+      // Eight bounds in flight together (past KB: the fill).
+      float ub[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ub[j] = bf16_bits_to_float(ub_l[(kb0 + j0 + j) * 64]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float u = ub[j] - L;
+        const uint64_t b = __builtin_amdgcn_ballot_w64(!(u < -near_gap));
+        const uint64_t f = __builtin_amdgcn_ballot_w64(!(u < -kLjNeedGap)) & ~b;
+        twice |= once & b;
+        once |= b;
+        if (c == j0 + j) {
+          w = g == 0 ? (unsigned)b : (unsigned)(b >> 32);
+          wf = g == 0 ? (unsigned)f : (unsigned)(f >> 32);
+        }
+      }
+    }
+    if (kb0 + c < KB && tile * 32 < N) {
+      need[tile * KB + kb0 + c] = w;
+      faint[tile * KB + kb0 + c] = wf;
+    }
+  }
+  const uint64_t one = once & ~twice;
+  const uint64_t many = __builtin_amdgcn_ballot_w64(valid) & ~one;
+  if (c == 0 && tile * 32 < N) single[tile] = g == 0 ? (unsigned)one : (unsigned)(one >> 32);
+  // The workgroup's listed rows: one atomic for all (one per wave, at N=400K
+  // K=300 D=50 where most waves have some, serialised on the counter: 110 us for the
+  // kernel, 48 us this way).
+  int* cnt_l = reinterpret_cast<int*>(lds_raw);   // the first stage's operands have been used
+  lds_barrier();
+  if (lane == 0) cnt_l[wave] = __builtin_popcountll(many);
+  lds_barrier();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int v = 0; v < kScreenWaves; ++v) {
+    const int n = cnt_l[v];
+    before += v < wave ? n : 0;
+    total += n;
+  }
+  if (total == 0) return;
+  if (tid == 0) cnt_l[kScreenWaves] = (int)atomicAdd(reinterpret_cast<unsigned*>(list), (unsigned)total);
+  lds_barrier();
+  const int pos = cnt_l[kScreenWaves] + before +
+                  (int)__builtin_amdgcn_mbcnt_hi((unsigned)(many >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)many, 0u));
+  if ((many >> lane) & 1) list[kListBase + pos] = (int)row;
+}
 
 // ---------------------------------------------------------------------------
 // Pass 1 of the default plan above D = 128 (any D).  The split operands of a row
@@ -1260,19 +1784,22 @@ __device__ __forceinline__ unsigned lj_pair_total(const unsigned* __restrict__ c
 // ---------------------------------------------------------------------------
 
 
+constexpr int kGatherSt = 36;   // row stride (floats) of a gathered tile's S in LDS
 __host__ __device__ constexpr size_t gather_lds_bytes(int DP) {
   return (size_t)(DP / 16) * 4 * 64 * 16                          // mu block (bf16x8 operands)
+         + (size_t)32 * sizeof(double2)                           // its constants
+         + (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float)  // S tile per wave
          + (size_t)kGatherWaves * 2 * 32 * gather_rs(DP) * 2      // x1, x2 tiles per wave
          + (size_t)kGatherWaves * 32 * sizeof(double2)             // row state per wave
          + (size_t)kGatherWaves * 64 * sizeof(int);                // row queue per wave
 }
 
-// Slab groups: kGatherWaves waves per workgroup, each taking spw slabs one after another.
-__host__ __device__ constexpr int gather_groups(int nslab, int spw = 1) {
-  return (nslab + kGatherWaves * spw - 1) / (kGatherWaves * spw);
+// Slab groups: kGatherWaves waves per workgroup, one slab each.
+__host__ __device__ constexpr int gather_groups(int nslab) {
+  return (nslab + kGatherWaves - 1) / kGatherWaves;
 }
-__host__ inline int64_t gather_grid(int nslab, int KB, int spw = 1) {
-  return gather_item_grid(gather_groups(nslab, spw), KB);
+__host__ inline int64_t gather_grid(int nslab, int KB) {
+  return gather_item_grid(gather_groups(nslab), KB);
 }
 
 // Waves per SIMD of the gathering and tile passes: two where a wave's registers and
@@ -1285,22 +1812,29 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kGatherWaves, 64 * kG
                           amdgpu_waves_per_eu(gather_waves_per_simd(DP), gather_waves_per_simd(DP))))
 void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
                       const bf16x8* __restrict__ mu3, const double4* __restrict__ kc_gat, int KB, int KP,
-                      const double2* __restrict__ rowstat, const unsigned* __restrict__ need,
+                      double2* __restrict__ rowstat, const unsigned* __restrict__ need,
                       const unsigned* __restrict__ needcount, int64_t dense_min, int nslab,
                       int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_nk,
-                      float* __restrict__ part_sig, int dense, ProbeSel sel, int spw) {
+                      float* __restrict__ part_sig, int dense, const int* __restrict__ sel,
+                      const unsigned* __restrict__ single, const double2* __restrict__ kc_blk,
+                      float* __restrict__ logZ, int lse_only, float* __restrict__ near_nk, int faint) {
   constexpr int NQ = DP / 16;
   constexpr int NJ = DP / 32;
   constexpr int RS = gather_rs(DP);
   constexpr int BLK = NQ * 4 * 64;   // bf16x8 per component block
-  // With at least dense_min needed rows iso_accum_tiles runs instead (uniform exit).
-  if (need_total(needcount) >= dense_min) return;
-  // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO runs instead when selected.
-  if (probe_selects(sel)) return;
+  // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO runs instead when selected; after
+  // the screened pass 1 this kernel always runs, else with at least dense_min needed rows
+  // iso_accum_tiles does (uniform exits).
+  const int mode = iso_mode(sel);
+  if (mode == kModeStored) return;
+  if (mode == kModeDefault && (lse_only || faint || need_total(needcount) >= dense_min)) return;
+  const bool fused = mode == kModeScreen && single != nullptr;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   unsigned char* lp = lds_raw;
   bf16x8* mu_l = reinterpret_cast<bf16x8*>(lp);    lp += (size_t)BLK * sizeof(bf16x8);
+  double2* kb_l = reinterpret_cast<double2*>(lp);  lp += 32 * sizeof(double2);
+  float* st_all = reinterpret_cast<float*>(lp);    lp += (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float);
   __bf16* xt_all = reinterpret_cast<__bf16*>(lp);  lp += (size_t)kGatherWaves * 2 * 32 * RS * 2;
   double2* rs_all = reinterpret_cast<double2*>(lp); lp += (size_t)kGatherWaves * 32 * sizeof(double2);
   int* q_all = reinterpret_cast<int*>(lp);
@@ -1309,18 +1843,29 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
 
-  // Workgroup -> (slab group, block), spread over the XCDs by gather_item.  Up to
-  // D = 64 (two waves per SIMD) a wave takes one slab (the host passes spw = 1).
-  const int nsw = DP > 64 ? spw : 1;
+  // Workgroup -> (slab group, block), spread over the XCDs by gather_item.
   int sg, kb;
-  if (!gather_item(blockIdx.x, gather_groups(nslab, nsw), KB, sg, kb)) return;   // uniform over the workgroup
+  if (!gather_item(blockIdx.x, gather_groups(nslab), KB, sg, kb)) return;   // uniform over the workgroup
+  if (faint) {
+    // The second run after the screened pass 1: the block's faint pairs, where one of its
+    // components has too small an Nk to absorb them (one of zero weight has none).
+    float* nk_l = reinterpret_cast<float*>(lds_raw);   // [8][32]
+    float v = 0.0f;
+    for (int sl = tid >> 5; sl < nslab; sl += 8) v += near_nk[(int64_t)sl * KP + kb * 32 + c];
+    nk_l[tid] = v;
+    __syncthreads();
+    v = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v += nk_l[j * 32 + c];
+    const bool none = kc_gat[(int64_t)kb * 32 + c].x == -INFINITY;
+    if (__builtin_amdgcn_ballot_w64(!(v >= kNearNk) && !none) == 0) return;
+    __syncthreads();
+  }
   for (int idx = tid; idx < BLK; idx += 64 * kGatherWaves) mu_l[idx] = mu3[(int64_t)kb * BLK + idx];
+  if (tid < 32) kb_l[tid] = kc_blk[(int64_t)kb * 32 + tid];
   __syncthreads();
-  // The wave's nsw slabs, one after another, each into its own partial (no barrier
-  // follows).
-  for (int s2 = 0; s2 < nsw; ++s2) {
-  const int slab = (sg * nsw + s2) * kGatherWaves + wave;
-  if (slab >= nslab) break;
+  const int slab = sg * kGatherWaves + wave;
+  if (slab >= nslab) return;   // no barrier follows
 
   __bf16* xt = xt_all + wave * 2 * 32 * RS;   // [split][row][RS]
   double2* rs_l = rs_all + wave * 32;
@@ -1361,6 +1906,8 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   // state.  Stage P holds the tile after next while tile P is computed.
   f32x4 raw[2][2 * NQ];
   double2 rst[2];
+  unsigned sgl[2] = {0u, 0u};   // the single-block word of the row's tile (fused)
+  int erow[2] = {0, 0};
   // The rows come through resources over the slab: a lane without a row reads zeros
   // and makes no access, and the loads of a tile issue back to back.  X so while the
   // slab spans under 2 GiB (uniform; with one offset per lane where D fills whole
@@ -1369,8 +1916,12 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const bool xfull = xbuf && D == DP;
   const buf_rsrc xres = slab_rsrc(X, ldx, r_begin, xbuf ? r_end : r_begin);
   const buf_rsrc rres = make_rsrc(rowstat + r_begin, (uint32_t)((r_end - r_begin) * sizeof(double2)));
-  auto issue = [&](int e, f32x4 (&rw)[2 * NQ], double2& rs) __attribute__((always_inline)) {
+  const buf_rsrc sres = make_rsrc(fused ? single + t_begin : nullptr,
+                                  fused ? (uint32_t)((t_end - t_begin) * sizeof(unsigned)) : 0u);
+  auto issue = [&](int e, f32x4 (&rw)[2 * NQ], double2& rs, unsigned& sw, int& er) __attribute__((always_inline)) {
     const bool ok = e >= 0;
+    er = e;
+    sw = buf_load_u32(sres, buf_off(ok ? (e >> 5) * (int)sizeof(unsigned) : kBufOob));
     if (xfull) {
       const int off = buf_off(ok ? (int)((int64_t)e * ldx * (int64_t)sizeof(float)) + 32 * g : kBufOob);
 #pragma unroll
@@ -1408,6 +1959,22 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   auto tile = [&](auto par) __attribute__((always_inline)) -> int {
     constexpr int P = decltype(par)::value;
     // This tile's rows: bf16 splits in registers, x1 and x2 to LDS, row state to LDS.
+    // A row whose one needed block is this one (fused) has no row state yet: its ||x||^2
+    // is formed here as pass 1 does, its logZ2 below.
+    const bool own = fused && erow[P] >= 0 && ((sgl[P] >> (erow[P] & 31)) & 1u);
+    const bool owns = fused && __builtin_amdgcn_ballot_w64(own) != 0;
+    const int64_t orow = r_begin + erow[P];
+    if (owns) {
+      double xsq = 0.0;
+#pragma unroll
+      for (int q = 0; q < 2 * NQ; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) xsq = fma((double)raw[P][q][e], (double)raw[P][q][e], xsq);
+      }
+      xsq += __shfl_xor(xsq, 32);
+      if (own) rst[P].x = xsq;
+    }
+    const double xsq_own = rst[P].x;
     bf16x8 xa[NQ][3];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) split3_bf16(raw[P][2 * q], raw[P][2 * q + 1], xa[q]);
@@ -1421,10 +1988,47 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
     if (g == 0) rs_l[c] = rst[P];
     int en;
     const int cnt_ahead = take(en);
-    if (cnt_ahead > 0) issue(en, raw[P], rst[P]);
+    if (cnt_ahead > 0) issue(en, raw[P], rst[P], sgl[P], erow[P]);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
     const f32x16 S = x6c_tile_rows<NQ, kIsoChains>(xa, ones, [&](int q, int t) { return mu_l[(q * 4 + t) * 64 + lane]; });
+    if (owns) {
+      // logZ2 of the tile's own rows, over the block's 32 components as pass 1 forms it
+      // (lane = row, the components of a half-wave in register order, the halves merged):
+      // every other block's terms are exactly zero there, so these are the same bits.
+      float* st = st_all + wave * 32 * kGatherSt;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) st[acc_row(i, g) * kGatherSt + c] = S[i];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      double ll[16], bm = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(st + c * kGatherSt + 8 * j + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double2 cb = kb_l[g * 16 + 4 * j + e];
+          ll[4 * j + e] = fma(-cb.y, fma(-2.0, (double)v[e], xsq_own), cb.x);
+          bm = fmax(bm, ll[4 * j + e]);
+        }
+      }
+      const double ms = (bm == -INFINITY) ? 0.0 : bm;
+      float sm = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sm += fast_exp2((float)(ll[i] - ms));
+      const double mo = __shfl_xor(bm, 32);
+      const float so = __shfl_xor(sm, 32);
+      const double mn = fmax(bm, mo);
+      const double mt = (mn == -INFINITY) ? 0.0 : mn;
+      const float tot = sm * fast_exp2((float)(bm - mt)) + so * fast_exp2((float)(mo - mt));
+      const double lz2 = mn + (double)log2f(tot);
+      if (own && g == 0) {
+        rs_l[c].y = lz2;
+        rowstat[orow] = make_double2(xsq_own, lz2);
+        if (logZ) logZ[orow] = (float)(lz2 * kLn2);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if (lse_only) return cnt_ahead;
     float r[16], res[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -1459,18 +2063,29 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
 
   int e;
   int cnt0 = take(e);
-  if (cnt0 > 0) issue(e, raw[0], rst[0]);
+  if (cnt0 > 0) issue(e, raw[0], rst[0], sgl[0], erow[0]);
   int cnt1 = cnt0 > 0 ? take(e) : 0;
-  if (cnt1 > 0) issue(e, raw[1], rst[1]);
+  if (cnt1 > 0) issue(e, raw[1], rst[1], sgl[1], erow[1]);
   while (cnt0 > 0) {
     cnt0 = tile(std::integral_constant<int, 0>{});
     if (cnt1 == 0) break;
     cnt1 = tile(std::integral_constant<int, 1>{});
   }
+  if (lse_only) return;
 
   nk += __shfl_xor(nk, 32);
   sig += __shfl_xor(sig, 32);
   const int64_t kbase = (int64_t)slab * KP + (int64_t)kb * 32;
+  if (faint) {   // added to the near pairs' sums
+    if (qt == 0) return;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[j][i] += part_mu[(kbase + acc_row(i, g)) * DP + 32 * j + c];
+    }
+    nk += part_nk[kbase + c];
+    sig += part_sig[kbase + c];
+  }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
 #pragma unroll
@@ -1479,7 +2094,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   if (g == 0) {
     part_nk[kbase + c] = nk;
     part_sig[kbase + c] = sig;
-  }
+    if (mode == kModeScreen && !faint) near_nk[kbase + c] = nk;
   }
 }
 
@@ -1511,7 +2126,7 @@ void iso_accum_tiles(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
                      const double2* __restrict__ rowstat, const unsigned* __restrict__ need,
                      const unsigned* __restrict__ needcount, int64_t dense_min, int nslab,
                      int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_nk,
-                     float* __restrict__ part_sig, int dense, ProbeSel sel) {
+                     float* __restrict__ part_sig, int dense, const int* __restrict__ sel) {
   constexpr int NQ = DP / 16;
   constexpr int NJ = DP / 32;
   constexpr int RS = gather_rs(DP);
@@ -1520,8 +2135,8 @@ void iso_accum_tiles(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   constexpr int V4 = DP / 4;              // float4 per row
   constexpr int LPT = 32 * V4 / NT;       // float4 per thread per tile
   static_assert((32 * V4) % NT == 0, "tile split");
-  if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exit)
-  if (probe_selects(sel)) return;   // the stored branch runs
+  if (iso_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
+  if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exits)
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __bf16* xs = reinterpret_cast<__bf16*>(lds_raw);                                   // [2][3][32][RS]
@@ -1714,7 +2329,7 @@ void iso_accum_tiles2(const float* __restrict__ X, int64_t ldx, int64_t N, int D
                       const double2* __restrict__ rowstat, const unsigned* __restrict__ need,
                       const unsigned* __restrict__ needcount, int64_t dense_min, int nslab,
                       int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_nk,
-                      float* __restrict__ part_sig, int dense, ProbeSel sel) {
+                      float* __restrict__ part_sig, int dense, const int* __restrict__ sel) {
   constexpr int NQ = DP / 16;
   constexpr int NQH = NQ / 2;              // chunks of this wave's chain
   constexpr int NJ = DP / 32;
@@ -1725,8 +2340,8 @@ void iso_accum_tiles2(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   constexpr int NV = 32 * V4;              // float4 per tile
   constexpr int LPT = (NV + NT - 1) / NT;  // float4 per thread per tile
   static_assert(NQ % 2 == 0 && kIsoChains == 2, "one chain per wave of a pair");
-  if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exit)
-  if (probe_selects(sel)) return;   // the stored branch runs
+  if (iso_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
+  if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exits)
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __bf16* xs = reinterpret_cast<__bf16*>(lds_raw);                                   // [3][3][32][RS]
@@ -2499,7 +3114,7 @@ template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kLjtWaves, 64 * kLjtWaves), amdgpu_waves_per_eu(2, 2)))
 void iso_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xsplit, const float2* __restrict__ zpair,
                    int64_t N, const unsigned* __restrict__ ljmask, const unsigned* __restrict__ ljcount,
-                   int64_t sparse_max, ProbeSel sel, const double4* __restrict__ kc_lin,
+                   int64_t sparse_max, const int* __restrict__ sel, const double4* __restrict__ kc_lin,
                    int KB, int KP, int nslab, int64_t rows_per_slab, int ncg, float* __restrict__ part_mu,
                    float* __restrict__ part_nk, float* __restrict__ part_sig, int dense) {
   static_assert(DP <= 128 && DP % 32 == 0, "one 32-row tile of X per stage");
@@ -2511,7 +3126,7 @@ void iso_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xspl
   // iso_accum_sparse takes the call when pass 1 found the masks sparse; with a
   // selector word, the recomputing kernels take it unless the word is set.
   if (sparse_max >= 0 && need_total(ljcount) <= sparse_max) return;
-  if (sel.count != nullptr && !probe_selects(sel)) return;
+  if (sel != nullptr && iso_mode(sel) != kModeStored) return;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
 
@@ -2940,65 +3555,64 @@ void iso_accum_sparse(const float* __restrict__ X, int64_t ldx, int64_t N, const
 // ---------------------------------------------------------------------------
 // Finish: fixed-order fp64 reduction over slabs (deterministic).
 // ---------------------------------------------------------------------------
+// The partials a call left: `stored` of them where the stored branch ran, else `n`.
+struct PartCount {
+  const int* sel;
+  int n, stored;
+};
+__device__ __forceinline__ int part_count(const PartCount& p) {
+  return iso_mode(p.sel) == kModeStored ? p.stored : p.n;
+}
+
+// A workgroup sums 256 / G consecutive output columns (mu_acc rows, then Nk, then
+// sig_acc, as one list): G threads a column take the partials in turn (G = 4, 16), so the
+// loads of a wave stay in whole lines, and their sums are added in order.  One wave per
+// output over the partials instead read a line per lane: 19 us at N=400K K=300 D=50
+// (112 partials), 8 us here.
+template <int G>
 __global__ __launch_bounds__(256) void iso_reduce(const float* __restrict__ part_mu,
                                                   const float* __restrict__ part_nk,
-                                                  const float* __restrict__ part_sig, int nslab,
+                                                  const float* __restrict__ part_sig, PartCount parts,
                                                   int KP, int DP, int64_t K, int D,
                                                   float* __restrict__ Nk, float* __restrict__ mu_acc,
                                                   float* __restrict__ sig_acc, int accumulate) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int W = D + 2;
-  if (idx >= K * W) return;
-  const int64_t k = idx / W;
-  const int col = (int)(idx % W);
+  constexpr int C = 256 / G;
+  __shared__ double sum[G][C];
+  const int np = part_count(parts);
+  const int col = threadIdx.x % C, grp = threadIdx.x / C;
+  const int64_t idx = (int64_t)blockIdx.x * C + col, nmu = K * D;
+  const float* p = nullptr;
+  int64_t stride = KP;
+  float* o = nullptr;
+  if (idx < nmu) {
+    const int64_t k = idx / D;
+    p = part_mu + k * DP + (idx - k * D);
+    stride = (int64_t)KP * DP;
+    o = mu_acc + idx;
+  } else if (idx < nmu + K) {
+    p = part_nk + (idx - nmu);
+    o = Nk + (idx - nmu);
+  } else if (idx < nmu + 2 * K) {
+    p = part_sig + (idx - nmu - K);
+    o = sig_acc + (idx - nmu - K);
+  }
+  sum[grp][col] = (p && grp < np) ? strided_sum(p + grp * stride, (np - grp + G - 1) / G, G * stride) : 0.0;
+  __syncthreads();
+  if (grp != 0 || !o) return;
   double s = 0.0;
-  if (col < D) {
-    s = strided_sum(part_mu + k * DP + col, nslab, (int64_t)KP * DP);
-    float* o = mu_acc + k * D + col;
-    *o = accumulate ? (float)((double)*o + s) : (float)s;
-  } else if (col == D) {
-    s = strided_sum(part_nk + k, nslab, KP);
-    Nk[k] = accumulate ? (float)((double)Nk[k] + s) : (float)s;
-  } else {
-    s = strided_sum(part_sig + k, nslab, KP);
-    sig_acc[k] = accumulate ? (float)((double)sig_acc[k] + s) : (float)s;
-  }
-}
-
-// The same finish with one wave per output element, for many partials (few
-// components over many row slabs).
-__global__ __launch_bounds__(256) void iso_reduce_wide(const float* __restrict__ part_mu,
-                                                       const float* __restrict__ part_nk,
-                                                       const float* __restrict__ part_sig, int nslab,
-                                                       int KP, int DP, int64_t K, int D,
-                                                       float* __restrict__ Nk, float* __restrict__ mu_acc,
-                                                       float* __restrict__ sig_acc, int accumulate) {
-  const int64_t idx = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int W = D + 2;
-  if (idx >= K * W) return;
-  const int64_t k = idx / W;
-  const int col = (int)(idx % W);
-  if (col < D) {
-    const double s = wave_strided_sum(part_mu + k * DP + col, nslab, (int64_t)KP * DP, lane);
-    float* o = mu_acc + k * D + col;
-    if (lane == 0) *o = accumulate ? (float)((double)*o + s) : (float)s;
-  } else if (col == D) {
-    const double s = wave_strided_sum(part_nk + k, nslab, KP, lane);
-    if (lane == 0) Nk[k] = accumulate ? (float)((double)Nk[k] + s) : (float)s;
-  } else {
-    const double s = wave_strided_sum(part_sig + k, nslab, KP, lane);
-    if (lane == 0) sig_acc[k] = accumulate ? (float)((double)sig_acc[k] + s) : (float)s;
-  }
+#pragma unroll
+  for (int j = 0; j < G; ++j) s += sum[j][col];
+  *o = accumulate ? (float)((double)*o + s) : (float)s;
 }
 
 // Atomic finish: every slab partial is added into the (zeroed or accumulated) outputs.
 __global__ __launch_bounds__(256) void iso_reduce_atomic(const float* __restrict__ part_mu,
                                                          const float* __restrict__ part_nk,
-                                                         const float* __restrict__ part_sig, int nslab,
+                                                         const float* __restrict__ part_sig, PartCount parts,
                                                          int KP, int DP, int64_t K, int D,
                                                          float* __restrict__ Nk, float* __restrict__ mu_acc,
                                                          float* __restrict__ sig_acc) {
+  const int nslab = part_count(parts);
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int W = D + 2;
   const int sl = blockIdx.y;
@@ -3075,6 +3689,11 @@ hipError_t launch_ctile(const IsoPlan& pl, const float* X, int64_t ldx, unsigned
   return hipGetLastError();
 }
 
+// The word that holds the device's choice of the call's branches (nullptr: none to make).
+const int* iso_sel(const IsoPlan& pl, unsigned char* ws) {
+  return pl.nprobe > 0 ? reinterpret_cast<const int*>(ws + pl.off_probe) + kProbeMode : nullptr;
+}
+
 // The default plan up to D = 128, the stored plan's passes up to D = 128 and its
 // pass 2 above (pass 1 there is launch_ctile's).
 template <int DP>
@@ -3089,19 +3708,37 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
   float* lj = (pl.lj || pl.autolj) ? reinterpret_cast<float*>(ws + pl.off_lj) : nullptr;
   unsigned* ljmask = reinterpret_cast<unsigned*>(ws + pl.off_ljmask);
   unsigned* ljcount = reinterpret_cast<unsigned*>(ws + pl.off_ljcount);
+  // A dense call computes every pair, so it never screens.  Both phases of a split call
+  // evaluate the same choice.
+  const bool screen = pl.screen && !dense && ldx <= kMaxScreenLdx;
+  unsigned* single = screen ? reinterpret_cast<unsigned*>(ws + pl.off_single) : nullptr;
+  int* list = screen ? reinterpret_cast<int*>(ws + pl.off_list) : nullptr;
+  unsigned* faint = screen ? reinterpret_cast<unsigned*>(ws + pl.off_faint) : nullptr;
+  float* near_nk = screen ? reinterpret_cast<float*>(ws + pl.off_nearnk) : nullptr;
+  const int* sel = iso_sel(pl, ws);
   if (run1) {
     if constexpr (DP <= 128) {
       hipError_t e = hipSuccess;
       if (pl.need || pl.lj) {
         // The software-pipelined pass 1 (the stored plan's also writes the log-joint;
         // with FGMM_FLAG_STORE_LOGJOINT_AUTO the probe's selector decides first).
-        unsigned* probe = pl.autolj ? reinterpret_cast<unsigned*>(ws + pl.off_probe) : nullptr;
-        if (pl.autolj)
+        if (sel)
           hipLaunchKernelGGL((iso_store_probe<DP>), dim3((unsigned)pl.nprobe), dim3(64 * kProbeWaves), 0, stream, X, ldx, pl.N,
-                             (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3), kc_blk, pl.KB, pl.nprobe,
-                             probe);
-        const ProbeSel psel = probe ? ProbeSel{probe, pl.nprobe, probe_min_pairs(pl.N, pl.nprobe, pl.KB)}
-                                    : ProbeSel{nullptr, 0, 0};
+                             (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3), kc_blk, pl.KB,
+                             screen ? reinterpret_cast<const float4*>(ws + pl.off_sce) : nullptr, pl.nprobe,
+                             IsoRule{screen ? (int64_t)pl.nprobe * 32 / 2 : -1, probe_min_pairs(pl.N, pl.nprobe, pl.KB),
+                                     pl.autolj ? 1 : 0},
+                             reinterpret_cast<unsigned*>(ws + pl.off_probe));
+        if (screen) {
+          const size_t lds = screen_lds_bytes(DP, pl.KB);
+          if (lds > 65536)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&iso_screen<DP>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+          if (e != hipSuccess) return e;
+          hipLaunchKernelGGL(iso_screen<DP>, dim3((unsigned)cdiv(pl.N, 64 * kScreenWaves)), dim3(64 * kScreenWaves), lds,
+                             stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_scop),
+                             reinterpret_cast<const float4*>(ws + pl.off_sce), pl.KB, ljmask, faint, single, list, sel);
+        }
         const bool st = pl.lj || pl.autolj;
         const size_t lds1 = lse_pipe_lds_bytes<DP>() + (pl.rexact ? (size_t)kPipeWaves * 32 * pl.KB * 2 : 0) +
                             (st ? kPipeStoreLds : 0);
@@ -3113,15 +3750,16 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
         const PipeGrid pg = pipe_grid(pl.N);
         hipLaunchKernelGGL(kern, dim3((unsigned)pg.grid), dim3(kPipeThreads), lds1, stream,
                            X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3), kc_blk,
-                           pl.KB, logZ, rowstat, ljmask, ljcount, dense ? 1 : 0, lj, psel,
+                           pl.KB, logZ, rowstat, ljmask, ljcount, dense ? 1 : 0, lj, sel,
                            reinterpret_cast<__bf16*>(ws + pl.off_xsplit), reinterpret_cast<float2*>(ws + pl.off_zpair),
-                           pg.full, pg.small);
+                           pg.full, pg.small, list,
+                           std::min<int64_t>((int64_t)kFewRounds * 32 * current_device_cus(), pg.grid * 32));
       }
     } else {
       return hipErrorInvalidValue;   // launch_ctile runs pass 1 above D = 128
     }
   }
-  if (!run2) return hipGetLastError();
+  if (!run2 && !screen) return hipGetLastError();
   if constexpr (DP <= 128) {
     if (pl.need) {
       // Both forms are launched; the needed-row count pass 1 left selects one on the
@@ -3131,20 +3769,17 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
       const int64_t dense_min = cdiv(cdiv(pl.N, 32) * 32 * (int64_t)pl.KB * 3, 4);
       // FGMM_FLAG_STORE_LOGJOINT_AUTO: the stored branch (iso_accum_ljt over the same
       // slabs and partials) is launched too; the probe's selector picks one side.
-      const ProbeSel sel = pl.autolj ? ProbeSel{reinterpret_cast<const unsigned*>(ws + pl.off_probe), pl.nprobe,
-                                                probe_min_pairs(pl.N, pl.nprobe, pl.KB)}
-                                     : ProbeSel{nullptr, 0, 0};
-      if (pl.autolj) {
+      if (pl.autolj && run2) {
         constexpr size_t ldsj = LjtShape<DP>::lds;
         static_assert(ldsj <= kMaxLds, "stored pass-2 stages exceed LDS");
         hipError_t ej = hipFuncSetAttribute(reinterpret_cast<const void*>(&iso_accum_ljt<DP>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)ldsj);
         if (ej != hipSuccess) return ej;
         const int ncg = (int)cdiv(pl.KB, kLjtWaves);
-        hipLaunchKernelGGL((iso_accum_ljt<DP>), dim3((unsigned)ljt_grid(pl.nslab, ncg)), dim3(64 * kLjtWaves), ldsj,
+        hipLaunchKernelGGL((iso_accum_ljt<DP>), dim3((unsigned)ljt_grid(pl.nslab_lj, ncg)), dim3(64 * kLjtWaves), ldsj,
                            stream, lj, reinterpret_cast<const __bf16*>(ws + pl.off_xsplit),
                            reinterpret_cast<const float2*>(ws + pl.off_zpair), pl.N, ljmask, ljcount, (int64_t)-1,
-                           sel, kc_lin, pl.KB, pl.KP, pl.nslab, pl.rows_per_slab, ncg, pmu, pnk, psig,
+                           sel, kc_lin, pl.KB, pl.KP, pl.nslab_lj, pl.rows_per_slab_lj, ncg, pmu, pnk, psig,
                            dense ? 1 : 0);
       }
       constexpr size_t lds = gather_lds_bytes(DP);
@@ -3152,17 +3787,18 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&iso_accum_gather<DP>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) return e;
-      // Above D = 64 the gather runs one wave per SIMD: where its (slab, block) items
-      // would take two rounds of waves, each wave takes two slabs in turn (C2, same
-      // box: 0.221 -> 0.197 ms), keeping the slabs and partials the stored branch's
-      // pass 2 shares.
-      const int spw = (DP > 64 && (int64_t)pl.nslab * pl.KB >= (int64_t)2 * 4 * current_device_cus()) ? 2 : 1;
-      hipLaunchKernelGGL(iso_accum_gather<DP>, dim3((unsigned)gather_grid(pl.nslab, pl.KB, spw)),
-                         dim3(64 * kGatherWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
-                         reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
-                         reinterpret_cast<const double4*>(ws + pl.off_kcgat), pl.KB, pl.KP, rowstat,
-                         ljmask, ljcount, dense_min, pl.nslab, pl.rows_per_slab, pmu, pnk, psig,
-                         dense ? 1 : 0, sel, spw);
+      auto gather = [&](const unsigned* words, int faint_pass) {
+        hipLaunchKernelGGL(iso_accum_gather<DP>, dim3((unsigned)gather_grid(pl.nslab, pl.KB)),
+                           dim3(64 * kGatherWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
+                           reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
+                           reinterpret_cast<const double4*>(ws + pl.off_kcgat), pl.KB, pl.KP, rowstat,
+                           words, ljcount, dense_min, pl.nslab, pl.rows_per_slab, pmu, pnk, psig,
+                           dense ? 1 : 0, sel, run1 && !faint_pass ? single : nullptr, kc_blk, logZ, run2 ? 0 : 1,
+                           near_nk, faint_pass);
+      };
+      gather(ljmask, 0);
+      if (!run2) return hipGetLastError();
+      if (screen) gather(faint, 1);
       // The tile pass: one wave per block up to D = 64, a pair of waves (one chain
       // each) at D = 96 and 128.
       auto tiles = [&](auto kern, size_t lds_t, int waves) -> hipError_t {
@@ -3208,7 +3844,7 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
     hipLaunchKernelGGL((iso_accum_ljt<DP>), dim3((unsigned)ljt_grid(pl.nslab, pl.ncg)), dim3(64 * kLjtWaves), lds,
                        stream, lj, reinterpret_cast<const __bf16*>(ws + pl.off_xsplit),
                        reinterpret_cast<const float2*>(ws + pl.off_zpair), pl.N, ljmask, ljcount, sparse_max,
-                       ProbeSel{nullptr, 0, 0}, kc_lin, pl.KB, pl.KP, pl.nslab, pl.rows_per_slab, pl.ncg, pmu, pnk,
+                       nullptr, kc_lin, pl.KB, pl.KP, pl.nslab, pl.rows_per_slab, pl.ncg, pmu, pnk,
                        psig, dense ? 1 : 0);
     return hipGetLastError();
   }
@@ -4309,6 +4945,17 @@ extern "C" size_t fgmm_iso_workspace_bytes_ex(int64_t N, int64_t K, int64_t D, u
   return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags)).total;
 }
 
+// The least workspace fgmm_iso_estep_f32 takes for the call (without the screened pass
+// 1); fgmm_iso_workspace_bytes_ex gives what it can use.
+namespace fgmm {
+size_t iso_min_workspace(int64_t N, int64_t K, int64_t D, unsigned flags);
+}
+size_t fgmm::iso_min_workspace(int64_t N, int64_t K, int64_t D, unsigned flags) {
+  const int64_t rows = iso_bw_call(D, flags) ? std::min(N, iso_bw_chunk_rows(K)) : N;
+  return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags), false)
+      .total;
+}
+
 extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_t D, const float* mu,
                                   int64_t ldmu, int64_t K, const float* log_sigma_sq,
                                   const float* log_pi, float* logZ, float* Nk, float* mu_acc,
@@ -4347,7 +4994,10 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
   }
   // The stored log-joint path streams X with 32-bit buffer offsets (row stride at
   // most kMaxBufLdx floats); wider strides recompute, which needs less workspace.
-  const IsoPlan pl = make_plan(N, K, D, wants_stored_lj(flags) && ldx <= kMaxBufLdx, bf16, wants_auto_lj(flags));
+  // A workspace without room for the screened pass 1 runs the call without it.
+  const bool stored = wants_stored_lj(flags) && ldx <= kMaxBufLdx;
+  IsoPlan pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags));
+  if (workspace_bytes < pl.total && pl.screen) pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags), false);
   if (workspace_bytes < pl.total || (pl.total > 0 && workspace == nullptr)) return FGMM_ERR_WORKSPACE;
   if (!want_logz) logZ = nullptr;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
@@ -4368,12 +5018,16 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
                        reinterpret_cast<f32x4*>(ws + pl.off_kcblk),
                        pl.bfneed ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr);
   else if (run1)
-    hipLaunchKernelGGL(iso_prep, dim3(pl.KB), dim3(64), 0, stream, mu, ldmu, K, (int)D, pl.DP,
+    hipLaunchKernelGGL(iso_prep, dim3(pl.KB), dim3(64 * kPrepWaves), 0, stream, mu, ldmu, K, (int)D, pl.DP,
                        log_sigma_sq, log_pi, reinterpret_cast<double2*>(ws + pl.off_kcblk),
                        reinterpret_cast<double4*>(ws + pl.off_kclin),
                        reinterpret_cast<double4*>(ws + pl.off_kcgat),
                        reinterpret_cast<bf16x8*>(ws + pl.off_mu3),
-                       (pl.lj || pl.need) ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr);
+                       (pl.lj || pl.need) ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr,
+                       pl.screen ? reinterpret_cast<bf16x8*>(ws + pl.off_scop) : nullptr,
+                       pl.screen ? reinterpret_cast<float4*>(ws + pl.off_sce) : nullptr,
+                       pl.screen ? reinterpret_cast<unsigned*>(ws + pl.off_list) : nullptr,
+                       pl.nprobe > 0 ? reinterpret_cast<unsigned*>(ws + pl.off_probe) : nullptr);
   if (N > 0) {
     auto run = [&](auto dp_tag) -> hipError_t {
       constexpr int DP = decltype(dp_tag)::value;
@@ -4406,6 +5060,7 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
   const float* pnk = reinterpret_cast<const float*>(ws + pl.off_part_nk);
   const float* psig = reinterpret_cast<const float*>(ws + pl.off_part_sig);
   const int64_t nout = K * (D + 2);
+  const PartCount parts{iso_sel(pl, ws), pl.nslab * pl.rgroups, pl.nslab_lj * pl.rgroups};
   if (atomic) {
     if (!accumulate) {
       hipLaunchKernelGGL(fill_f32, dim3((unsigned)cdiv(K, 256)), dim3(256), 0, stream, Nk, K, 0.0f);
@@ -4416,16 +5071,16 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
     }
     if (pl.npart > 0)
       hipLaunchKernelGGL(iso_reduce_atomic, dim3((unsigned)cdiv(nout, 256), (unsigned)pl.npart),
-                         dim3(256), 0, stream, pmu, pnk, psig, pl.npart, pl.KP, pl.DP, K, (int)D, Nk,
+                         dim3(256), 0, stream, pmu, pnk, psig, parts, pl.KP, pl.DP, K, (int)D, Nk,
                          mu_acc, sig_acc);
-  } else if (pl.npart >= kWideReduce) {
-    hipLaunchKernelGGL(iso_reduce_wide, dim3((unsigned)cdiv(nout, 4)), dim3(256), 0, stream, pmu, pnk,
-                       psig, pl.npart, pl.KP, pl.DP, K, (int)D, Nk, mu_acc, sig_acc,
-                       accumulate ? 1 : 0);
   } else {
-    hipLaunchKernelGGL(iso_reduce, dim3((unsigned)cdiv(nout, 256)), dim3(256), 0, stream, pmu, pnk,
-                       psig, pl.npart, pl.KP, pl.DP, K, (int)D, Nk, mu_acc, sig_acc,
-                       accumulate ? 1 : 0);
+    auto reduce = [&](auto g_tag) {
+      constexpr int G = decltype(g_tag)::value;
+      hipLaunchKernelGGL(iso_reduce<G>, dim3((unsigned)cdiv(nout, 256 / G)), dim3(256), 0, stream, pmu, pnk, psig,
+                         parts, pl.KP, pl.DP, K, (int)D, Nk, mu_acc, sig_acc, accumulate ? 1 : 0);
+    };
+    if (pl.npart >= kWideReduce) reduce(std::integral_constant<int, 16>{});
+    else reduce(std::integral_constant<int, 4>{});
   }
   return hipGetLastError() == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
 }

@@ -14,6 +14,10 @@
 
 #include "flashgmm.h"
 
+namespace fgmm {
+size_t iso_min_workspace(int64_t N, int64_t K, int64_t D, unsigned flags);   // fgmm_iso.hip
+}
+
 // Workspace of fgmm_iso_estep_f32_noalloc: one array per GPU.  Host code never passes
 // the name `scratch` itself (on the host it is a stand-in, not a device address): the
 // device address comes from hipGetSymbolAddress, looked up once per device.
@@ -41,7 +45,7 @@ int current_scratch(void** out) {
 
 namespace {
 bool fits(int64_t n, int64_t K, int64_t D, unsigned flags) {
-  return fgmm_iso_workspace_bytes_ex(n, K, D, flags) <= FGMM_NOALLOC_SCRATCH_BYTES;
+  return fgmm::iso_min_workspace(n, K, D, flags) <= FGMM_NOALLOC_SCRATCH_BYTES;
 }
 }  // namespace
 
