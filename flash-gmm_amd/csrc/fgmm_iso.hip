@@ -333,7 +333,7 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     const int64_t want = gather_slab_count(cdiv(rounds * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double2));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
-    if (p.autolj) {
+    if (p.DP <= 128) {   // its partials are laid out with or without the branch
       const int64_t wl = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
       p.rows_per_slab_lj = cap_slab_rows(round_up(cdiv(N, wl), 32), sizeof(double2));
       p.nslab_lj = (int)cdiv(N, p.rows_per_slab_lj);
