@@ -28,7 +28,7 @@
 // Row slabs are disjoint ([s*R, min(N, (s+1)*R))), so no row is counted twice at a
 // slab boundary.
 
-#include "fgmm_common.hpp"
+#include "fgmm_screen.hpp"
 
 #include <math.h>
 
@@ -109,6 +109,10 @@ __host__ __device__ constexpr bool ljd_applies(int DP) { return DP <= 96; }
 // distinct banks.
 __device__ __forceinline__ int ljd_swz(int r) { return (((r >> 2) & 1) << 1) | (((r >> 1) ^ (r >> 3)) & 1); }
 
+// Partials a slab of the gathering pass 2 leaves (two above D = 64, where one round of
+// waves takes half the slabs: the float32 sums stay as short).
+__host__ __device__ constexpr int gather_parts(int DP) { return DP <= 64 ? 1 : 2; }
+
 struct DiagPlan {
   int64_t N, K, D;
   int DP, FP;   // D padded (32 up to 128, then 64); feature count 2*DP
@@ -129,9 +133,14 @@ struct DiagPlan {
                     // (or diag_bf16_accum where most pairs are needed)
   bool autolj;      // the default plan with a stored branch that a row-sample probe selects on the
                     // device (FGMM_FLAG_STORE_LOGJOINT_AUTO, D <= 96)
+  bool screen;      // default plan up to D = 128, large calls: a probe selects the screened pass 1
+                    // (screen_pairs) on the device where most rows are near one component block
   int nprobe;       // the probe's sampled tiles
-  size_t off_xsplit, off_zpair, off_probe;
-  size_t off_musw, off_mu3, off_kcx6, off_kcx6lin, off_kclin, off_rowstat, off_part_mu,
+  int spp;          // partials per slab (pass 2)
+  int nslab_lj;     // row slabs of the stored branch's pass 2
+  int64_t rows_per_slab_lj;
+  size_t off_xsplit, off_zpair, off_probe, off_scop, off_sce, off_list, off_state;
+  size_t off_musw, off_mu3, off_kcx6, off_kclin, off_rowstat, off_part_mu,
       off_part_sq, off_part_nk, off_lj, off_ljmax, off_ljmask, off_ljcount, total;
 };
 
@@ -157,19 +166,21 @@ __host__ inline bool use_stored_lj(int64_t N, int KB, int DP, bool allow) {
 }
 
 DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool bf16 = false,
-                   bool auto_lj = false) {
+                   bool auto_lj = false, bool allow_screen = true) {
   DiagPlan p{};
   p.N = N; p.K = K; p.D = D;
   p.DP = diag_padded_dim(D);
   p.FP = 2 * p.DP;
   p.KB = (int)cdiv(K, 32);
   p.KP = p.KB * 32;
+  p.spp = 1;
   p.bf16 = bf16;
   p.lj = !bf16 && use_stored_lj(N, p.KB, p.DP, allow_lj);
   p.need = !bf16 && !p.lj;
   p.autolj = p.need && auto_lj && ljd_applies(p.DP) && N > 0 && p.KB > 0 && p.KB <= kProbeMaxKB &&
              (size_t)round_up(cdiv(N, 32), 4) * (size_t)p.KB * kLjTile * sizeof(float) <= kMaxLjBytes;
-  p.nprobe = p.autolj ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
+  p.screen = p.need && allow_screen && use_screen(N, p.DP, true, p.KB);
+  p.nprobe = (p.autolj || p.screen) ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
   p.ctile = !bf16 && !diag_uses_x6(p.DP);
   p.rexact = p.need && p.KB <= (p.ctile ? ctile_need_exact_cap(ctile_blocks(p.DP)) : need_exact_cap(p.DP));
   p.ndr = p.ctile ? (int)cdiv(p.DP, kDrange) : 1;
@@ -209,11 +220,17 @@ DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
   } else if (p.need && N > 0 && p.KB > 0) {
-    // The gathering pass 2: eight waves per compute unit, two rounds at one wave per
-    // SIMD (one round where two fit).
-    const int64_t want = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
-    p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
-    p.nslab = (int)cdiv(N, p.rows_per_slab);
+    // The gathering pass 2: one round of waves, two per SIMD up to D = 64, one above.
+    // The stored branch's pass 2 takes eight blocks per compute unit; the partials are
+    // laid out for it with or without the branch.
+    auto slabs = [&](int64_t waves, int64_t& rows) {
+      const int64_t want = gather_slab_count(cdiv(waves * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
+      rows = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
+      return (int)cdiv(N, rows);
+    };
+    p.spp = gather_parts(p.DP);
+    p.nslab = slabs(p.DP <= 64 ? 8 : 4, p.rows_per_slab);
+    p.nslab_lj = slabs(8, p.rows_per_slab_lj);
   } else if (N > 0 && p.ncg > 0) {
     int64_t want = (int64_t)current_device_cus() / p.ncg;
     if (want >= 8) want = (want / 8) * 8;
@@ -226,16 +243,27 @@ DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
     p.rows_per_slab = tile_rows;
     p.nslab = 0;
   }
-  p.npart = p.nslab * p.rgroups;
+  p.npart = std::max(p.nslab * p.spp, p.nslab_lj) * p.rgroups;
   size_t off = 0;
   // The bf16 contract's operands and constants; the fp32 plans' split operands.
   p.off_musw = off;    off = align256(off + (bf16 ? (size_t)p.KP * p.FP * sizeof(float) : 0));
   p.off_kclin = off;   off = align256(off + (bf16 ? (size_t)p.KP * sizeof(double) : 0));
   p.off_mu3 = off;     off = align256(off + (bf16 ? 0 : (size_t)p.KP * (p.DP / 8) * 4 * 2 * sizeof(bf16x8)));
   p.off_kcx6 = off;    off = align256(off + (bf16 ? 0 : (size_t)p.KP * sizeof(double)));
-  p.off_kcx6lin = off; off = align256(off + (bf16 ? 0 : (size_t)p.KP * sizeof(double)));
   p.off_rowstat = off; off = align256(off + (size_t)(N > 0 ? N : 0) * sizeof(double));
-  p.off_part_mu = off; off = align256(off + (size_t)p.npart * p.KP * p.DP * sizeof(float));
+  p.off_part_mu = off;
+  if (p.screen) {
+    // Read by pass 1 only, so they share the space of the slab partials pass 2 writes
+    // after it: the screening operands and error bounds, and the list of rows near
+    // several blocks (its length first).
+    size_t so = off;
+    p.off_scop = so; so = align256(so + (size_t)p.KB * screen_chunks(p.DP, true) * 64 * 16);
+    p.off_sce = so;  so = align256(so + (size_t)p.KB * sizeof(float4));
+    p.off_list = so; so = align256(so + kListBase * sizeof(int) + (size_t)N * sizeof(int));
+    p.off_probe = so; so = align256(so + kProbeBytes);
+    off = so;
+  }
+  off = std::max(off, align256(p.off_part_mu + (size_t)p.npart * p.KP * p.DP * sizeof(float)));
   p.off_part_sq = off; off = align256(off + (size_t)p.npart * p.KP * p.DP * sizeof(float));
   p.off_part_nk = off; off = align256(off + (size_t)p.npart * p.KP * sizeof(float));
   // One log-joint tile per pass-1 wave (the grid's 32-row tiles, rounded up to 4);
@@ -260,7 +288,10 @@ DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   const size_t ptiles = p.autolj ? (size_t)round_up(cdiv(N, 32), 4) : 0;
   p.off_xsplit = off;  off = align256(off + ptiles * ljd_xsplit_bytes(p.DP));
   p.off_zpair = off;   off = align256(off + ptiles * 32 * sizeof(float2));
-  p.off_probe = off;   off = align256(off + (p.autolj ? probe_bytes() : 0));
+  if (p.nprobe > 0 && !p.screen) { p.off_probe = off; off = align256(off + kProbeBytes); }
+  // The call's state words.  (The screened pass 1's need words are the masks' first words,
+  // the faint pairs' the second.)
+  p.off_state = off;   off = align256(off + (p.nprobe > 0 ? state_bytes(p.KB) : 0));
   p.total = off;
   return p;
 }
@@ -301,84 +332,168 @@ constexpr size_t x6_lds_bytes() {
 }
 
 // Prologue of that pass: the split operands [kb][chunk][split 0..2, offset][lane] and
-// C'_k in the accumulator's row order.  One 64-thread block per 32 components.
-__global__ __launch_bounds__(64) void diag_x6_prep(const float* __restrict__ mu, int64_t ldmu,
+// C'_k in the accumulator's row order.  One workgroup of kPrepWaves waves per 32
+// components, the chunks dealt to the waves, each lane forming the exponentials of its
+// own four dimensions (one wave walking all chunks, every lane forming all eight and the
+// constants' again, took 35 us at K = 1024, D = 96; 9 us here).
+constexpr int kPrepWaves = 8;
+constexpr int kPrepChunks = 16;   // chunks whose sums are kept at a time
+__global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __restrict__ mu, int64_t ldmu,
                                                    const float* __restrict__ lss, int64_t ldlss, int64_t K,
                                                    int D, int DP, const float* __restrict__ lpi,
                                                    bf16x8* __restrict__ mu3, double* __restrict__ kc_x6,
-                                                   double* __restrict__ kc_x6lin, unsigned* __restrict__ ljcount) {
-  __shared__ double sC[32];
+                                                   unsigned* __restrict__ ljcount, bf16x8* __restrict__ sc_op,
+                                                   float4* __restrict__ sc_e, unsigned* __restrict__ list_count,
+                                                   unsigned* __restrict__ state) {
+  __shared__ double sC[32], sO[kPrepChunks][32], sL[kPrepChunks][32], sW[kPrepChunks][32], sV[kPrepChunks][32];
   const int kb = blockIdx.x;
-  const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Pass 1 counts the needed row pairs of the sparse log-joint into these.
-  if (ljcount && kb == 0) ljcount[lane] = 0u;
+  if (ljcount && kb == 0 && wave == 0) ljcount[lane] = 0u;
+  if (list_count && kb == 0 && tid == 0) *list_count = 0u;
+  if (state && tid == 0) {
+    if (kb == 0) state[kStateDone] = 0u;
+    state[kStateAlive + kb] = 0u;
+  }
   const int64_t comp = (int64_t)kb * 32 + c;
   const bool valid = comp < K;
-  const int NQ = DP / 8;
-  double osum = 0.0;
-  for (int q = 0; q < NQ; ++q) {
-    f32x4 fw = zero4(), fv = zero4();
-    double o = 0.0;
-    if (valid) {
-#pragma unroll 8
-      for (int d = 8 * q; d < 8 * q + 8 && d < D; ++d) {
-        const double m = (double)mu[comp * ldmu + d];
-        const double w = 0.5 * exp(-(double)lss[comp * ldlss + d]) * kLog2e;
-        o = fma(m * m, w, o);
-        const int e = d - 8 * q - 4 * g;
-        if (e >= 0 && e < 4) {
-          fw[e] = (float)(-w);
-          fv[e] = (float)(2.0 * m * w);
-        }
+  const int NQ = DP / 8, NC = DP / 8 + 1;   // NC: the screening's chunks (16 x, then 16 x^2, then constants)
+  const float* mrow = mu + (valid ? comp : 0) * ldmu;
+  const float* lrow = lss + (valid ? comp : 0) * ldlss;
+  double osum = 0.0, qs = 0.0, lsum = 0.0, w2 = 0.0, v2 = 0.0;
+  for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
+    const int q1 = q0 + kPrepChunks < NQ ? q0 + kPrepChunks : NQ;
+    for (int q = q0 + wave; q < q1; q += kPrepWaves) {
+      const int d0 = 8 * q + 4 * g;
+      float fm[4], fl[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = d0 + e < D ? d0 + e : D - 1;
+        fm[e] = mrow[d];
+        fl[e] = lrow[d];
       }
-    }
-    bf16x8 s[3];
-    split3_bf16(fw, fv, s);
-    bf16x8* dst = mu3 + ((int64_t)kb * NQ + q) * 4 * 64 + lane;
+      f32x4 fw = zero4(), fv = zero4();
+      double o = 0.0, ls = 0.0, sw = 0.0, sv = 0.0;
 #pragma unroll
-    for (int t = 0; t < 3; ++t) dst[t * 64] = s[t];
-    const float of = (float)o;
-    osum += (double)of;
-    f32x4 ov = zero4();
-    if (g == 0) ov.x = -of;
-    bf16x8 so[3];
-    split3_bf16(ov, zero4(), so);
-    bf16x8 off;
+      for (int e = 0; e < 4; ++e) {
+        const bool in = valid && d0 + e < D;
+        const double m = in ? (double)fm[e] : 0.0, l = in ? (double)fl[e] : 0.0;
+        const double w = in ? 0.5 * exp(-l) * kLog2e : 0.0, v = 2.0 * m * w;
+        o = fma(m * m, w, o);
+        ls += l;
+        sw = fma(w, w, sw);
+        sv = fma(v, v, sv);
+        fw[e] = (float)(-w);
+        fv[e] = (float)v;
+      }
+      o += __shfl_xor(o, 32);   // both halves' dimensions (the sum commutes)
+      ls += __shfl_xor(ls, 32);
+      sw += __shfl_xor(sw, 32);
+      sv += __shfl_xor(sv, 32);
+      bf16x8 s[3];
+      split3_bf16(fw, fv, s);
+      bf16x8* dst = mu3 + ((int64_t)kb * NQ + q) * 4 * 64 + lane;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) off[e] = (__bf16)0.0f;
-    if (g == 0) {
+      for (int t = 0; t < 3; ++t) dst[t * 64] = s[t];
+      if (sc_op) {
+        // The screening's lanes take 8 dimensions: chunk q is half of its chunk q / 2.
+        unsigned* po = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
+        unsigned* pw = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + NQ / 2 + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
+        *reinterpret_cast<uint2*>(po) = uint2{bf16_pair(f32x2{fv.x, fv.y}), bf16_pair(f32x2{fv.z, fv.w})};
+        *reinterpret_cast<uint2*>(pw) = uint2{bf16_pair(f32x2{fw.x, fw.y}), bf16_pair(f32x2{fw.z, fw.w})};
+      }
+      f32x4 ov = zero4();
+      if (g == 0) ov.x = -(float)o;
+      bf16x8 so[3];
+      split3_bf16(ov, zero4(), so);
+      bf16x8 off;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) off[e] = (__bf16)0.0f;
       off[0] = so[0][0];
       off[1] = so[1][0];
       off[2] = so[2][0];
-    }
-    dst[3 * 64] = off;
-  }
-  if (g == 0) {
-    double C = -INFINITY;
-    if (valid) {
-      double lsum = 0.0, qs = 0.0;
-#pragma unroll 8
-      for (int d = 0; d < D; ++d) {
-        const double l = (double)lss[comp * ldlss + d];
-        const double m = (double)mu[comp * ldmu + d];
-        lsum += l;
-        qs = fma(m * m, 0.5 * exp(-l) * kLog2e, qs);
+      dst[3 * 64] = off;
+      if (g == 0) {
+        sO[q - q0][c] = o;
+        sL[q - q0][c] = ls;
+        sW[q - q0][c] = sw;
+        sV[q - q0][c] = sv;
       }
-      C = ((double)lpi[comp] - 0.5 * ((double)D * kLog2Pi + lsum)) * kLog2e - qs + osum;
     }
-    sC[c] = C;
-    kc_x6lin[comp] = C;   // component order, for the gathering pass 2
+    __syncthreads();
+    if (tid < 32) {
+      for (int q = 0; q < q1 - q0; ++q) {
+        const double o = sO[q][c];
+        qs += o;
+        osum += (double)(float)o;
+        lsum += sL[q][c];
+        w2 += sW[q][c];
+        v2 += sV[q][c];
+      }
+    }
+    if (q1 < NQ) __syncthreads();
   }
-  __syncthreads();
+  if (wave != 0) return;
+  double C0 = -INFINITY;   // C'_k without the centring offsets
+  double eW = 0.0, eV = 0.0, eC = 0.0;   // the component's part of the screening's error bound
+  if (g == 0) {
+    if (valid) C0 = ((double)lpi[comp] - 0.5 * ((double)D * kLog2Pi + lsum)) * kLog2e - qs;
+    sC[c] = valid ? C0 + osum : C0;
+    if (valid) {
+      eW = sqrt(w2);
+      eV = sqrt(v2);
+      eC = C0 == -INFINITY ? 0.0 : fabs(C0);
+      // A component whose constants are not ordinary numbers gets no finite bound: every
+      // row then needs its block, and the exact passes see it.
+      if (!(eW < 1e30) || !(eV < 1e30) || !(eC < 1e30)) eC = INFINITY;
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
+  if (sc_op) {
+    // The constants' chunk: C in three parts against screen_pairs' ones (second half).
+    const double C = __shfl(C0, c);
+    f32x4 lo = zero4();
+    lo.x = !valid || C == -INFINITY ? -1e30f : (float)C;
+    bf16x8 sp[3], a;
+    split3_bf16(lo, zero4(), sp);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = (__bf16)0.0f;
+    if (g == 1) {
+      a[0] = sp[0][0];
+      a[1] = sp[1][0];
+      a[2] = sp[2][0];
+    }
+    sc_op[((int64_t)kb * NC + NC - 1) * 64 + lane] = a;
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) {
+      eW = fmax(eW, __shfl_xor(eW, o));
+      eV = fmax(eV, __shfl_xor(eV, o));
+      eC = fmax(eC, __shfl_xor(eC, o));
+    }
+    if (lane == 0)
+      sc_e[kb] = make_float4((float)(eV * 0x1.06p-8), (float)(eW * 0x1.06p-8), (float)(eC * 0x1p-14 + 1.0), 0.0f);
+  }
   if (lane < 32) {
     const int i = lane & 15, gg = lane >> 4;
     kc_x6[(int64_t)kb * 32 + gg * 16 + i] = sC[acc_row(i, gg)];
   }
 }
 
+// Where kc_x6 holds component c of a block (entry 16 g + i is component acc_row(i, g)).
+__host__ __device__ constexpr int kc_x6_index(int c) { return 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3); }
+
 // What pass 1 leaves for pass 2 besides logZ2.
 constexpr int kLjmStore = 1;   // the stored log-joint, its half-block maxima and need masks
 constexpr int kLjmNeed = 2;    // need masks only (the default plan)
+
+// logZ2 from the (max, sum) pairs of a row's two halves of the components.
+__device__ __forceinline__ double merge_halves(const double (&m)[2], const float (&s)[2]) {
+  const double mn = fmax(m[0], m[1]);
+  const double ms = (mn == -INFINITY) ? 0.0 : mn;
+  const float tot = s[0] * fast_exp2((float)(m[0] - ms)) + s[1] * fast_exp2((float)(m[1] - ms));
+  return mn + (double)log2f(tot);
+}
 
 template <int DP, int LJM, bool ST = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(kAccThreads, kAccThreads), amdgpu_waves_per_eu(2, 2)))
@@ -386,8 +501,8 @@ void diag_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
                  const bf16x8* __restrict__ mu3, const double* __restrict__ kc_x6, int KB,
                  float* __restrict__ logZ, double* __restrict__ rowstat, float* __restrict__ lj,
                  float* __restrict__ ljmax, unsigned* __restrict__ ljmask, unsigned* __restrict__ ljcount,
-                 int dense, int rexact, ProbeSel probe, float* __restrict__ ljd, __bf16* __restrict__ xsplit,
-                 float2* __restrict__ zpair) {
+                 int dense, int rexact, const int* __restrict__ sel, float* __restrict__ ljd,
+                 __bf16* __restrict__ xsplit, float2* __restrict__ zpair, const int* __restrict__ list, int64_t few) {
   constexpr bool LJ = LJM == kLjmStore;
   constexpr int NQ = DP / 8;              // chunks of 8 dimensions (16 features)
   constexpr int NQH = NQ / 2;             // per half
@@ -409,15 +524,93 @@ void diag_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
   const int rg = wave & 3, h = wave >> 2;
-  const int64_t tile = (int64_t)blockIdx.x * kWaves + rg;   // 32-row tile
-  const int64_t row = tile * 32 + c;
-  const bool valid = row < N;
   // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO (default plan) is the ST
   // instance: it also writes every log-joint tile, the rows' feature parts and logZ2
-  // pairs for diag_accum_ljt.  Both instances are launched; the probe's counts let
+  // pairs for diag_accum_ljt.  Both instances are launched; the probe's choice lets
   // one of them run.
   static_assert(!ST || LJM == kLjmNeed, "the stored branch is the default plan's");
-  if (probe.count != nullptr && probe_selects(probe) != ST) return;
+  const int mode = call_mode(sel);
+  if (sel != nullptr && (mode == kModeStored) != ST) return;
+  // After the screening (screen_pairs) only the rows on its list are left, the listed
+  // rows taking the place of rows 0 .. n - 1; it has written the need masks.
+  const bool listed = LJM == kLjmNeed && !ST && mode == kModeScreen;
+  const int64_t nrow = listed ? (int64_t)(unsigned)list[0] : N;
+  if constexpr (LJM == kLjmNeed && !ST) {
+    if (listed && nrow <= few) {
+      // A short list: a workgroup per 32 rows, whose waves contract eight blocks at a
+      // time and then take turns to add theirs to the row's running (max, sum) pairs, in
+      // block order: the same operations on the same values, so the same bits.
+      if ((int64_t)blockIdx.x * 32 >= nrow) return;   // uniform over the workgroup
+      double* smx = reinterpret_cast<double*>(lds_raw);   // [half][64] running max of the lane's half
+      float* ssm = reinterpret_cast<float*>(smx + 128);   // [half][64] and sum
+      const bool ok = (int64_t)blockIdx.x * 32 + c < nrow;
+      const int64_t r = ok ? (int64_t)list[kListBase + (int64_t)blockIdx.x * 32 + c] : 0;
+      const bf16x8 ones = x6c_ones(lane);
+      for (int kb0 = 0; kb0 < KB; kb0 += kAccWaves) {
+        const int kb = kb0 + wave;
+        double ll[16];
+        if (kb < KB) {
+          f32x16 sh[2];
+#pragma unroll
+          for (int H = 0; H < 2; ++H) {
+            bf16x8 xf[NQH][3];
+#pragma unroll
+            for (int qq = 0; qq < NQH; ++qq) {
+              const f32x4 x = load_row4(X, ldx, r, 8 * (H * NQH + qq) + 4 * g, D, ok);
+              split3_bf16(x * x, x, xf[qq]);
+            }
+            const bf16x8* mp = mu3 + (int64_t)kb * BLK + H * NQH * 4 * 64 + lane;
+            sh[H] = x6c_tile<NQH, 2>([&](int q, int t) { return mp[(q * 4 + t) * 64]; }, xf, ones);
+          }
+          const double* kp = kc_x6 + (int64_t)kb * 32 + g * 16;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) ll[i] = kp[i] + (double)(sh[0][i] + sh[1][i]);
+        }
+        for (int w = 0; w < kAccWaves && kb0 + w < KB; ++w) {
+          if (w == wave) {
+#pragma unroll
+            for (int H = 0; H < 2; ++H) {
+              const double m0 = kb > 0 ? smx[H * 64 + lane] : -INFINITY;
+              const float s0 = kb > 0 ? ssm[H * 64 + lane] : 0.0f;
+              double bm = -INFINITY;
+#pragma unroll
+              for (int j = 0; j < 8; ++j) bm = fmax(bm, ll[8 * H + j]);
+              const double mn = fmax(m0, bm);
+              const double ms = (mn == -INFINITY) ? 0.0 : mn;
+              float acc = s0 * fast_exp2((float)(m0 - ms));
+#pragma unroll
+              for (int j = 0; j < 8; ++j) acc += fast_exp2((float)(ll[8 * H + j] - ms));
+              smx[H * 64 + lane] = mn;
+              ssm[H * 64 + lane] = acc;
+            }
+          }
+          lds_barrier();
+        }
+      }
+      if (wave == 0) {
+        double m1[2];
+        float s1[2];
+#pragma unroll
+        for (int H = 0; H < 2; ++H) {
+          const double mx = smx[H * 64 + lane], mo = __shfl_xor(mx, 32);
+          const float sm = ssm[H * 64 + lane], so = __shfl_xor(sm, 32);
+          m1[H] = fmax(mx, mo);
+          const double ms = (m1[H] == -INFINITY) ? 0.0 : m1[H];
+          s1[H] = sm * fast_exp2((float)(mx - ms)) + so * fast_exp2((float)(mo - ms));
+        }
+        const double lz2 = merge_halves(m1, s1);
+        if (ok && g == 0) {
+          rowstat[r] = lz2;
+          if (logZ) logZ[r] = (float)(lz2 * kLn2);
+        }
+      }
+      return;
+    }
+    if (listed && (int64_t)blockIdx.x * kWaves * 32 >= nrow) return;   // uniform over the workgroup
+  }
+  const int64_t tile = (int64_t)blockIdx.x * kWaves + rg;   // 32-row tile
+  const bool valid = tile * 32 + c < nrow;
+  const int64_t row = (listed && valid) ? (int64_t)list[kListBase + tile * 32 + c] : tile * 32 + c;
 
   // Blocks go global -> registers -> LDS.  Up to D = 96 through two register
   // stages: block kb + 2 is fetched while block kb is contracted and lands in LDS at
@@ -534,7 +727,7 @@ void diag_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
           run_max = fmaxf(run_max, R);
           const bool nb = valid && (dense != 0 || !(R - run_max < -kLjSkipGap));
           const unsigned bits = (unsigned)__builtin_amdgcn_ballot_w64(nb);
-          if (lane == 0) ljmask[(tile * KB + kb) * 2 + H] = bits;
+          if (lane == 0 && !listed) ljmask[(tile * KB + kb) * 2 + H] = bits;
         }
       }
       if (MB == 1) lds_barrier();
@@ -597,6 +790,7 @@ void diag_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
       zpair[tile * 32 + c] = make_float2(zh, zl);
     }
   }
+  if (listed) return;
   // Each wave's need masks from its own maxima; pass 2 ORs the two words.
   if constexpr (LJ) {
     if (g == 0)
@@ -619,14 +813,13 @@ void diag_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
 }
 
 // ---------------------------------------------------------------------------
-// The probe of FGMM_FLAG_STORE_LOGJOINT_AUTO: one workgroup per sampled 32-row tile;
-// its waves take the component blocks in turn and form each row's block maximum R
-// of the log-joint in LDS.  An estimate suffices here, so the contraction keeps two
-// of pass 1's seven steps per 16-feature chunk (the centring step and x1 w1), each
-// row's chunks whole in one wave.  Then, per row, the blocks with R >= M -
-// kLjNeedGap (M the row's largest R) are counted: an estimate of the pairs pass 1
-// will mark as needed, since logZ2 >= M.  The tile's count is written; the kernels
-// that need the choice sum the counts themselves (probe_selects).
+// The probe of FGMM_FLAG_STORE_LOGJOINT_AUTO and of the screened pass 1: one workgroup per
+// sampled 32-row tile; its waves take the component blocks in turn and form each row's
+// block maximum R of the log-joint in LDS.  An estimate suffices here, so the
+// contraction keeps two of pass 1's seven steps per 16-feature chunk (the centring step
+// and x1 w1), each row's chunks whole in one wave.  Then the pairs that need the exact
+// pass 1's bit and the rows the screening would find near several blocks are counted,
+// and the last workgroup makes the call's choice (probe_finish).
 // ---------------------------------------------------------------------------
 constexpr int kProbeWaves = 16;
 template <int DP>
@@ -634,38 +827,55 @@ __global__ __launch_bounds__(64 * kProbeWaves) void diag_store_probe(const float
                                                                      int64_t N, int D,
                                                                      const bf16x8* __restrict__ mu3,
                                                                      const double* __restrict__ kc_x6, int KB,
-                                                                     int ntile, unsigned* __restrict__ count) {
-  constexpr int NQ = DP / 8;
-  __shared__ float rmax[kProbeMaxKB * 32];
-  __shared__ unsigned part[kProbeWaves];
+                                                                     const float4* __restrict__ sc_e, int ntile,
+                                                                     ProbeRule rule, unsigned* __restrict__ count,
+                                                                    unsigned* __restrict__ state) {
+  constexpr int NQ = DP / 8, V4 = DP / 4, XRS = DP + 4;
+  // The rows' block maxima and the screening's error bounds; the tile's rows, loaded once
+  // by all waves, in fp32 over the bounds' space.
+  __shared__ float rmax[kProbeMaxKB * 32], rerr[kProbeMaxKB * 32];
+  __shared__ ProbeScratch sh;
+  float* xt = rerr;                    // [32][XRS]
+  float* sq = rerr + 32 * XRS;         // [32][V4 + 1][2]
+  static_assert(32 * XRS + 64 * (V4 + 1) <= kProbeMaxKB * 32, "probe LDS");
   const int s = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
   const int64_t tile = probe_tile(s, N, ntile);
-  const int64_t row = tile * 32 + c;
-  const bool valid = row < N;
-
+  const bool valid = tile * 32 + c < N;
+  for (int idx = tid; idx < 32 * V4; idx += 64 * kProbeWaves) {
+    const int rr = idx / V4, v = idx % V4;
+    const int64_t xr = tile * 32 + rr;
+    const f32x4 x = load_row4(X, ldx, xr, 4 * v, D, xr < N), y = x * x;
+    *reinterpret_cast<f32x4*>(xt + rr * XRS + 4 * v) = x;
+    *reinterpret_cast<float2*>(sq + (rr * (V4 + 1) + v) * 2) =
+        make_float2((y.x + y.y) + (y.z + y.w), fmaf(y.x, y.x, fmaf(y.y, y.y, fmaf(y.z, y.z, y.w * y.w))));
+  }
+  __syncthreads();
   bf16x8 xh[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
-    const f32x4 x = load_row4(X, ldx, row, 8 * q + 4 * g, D, valid);
+    const f32x4 x = *reinterpret_cast<const f32x4*>(xt + c * XRS + 8 * q + 4 * g);
     xh[q] = to_bf16x8(x * x, x);
   }
+  float xs = 0.0f, xq = 0.0f;
+#pragma unroll
+  for (int v = 0; v < V4; ++v) {
+    xs += sq[(c * (V4 + 1) + v) * 2];
+    xq += sq[(c * (V4 + 1) + v) * 2 + 1];
+  }
+  const float nx = sqrtf(xs), ny = sqrtf(xq);
+  __syncthreads();   // the rows are read: rerr may be written
   const bf16x8 ones = x6c_ones(lane);
   for (int kb = wave; kb < KB; kb += kProbeWaves) {
+    const float4 e = sc_e ? sc_e[kb] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const bf16x8* mp = mu3 + (int64_t)kb * NQ * 4 * 64 + lane;
-    bf16x8 a0[NQ], a3[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      a0[q] = mp[(q * 4 + 0) * 64];
-      a3[q] = mp[(q * 4 + 3) * 64];
-    }
     f32x16 acc[4] = {zero16(), zero16(), zero16(), zero16()};
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      acc[q & 3] = mfma_bf16(a3[q], ones, acc[q & 3]);
-      acc[q & 3] = mfma_bf16(a0[q], xh[q], acc[q & 3]);
+      acc[q & 3] = mfma_bf16(mp[(q * 4 + 3) * 64], ones, acc[q & 3]);
+      acc[q & 3] = mfma_bf16(mp[(q * 4 + 0) * 64], xh[q], acc[q & 3]);
     }
     const double* kp = kc_x6 + (int64_t)kb * 32 + g * 16;
     double bm = -INFINITY;
@@ -675,25 +885,12 @@ __global__ __launch_bounds__(64 * kProbeWaves) void diag_store_probe(const float
       bm = fmax(bm, kp[i] + (double)xm);
     }
     const float R = lj_row_max(bm);
-    if (g == 0) rmax[kb * 32 + c] = R;
+    if (g == 0) {
+      rmax[kb * 32 + c] = R;
+      rerr[kb * 32 + c] = sc_e ? fmaf(e.x, nx, fmaf(e.y, ny, e.z)) : 0.0f;
+    }
   }
-  __syncthreads();
-  // Row c's maximum and needed blocks; the waves split the blocks again.
-  unsigned need = 0;
-  if (g == 0 && valid) {
-    float M = -INFINITY;
-    for (int kb = 0; kb < KB; ++kb) M = fmaxf(M, rmax[kb * 32 + c]);
-    for (int kb = wave; kb < KB; kb += kProbeWaves) need += (rmax[kb * 32 + c] - M >= -kLjNeedGap) ? 1u : 0u;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) need += __shfl_xor(need, o);
-  if (lane == 0) part[wave] = need;
-  __syncthreads();
-  if (tid == 0) {
-    unsigned tot = 0;
-    for (int w = 0; w < kProbeWaves; ++w) tot += part[w];
-    count[s] = tot;
-  }
+  probe_finish(rmax, rerr, sh, KB, valid, nx, sc_e != nullptr, s, ntile, rule, count, state);
 }
 
 // ---------------------------------------------------------------------------
@@ -1582,9 +1779,12 @@ __host__ size_t x6_lds_bytes_rt(int DP) {
 // fp32 row stride of the X tiles: rows 8 apart (the two lane-halves of a B operand)
 // and the 16-byte row accesses of the contraction fall in distinct banks.
 __host__ __device__ constexpr int gather_rs(int DP) { return DP + 4; }
+constexpr int kGatherSt = 20;   // row stride (floats) of half an S tile in LDS
 
 __host__ __device__ constexpr size_t gather_lds_bytes(int DP) {
   return (size_t)(DP / 8) * 4 * 64 * 16                          // mu block (bf16x8 operands)
+         + (size_t)32 * sizeof(double)                            // its constants
+         + (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float)  // half an S tile per wave
          + (size_t)kGatherWaves * 32 * gather_rs(DP) * 4          // X tile per wave
          + (size_t)kGatherWaves * 32 * sizeof(double)              // logZ2 per wave
          + (size_t)kGatherWaves * 64 * sizeof(int);                // row queue per wave
@@ -1601,22 +1801,31 @@ template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kGatherWaves, 64 * kGatherWaves),
                           amdgpu_waves_per_eu(gather_waves_per_simd(DP), gather_waves_per_simd(DP))))
 void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
-                       const bf16x8* __restrict__ mu3, const double* __restrict__ kc_x6lin, int KB, int KP,
-                       const double* __restrict__ rowstat, const uint2* __restrict__ need, int nslab,
+                       const bf16x8* __restrict__ mu3, const double* __restrict__ kc_x6, int KB, int KP,
+                       double* __restrict__ rowstat, const uint2* __restrict__ need, int nslab,
                        int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_sq,
-                       float* __restrict__ part_nk, int dense, ProbeSel sel) {
+                       float* __restrict__ part_nk, int dense, const int* __restrict__ sel,
+                       float* __restrict__ logZ, int own_lse, int lse_only, unsigned* __restrict__ alive,
+                       int faint) {
   constexpr int NQ = DP / 8;      // chunks of 8 dimensions (16 features)
   constexpr int NQH = NQ / 2;
   constexpr int NJ = DP / 32;
   constexpr int RS = gather_rs(DP);
+  constexpr int PW = gather_parts(DP);
   constexpr int BLK = NQ * 4 * 64;
   static_assert(NQ % 2 == 0, "two halves of chunks");
   // The stored branch's diag_accum_ljt takes the call when the probe selects it.
-  if (probe_selects(sel)) return;
+  const int mode = call_mode(sel);
+  if (mode == kModeStored || (mode == kModeDefault && (lse_only || faint))) return;
+  // After the screened pass 1 the rows near one block only (the pairs in both words) have
+  // no logZ2 yet: it is formed here.
+  const bool screened = mode == kModeScreen, fused = screened && own_lse;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   unsigned char* lp = lds_raw;
   bf16x8* mu_l = reinterpret_cast<bf16x8*>(lp);  lp += (size_t)BLK * sizeof(bf16x8);
+  double* kc_l = reinterpret_cast<double*>(lp);  lp += 32 * sizeof(double);
+  float* st_all = reinterpret_cast<float*>(lp);  lp += (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float);
   float* xt_all = reinterpret_cast<float*>(lp);  lp += (size_t)kGatherWaves * 32 * RS * 4;
   double* rs_all = reinterpret_cast<double*>(lp); lp += (size_t)kGatherWaves * 32 * sizeof(double);
   int* q_all = reinterpret_cast<int*>(lp);
@@ -1626,7 +1835,14 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   const int c = lane & 31, g = lane >> 5;
   int sg, kb;
   if (!gather_item(blockIdx.x, gather_groups(nslab), KB, sg, kb)) return;   // uniform over the workgroup
+  if (faint) {
+    // The second run after the screened pass 1: the block's faint pairs, where one of its
+    // components has too small an Nk to absorb them (one of zero weight has none).
+    const bool none = kc_x6[(int64_t)kb * 32 + kc_x6_index(c)] == -INFINITY;
+    if (((unsigned)__builtin_amdgcn_ballot_w64(!none) & ~alive[kb]) == 0u) return;   // uniform
+  }
   for (int idx = tid; idx < BLK; idx += 64 * kGatherWaves) mu_l[idx] = mu3[(int64_t)kb * BLK + idx];
+  if (tid < 32) kc_l[tid] = kc_x6[(int64_t)kb * 32 + tid];
   __syncthreads();
   const int slab = sg * kGatherWaves + wave;
   if (slab >= nslab) return;   // no barrier follows
@@ -1634,18 +1850,19 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   float* xt = xt_all + wave * 32 * RS;
   double* rs_l = rs_all + wave * 32;
   int* q_l = q_all + wave * 64;
-  const double Cc = kc_x6lin[(int64_t)kb * 32 + c];
+  const double Cc = kc_x6[(int64_t)kb * 32 + kc_x6_index(c)];
 
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
-  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32);
+  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32), t_mid = (t_begin + t_end) / 2;
 
   auto words = [&](int64_t tb) -> unsigned {
     const int64_t t = tb + lane;
     if (t >= t_end) return 0u;
     const uint2 w = need[t * KB + kb];
-    return w.x | w.y;
+    // The halves of the block, or (screened) its near and its faint pairs.
+    return !screened ? w.x | w.y : faint ? w.y & ~w.x : w.x;
   };
   int64_t tb = t_begin;
   unsigned mword = words(tb), mnext = words(tb + 64);
@@ -1666,12 +1883,18 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   // the slab spans under 2 GiB (uniform), else load_row4.
   f32x4 raw[NQ];
   double rst;
+  unsigned sgl = 0u;   // the own-pairs word of the row's tile (fused)
+  int erow = -1;
   const int64_t slab_bytes = (r_end - r_begin) * ldx * (int64_t)sizeof(float);
   const bool xbuf = D == DP && slab_bytes <= ((int64_t)1 << 31) - 256;
   const buf_rsrc xres = make_rsrc(X + r_begin * ldx, xbuf ? (uint32_t)slab_bytes : 0u);
   const buf_rsrc rres = make_rsrc(rowstat + r_begin, (uint32_t)((r_end - r_begin) * sizeof(double)));
+  const buf_rsrc sres = make_rsrc(fused ? need + t_begin * KB + kb : nullptr,
+                                  fused ? (uint32_t)((t_end - t_begin) * KB * sizeof(uint2)) : 0u);
   auto issue = [&](int e) {
     const bool ok = e >= 0;
+    erow = e;
+    sgl = buf_load_u32(sres, buf_off(ok ? (e >> 5) * KB * (int)sizeof(uint2) + 4 : kBufOob));
     if (xbuf) {
       const int off = buf_off(ok ? (int)((int64_t)e * ldx * (int64_t)sizeof(float)) + 16 * g : kBufOob);
 #pragma unroll
@@ -1695,14 +1918,54 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   float nk = 0.0f;
   const bf16x8 ones = x6c_ones(lane);
 
+  // Partial p of the slab (the faint pass adds to the first), and the sums start again.
+  auto store = [&](int p) __attribute__((always_inline)) {
+    nk += __shfl_xor(nk, 32);
+    const int64_t kbase = (int64_t)(slab * PW + p) * KP + (int64_t)kb * 32;
+    const int64_t o0 = kbase * DP + 4 * g * DP + c;
+    float *pm = part_mu + o0, *pq = part_sq + o0;
+    if (faint) {
+      nk += part_nk[kbase + c];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          accx[j][i] += pm[acc_row(i, 0) * DP + 32 * j];
+          accq[j][i] += pq[acc_row(i, 0) * DP + 32 * j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        pm[acc_row(i, 0) * DP + 32 * j] = accx[j][i];
+        pq[acc_row(i, 0) * DP + 32 * j] = accq[j][i];
+      }
+      accx[j] = zero16();
+      accq[j] = zero16();
+    }
+    if (g == 0) part_nk[kbase + c] = nk;
+    if (screened && !faint) mark_alive(alive, kb, nk);
+    nk = 0.0f;
+  };
+
   int e;
   int cnt = take(e);
   if (cnt > 0) issue(e);
+  // Above D = 64 a partial ends once half of the slab's tiles are queued.
+  const int parts = (lse_only || faint) ? 1 : PW;
+#pragma unroll 1
+  for (int part = 0; part < parts; ++part) {
   while (cnt > 0) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the previous tile's LDS reads are done
 #pragma unroll
     for (int q = 0; q < NQ; ++q) *reinterpret_cast<f32x4*>(xt + c * RS + 8 * q + 4 * g) = raw[q];
     if (g == 0) rs_l[c] = rst;
+    const bool own = fused && erow >= 0 && ((sgl >> (erow & 31)) & 1u);
+    const bool owns = fused && __builtin_amdgcn_ballot_w64(own) != 0;
+    const int64_t orow = r_begin + erow;
     int en;
     const int cnt_next = take(en);
     if (cnt_next > 0) issue(en);
@@ -1716,6 +1979,54 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     const f32x16 s0 = x6c_tile_rows_fn<NQH, 2>(loadX, ones, [&](int q, int t) { return mu_l[(q * 4 + t) * 64 + lane]; });
     const f32x16 s1 = x6c_tile_rows_fn<NQH, 2>([&](int q, bf16x8 (&xa)[3]) { loadX(NQH + q, xa); }, ones,
                                                [&](int q, int t) { return mu_l[((NQH + q) * 4 + t) * 64 + lane]; });
+    if (owns) {
+      // logZ2 of the tile's own rows, over the block's 32 components as pass 1 forms it
+      // (lane = row, the 16 components of each of its two waves in register order, the
+      // lane-halves merged, then the waves): every other block's terms are exactly zero
+      // there, so these are the same bits.  S passes through LDS 16 components at a time.
+      float* st = st_all + wave * 32 * kGatherSt;
+      double m1[2];
+      float t1[2];
+#pragma unroll
+      for (int H = 0; H < 2; ++H) {
+        if ((c >> 4) == H) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) st[acc_row(i, g) * kGatherSt + (c & 15)] = s0[i] + s1[i];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        double ll[8], bm = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(st + c * kGatherSt + 8 * j + 4 * g);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            ll[4 * j + e] = kc_l[g * 16 + 8 * H + 4 * j + e] + (double)v[e];
+            bm = fmax(bm, ll[4 * j + e]);
+          }
+        }
+        const double mb = (bm == -INFINITY) ? 0.0 : bm;
+        float sm = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sm += fast_exp2((float)(ll[j] - mb));
+        const double mo = __shfl_xor(bm, 32);
+        const float so = __shfl_xor(sm, 32);
+        m1[H] = fmax(bm, mo);
+        const double ms = (m1[H] == -INFINITY) ? 0.0 : m1[H];
+        t1[H] = sm * fast_exp2((float)(bm - ms)) + so * fast_exp2((float)(mo - ms));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      const double lz2 = merge_halves(m1, t1);
+      if (own && g == 0) {
+        rs_l[c] = lz2;
+        rowstat[orow] = lz2;
+        if (logZ) logZ[orow] = (float)(lz2 * kLn2);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    if (lse_only) {
+      cnt = cnt_next;
+      continue;
+    }
     float r[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -1769,19 +2080,11 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       }
     }
     cnt = cnt_next;
+    if (part + 1 < parts && tb >= t_mid) break;
   }
-
-  nk += __shfl_xor(nk, 32);
-  const int64_t kbase = (int64_t)slab * KP + (int64_t)kb * 32;
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      part_mu[(kbase + acc_row(i, g)) * DP + 32 * j + c] = accx[j][i];
-      part_sq[(kbase + acc_row(i, g)) * DP + 32 * j + c] = accq[j][i];
-    }
+  if (lse_only || (faint && qt == 0)) return;
+  store(part);
   }
-  if (g == 0) part_nk[kbase + c] = nk;
 }
 
 // ---------------------------------------------------------------------------
@@ -1830,7 +2133,7 @@ __host__ inline int64_t ljd_grid(int nslab, int ncg) { return (int64_t)8 * cdiv(
 template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kLjdWaves, 64 * kLjdWaves), amdgpu_waves_per_eu(2, 2)))
 void diag_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xsplit, const float2* __restrict__ zpair,
-                    int64_t N, const uint2* __restrict__ need, ProbeSel sel, int KB, int KP, int nslab,
+                    int64_t N, const uint2* __restrict__ need, const int* __restrict__ sel, int KB, int KP, int nslab,
                     int64_t rows_per_slab, int ncg, float* __restrict__ part_mu, float* __restrict__ part_sq,
                     float* __restrict__ part_nk) {
   using SH = LjdShape<DP>;
@@ -1840,7 +2143,7 @@ void diag_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xsp
   constexpr int RS = SH::RS;
   constexpr int NS = SH::NS;
   constexpr int NL = SH::NLOADS;
-  if (!probe_selects(sel)) return;
+  if (call_mode(sel) != kModeStored) return;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -2012,7 +2315,7 @@ void diag_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xsp
 // ---------------------------------------------------------------------------
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kCtWaves, 64 * kCtWaves), amdgpu_waves_per_eu(1, 1)))
 void diag_accum_drange(const float* __restrict__ X, int64_t ldx, int64_t N, int D, int NQ, int DP,
-                       const bf16x8* __restrict__ mu3, const double* __restrict__ kc_x6lin, int KB, int KP,
+                       const bf16x8* __restrict__ mu3, const double* __restrict__ kc_x6, int KB, int KP,
                        const double* __restrict__ rowstat, const uint2* __restrict__ need, int nslab,
                        int64_t rows_per_slab, int ndr, float* __restrict__ part_mu, float* __restrict__ part_sq,
                        float* __restrict__ part_nk, int dense) {
@@ -2047,7 +2350,7 @@ void diag_accum_drange(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   const int nj = njr - j0 < tj ? (njr - j0 > 0 ? njr - j0 : 0) : tj;   // this wave's column tiles
   const int nqw = NQ / kCtWaves;                                       // chunks per wave
 
-  const double Cc = kc_x6lin[(int64_t)kb * 32 + c];
+  const double Cc = kc_x6[(int64_t)kb * 32 + kc_x6_index(c)];
 
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
@@ -2220,30 +2523,40 @@ void diag_accum_drange(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   }
 }
 
-// Finish: one thread per (k, d); fixed-order fp64 sums over partials, then the
-// sig identity in fp64.  Thread d == 0 also writes Nk.
-template <bool WIDE>
+// Finish: fixed-order fp64 sums over partials, then the sig identity in fp64.  A
+// workgroup takes 256 / G consecutive (k, d), G threads each over the partials in turn
+// (G = 4, 16), so the loads of a wave stay in whole lines (one wave per (k, d) over the
+// partials read a line per lane); their sums are added in order.  d == 0 also writes Nk.
+template <int G>
 __global__ __launch_bounds__(256) void diag_reduce(const float* __restrict__ part_mu,
                                                    const float* __restrict__ part_sq,
-                                                   const float* __restrict__ part_nk, int npart, int KP,
+                                                   const float* __restrict__ part_nk, PartCount parts, int KP,
                                                    int DP, int64_t K, int D, const float* __restrict__ mu,
                                                    int64_t ldmu, float* __restrict__ Nk,
                                                    float* __restrict__ mu_acc, float* __restrict__ sig_acc,
                                                    int accumulate) {
-  // WIDE: one wave per (k, d) with the partials spread over its lanes (many partials).
-  const int64_t idx = WIDE ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)
-                           : (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  if (idx >= K * D) return;
-  const int64_t k = idx / D;
-  const int d = (int)(idx % D);
-  auto sum = [&](const float* p, int64_t stride) {
-    return WIDE ? wave_strided_sum(p, npart, stride, lane) : strided_sum(p, npart, stride);
-  };
-  const double sm = sum(part_mu + k * DP + d, (int64_t)KP * DP);
-  const double sq = sum(part_sq + k * DP + d, (int64_t)KP * DP);
-  const double nk = sum(part_nk + k, KP);
-  if (WIDE && lane != 0) return;
+  constexpr int C = 256 / G;
+  __shared__ double sum[3][G][C];
+  const int np = part_count(parts);
+  const int col = threadIdx.x % C, grp = threadIdx.x / C;
+  const int64_t idx = (int64_t)blockIdx.x * C + col;
+  const bool in = idx < K * D;
+  const int64_t k = in ? idx / D : 0;
+  const int d = in ? (int)(idx - k * D) : 0;
+  const int n = grp < np ? (np - grp + G - 1) / G : 0;
+  const int64_t stride = (int64_t)KP * DP, o = grp * stride + k * DP + d;
+  sum[0][grp][col] = strided_sum(part_mu + o, n, G * stride);
+  sum[1][grp][col] = strided_sum(part_sq + o, n, G * stride);
+  sum[2][grp][col] = strided_sum(part_nk + (int64_t)grp * KP + k, n, (int64_t)G * KP);
+  __syncthreads();
+  if (grp != 0 || !in) return;
+  double sm = 0.0, sq = 0.0, nk = 0.0;
+#pragma unroll
+  for (int j = 0; j < G; ++j) {
+    sm += sum[0][j][col];
+    sq += sum[1][j][col];
+    nk += sum[2][j][col];
+  }
   const double m = (double)mu[k * ldmu + d];
   const double sg = sq - 2.0 * m * sm + m * m * nk;
   float* om = mu_acc + k * D + d;
@@ -2258,12 +2571,12 @@ __global__ __launch_bounds__(256) void diag_reduce(const float* __restrict__ par
 // fp64 and added in fp32.
 __global__ __launch_bounds__(256) void diag_reduce_atomic(const float* __restrict__ part_mu,
                                                           const float* __restrict__ part_sq,
-                                                          const float* __restrict__ part_nk, int KP, int DP,
+                                                          const float* __restrict__ part_nk, PartCount parts, int KP, int DP,
                                                           int64_t K, int D, const float* __restrict__ mu,
                                                           int64_t ldmu, float* __restrict__ Nk,
                                                           float* __restrict__ mu_acc, float* __restrict__ sig_acc) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= K * D) return;
+  if (idx >= K * D || (int)blockIdx.y >= part_count(parts)) return;
   const int64_t k = idx / D;
   const int d = (int)(idx % D);
   const int64_t pk = (int64_t)blockIdx.y * KP + k;
@@ -2311,12 +2624,17 @@ hipError_t launch_ctile(const DiagPlan& pl, const float* X, int64_t ldx, unsigne
     const int64_t items = (int64_t)pl.KB * pl.nslab * pl.ndr;
     hipLaunchKernelGGL(diag_accum_drange, dim3((unsigned)(8 * cdiv(items, 8))), dim3(64 * kCtWaves), lds2,
                        stream, X, ldx, pl.N, (int)pl.D, NQ, pl.DP, mu3,
-                       reinterpret_cast<const double*>(ws + pl.off_kcx6lin), pl.KB, pl.KP, rowstat, masks,
+                       reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, pl.KP, rowstat, masks,
                        pl.nslab, pl.rows_per_slab, pl.ndr, reinterpret_cast<float*>(ws + pl.off_part_mu),
                        reinterpret_cast<float*>(ws + pl.off_part_sq), reinterpret_cast<float*>(ws + pl.off_part_nk),
                        dense ? 1 : 0);
   }
   return hipGetLastError();
+}
+
+// The word that holds the device's choice of the call's branches (nullptr: none to make).
+const int* diag_sel(const DiagPlan& pl, unsigned char* ws) {
+  return pl.nprobe > 0 ? reinterpret_cast<const int*>(ws + pl.off_state) + kStateMode : nullptr;
 }
 
 // Up to D = 128 both plans; above, the stored plan's pass 2 (pass 1 is launch_ctile's).
@@ -2331,22 +2649,40 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
   float* pmu = reinterpret_cast<float*>(ws + pl.off_part_mu);
   float* psq = reinterpret_cast<float*>(ws + pl.off_part_sq);
   float* pnk = reinterpret_cast<float*>(ws + pl.off_part_nk);
-  // FGMM_FLAG_STORE_LOGJOINT_AUTO: the probe's counts, which pass 1 and both pass-2
-  // kernels read to select the stored branch.
-  unsigned* probe = pl.autolj ? reinterpret_cast<unsigned*>(ws + pl.off_probe) : nullptr;
-  const ProbeSel psel = probe ? ProbeSel{probe, pl.nprobe, probe_min_pairs(pl.N, pl.nprobe, pl.KB)}
-                              : ProbeSel{nullptr, 0, 0};
+  // The probe's choice (stored branch, screened pass 1, or neither), which every later
+  // kernel reads.  A dense call computes every pair, so it never screens.
+  const int* sel = diag_sel(pl, ws);
+  const bool screen = pl.screen && !dense && ldx <= kMaxScreenLdx;
+  uint2* words = pl.need ? reinterpret_cast<uint2*>(ws + pl.off_ljmask) : ljmask;
+  int* list = screen ? reinterpret_cast<int*>(ws + pl.off_list) : nullptr;
+  unsigned* alive = screen ? reinterpret_cast<unsigned*>(ws + pl.off_state) + kStateAlive : nullptr;
   if (run1) {
     const unsigned nblk1 = (unsigned)cdiv(pl.N, 32 * kWaves);
     if constexpr (diag_uses_x6(DP)) {
-      if constexpr (ljd_applies(DP)) {
-        if (pl.autolj)
-          hipLaunchKernelGGL((diag_store_probe<DP>), dim3((unsigned)pl.nprobe), dim3(64 * kProbeWaves), 0, stream,
-                             X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
-                             reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, pl.nprobe, probe);
+      if (sel)
+        hipLaunchKernelGGL((diag_store_probe<DP>), dim3((unsigned)pl.nprobe), dim3(64 * kProbeWaves), 0, stream,
+                           X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
+                           reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB,
+                           screen ? reinterpret_cast<const float4*>(ws + pl.off_sce) : nullptr, pl.nprobe,
+                           ProbeRule{screen ? (int64_t)pl.nprobe * 32 / 2 : -1,
+                                     probe_min_pairs(pl.N, pl.nprobe, pl.KB), pl.autolj ? 1 : 0},
+                           reinterpret_cast<unsigned*>(ws + pl.off_probe),
+                             reinterpret_cast<unsigned*>(ws + pl.off_state));
+      if (screen) {
+        const size_t lds = screen_lds_bytes(DP, true, pl.KB);
+        if (lds > 65536) {
+          hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&screen_pairs<DP, true>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+          if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL((screen_pairs<DP, true>), dim3((unsigned)cdiv(pl.N, 64 * kScreenWaves)),
+                           dim3(64 * kScreenWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
+                           reinterpret_cast<const bf16x8*>(ws + pl.off_scop),
+                           reinterpret_cast<const float4*>(ws + pl.off_sce), pl.KB,
+                           reinterpret_cast<unsigned*>(words), reinterpret_cast<unsigned*>(words) + 1, 2,
+                           list, sel);
       }
       const size_t lds1 = x6_lds_bytes<DP>() + (pl.rexact ? (size_t)kAccWaves * 32 * pl.KB * 2 : 0);
-      uint2* masks = pl.need ? reinterpret_cast<uint2*>(ws + pl.off_ljmask) : ljmask;
       auto launch1 = [&](auto kern) -> hipError_t {
         if (lds1 > 65536) {
           hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -2356,10 +2692,11 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
         hipLaunchKernelGGL(kern, dim3(nblk1), dim3(kAccThreads), lds1, stream, X, ldx, pl.N, (int)pl.D,
                            reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
                            reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, logZ, rowstat, lj,
-                           ljmax, reinterpret_cast<unsigned*>(masks), ljcount, dense ? 1 : 0, pl.rexact ? 1 : 0,
-                           psel, pl.autolj ? reinterpret_cast<float*>(ws + pl.off_lj) : nullptr,
+                           ljmax, reinterpret_cast<unsigned*>(words), ljcount, dense ? 1 : 0, pl.rexact ? 1 : 0,
+                           sel, pl.autolj ? reinterpret_cast<float*>(ws + pl.off_lj) : nullptr,
                            reinterpret_cast<__bf16*>(ws + pl.off_xsplit),
-                           reinterpret_cast<float2*>(ws + pl.off_zpair));
+                           reinterpret_cast<float2*>(ws + pl.off_zpair), list,
+                           std::min<int64_t>((int64_t)kFewRounds * 32 * current_device_cus(), (int64_t)nblk1 * 32));
         return hipSuccess;
       };
       hipError_t e1 = launch1(pl.lj ? &diag_lse_x6<DP, kLjmStore> : &diag_lse_x6<DP, kLjmNeed>);
@@ -2374,25 +2711,24 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
       return hipErrorInvalidValue;   // launch_ctile runs pass 1 above D = 128
     }
   }
-  if (!run2) return hipGetLastError();
+  if (!run2 && !screen) return hipGetLastError();
   const dim3 grid2((unsigned)(pl.nslab * pl.ncg));
   if constexpr (diag_uses_x6(DP)) {
     if (pl.need) {
       // With the stored branch both pass-2 kernels are launched over the same slabs and
       // partials; the probe's selector lets one of them run.
       if constexpr (ljd_applies(DP)) {
-        if (pl.autolj) {
+        if (pl.autolj && run2) {
           using SH = LjdShape<DP>;
           hipError_t ej = hipFuncSetAttribute(reinterpret_cast<const void*>(&diag_accum_ljt<DP>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)SH::lds);
           if (ej != hipSuccess) return ej;
           const int ncg = (int)cdiv(pl.KB, kLjdWaves);
-          hipLaunchKernelGGL((diag_accum_ljt<DP>), dim3((unsigned)ljd_grid(pl.nslab, ncg)), dim3(64 * kLjdWaves),
+          hipLaunchKernelGGL((diag_accum_ljt<DP>), dim3((unsigned)ljd_grid(pl.nslab_lj, ncg)), dim3(64 * kLjdWaves),
                              SH::lds, stream, reinterpret_cast<const float*>(ws + pl.off_lj),
                              reinterpret_cast<const __bf16*>(ws + pl.off_xsplit),
                              reinterpret_cast<const float2*>(ws + pl.off_zpair), pl.N,
-                             reinterpret_cast<const uint2*>(ws + pl.off_ljmask), psel, pl.KB, pl.KP, pl.nslab,
-                             pl.rows_per_slab, ncg, pmu, psq, pnk);
+                             words, sel, pl.KB, pl.KP, pl.nslab_lj, pl.rows_per_slab_lj, ncg, pmu, psq, pnk);
         }
       }
       constexpr size_t lds = gather_lds_bytes(DP);
@@ -2400,12 +2736,16 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&diag_accum_gather<DP>),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(diag_accum_gather<DP>, dim3((unsigned)gather_grid(pl.nslab, pl.KB)),
-                         dim3(64 * kGatherWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
-                         reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
-                         reinterpret_cast<const double*>(ws + pl.off_kcx6lin), pl.KB, pl.KP, rowstat,
-                         reinterpret_cast<const uint2*>(ws + pl.off_ljmask), pl.nslab, pl.rows_per_slab,
-                         pmu, psq, pnk, dense ? 1 : 0, psel);
+      auto gather = [&](int faint_pass) {
+        hipLaunchKernelGGL(diag_accum_gather<DP>, dim3((unsigned)gather_grid(pl.nslab, pl.KB)),
+                           dim3(64 * kGatherWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
+                           reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
+                           reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, pl.KP, rowstat, words,
+                           pl.nslab, pl.rows_per_slab, pmu, psq, pnk, dense ? 1 : 0, sel,
+                           logZ, run1 && !faint_pass ? 1 : 0, run2 ? 0 : 1, alive, faint_pass);
+      };
+      gather(0);
+      if (screen && run2) gather(1);
       return hipGetLastError();
     }
     if (pl.lj_sparse) {
@@ -3630,7 +3970,10 @@ extern "C" int fgmm_diag_estep_f32(const float* X, int64_t ldx, int64_t N, int64
   // The stored-log-joint pass 2 addresses X tiles with 32-bit buffer offsets (row
   // stride at most kMaxBufLdx floats); wider strides recompute, which needs less
   // workspace.
-  const DiagPlan pl = make_plan(N, K, D, wants_stored_lj(flags) && ldx <= kMaxBufLdx, bf16, wants_auto_lj(flags));
+  // A workspace without room for the screened pass 1 runs the call without it.
+  const bool stored = wants_stored_lj(flags) && ldx <= kMaxBufLdx;
+  DiagPlan pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags));
+  if (workspace_bytes < pl.total && pl.screen) pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags), false);
   if (workspace_bytes < pl.total || (pl.total > 0 && workspace == nullptr)) return FGMM_ERR_WORKSPACE;
   if (!want_logz) logZ = nullptr;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
@@ -3649,11 +3992,14 @@ extern "C" int fgmm_diag_estep_f32(const float* X, int64_t ldx, int64_t N, int64
                        reinterpret_cast<float*>(ws + pl.off_kclin),
                        pl.bfneed ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr);
   else if (run1)
-    hipLaunchKernelGGL(diag_x6_prep, dim3(pl.KB), dim3(64), 0, stream, mu, ldmu, log_sigma_sq, ldlss, K,
+    hipLaunchKernelGGL(diag_x6_prep, dim3(pl.KB), dim3(64 * kPrepWaves), 0, stream, mu, ldmu, log_sigma_sq, ldlss, K,
                        (int)D, pl.DP, log_pi, reinterpret_cast<bf16x8*>(ws + pl.off_mu3),
                        reinterpret_cast<double*>(ws + pl.off_kcx6),
-                       reinterpret_cast<double*>(ws + pl.off_kcx6lin),
-                       pl.lj_sparse ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr);
+                       pl.lj_sparse ? reinterpret_cast<unsigned*>(ws + pl.off_ljcount) : nullptr,
+                       pl.screen ? reinterpret_cast<bf16x8*>(ws + pl.off_scop) : nullptr,
+                       pl.screen ? reinterpret_cast<float4*>(ws + pl.off_sce) : nullptr,
+                       pl.screen ? reinterpret_cast<unsigned*>(ws + pl.off_list) : nullptr,
+                       pl.nprobe > 0 ? reinterpret_cast<unsigned*>(ws + pl.off_state) : nullptr);
   if (N > 0) {
     auto run = [&](auto dp_tag) -> hipError_t {
       constexpr int DP = decltype(dp_tag)::value;
@@ -3682,6 +4028,7 @@ extern "C" int fgmm_diag_estep_f32(const float* X, int64_t ldx, int64_t N, int64
     if (e != hipSuccess) return FGMM_ERR_HIP;
   }
   if (!run2) return hipGetLastError() == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
+  const PartCount parts{diag_sel(pl, ws), pl.nslab * pl.spp * pl.rgroups, pl.nslab_lj * pl.rgroups};
   if ((flags & FGMM_FLAG_ATOMIC_REDUCE) && !bf16) {
     if (!accumulate) {
       hipLaunchKernelGGL(diag_fill, dim3((unsigned)cdiv(K, 256)), dim3(256), 0, stream, Nk, K, 0.0f);
@@ -3692,16 +4039,19 @@ extern "C" int fgmm_diag_estep_f32(const float* X, int64_t ldx, int64_t N, int64
       hipLaunchKernelGGL(diag_reduce_atomic, dim3((unsigned)cdiv(K * D, 256), (unsigned)pl.npart), dim3(256), 0,
                          stream, reinterpret_cast<const float*>(ws + pl.off_part_mu),
                          reinterpret_cast<const float*>(ws + pl.off_part_sq),
-                         reinterpret_cast<const float*>(ws + pl.off_part_nk), pl.KP, pl.DP, K, (int)D, mu,
+                         reinterpret_cast<const float*>(ws + pl.off_part_nk), parts, pl.KP, pl.DP, K, (int)D, mu,
                          ldmu, Nk, mu_acc, sig_acc);
     return hipGetLastError() == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
   }
-  const bool wide = pl.npart >= kWideReduce;
-  hipLaunchKernelGGL(wide ? diag_reduce<true> : diag_reduce<false>,
-                     dim3((unsigned)(wide ? cdiv(K * D, 4) : cdiv(K * D, 256))), dim3(256), 0, stream,
-                     reinterpret_cast<const float*>(ws + pl.off_part_mu),
-                     reinterpret_cast<const float*>(ws + pl.off_part_sq),
-                     reinterpret_cast<const float*>(ws + pl.off_part_nk), pl.npart, pl.KP, pl.DP, K,
-                     (int)D, mu, ldmu, Nk, mu_acc, sig_acc, accumulate ? 1 : 0);
+  auto reduce = [&](auto g_tag) {
+    constexpr int G = decltype(g_tag)::value;
+    hipLaunchKernelGGL(diag_reduce<G>, dim3((unsigned)cdiv(K * D, 256 / G)), dim3(256), 0, stream,
+                       reinterpret_cast<const float*>(ws + pl.off_part_mu),
+                       reinterpret_cast<const float*>(ws + pl.off_part_sq),
+                       reinterpret_cast<const float*>(ws + pl.off_part_nk), parts, pl.KP, pl.DP, K, (int)D, mu,
+                       ldmu, Nk, mu_acc, sig_acc, accumulate ? 1 : 0);
+  };
+  if (pl.npart >= kWideReduce) reduce(std::integral_constant<int, 16>{});
+  else reduce(std::integral_constant<int, 4>{});
   return hipGetLastError() == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
 }

@@ -16,7 +16,7 @@
 //               8-wave workgroup whose two waves per SIMD run a block's contraction
 //               and the previous block's epilogue in opposite orders (ping-pong), so
 //               one wave's VALU work runs under the other's matrix steps.
-//   iso_screen  the screened pass 1 of large calls, where the probe finds that most rows
+//   screen_pairs  the screened pass 1 of large calls, where the probe finds that most rows
 //               are near one component block: one bf16 step per chunk with a proven
 //               error bound tells near, faint and zero pairs apart; the gathering pass 2
 //               then forms logZ of a row near one block itself, and iso_lse_pipe runs
@@ -64,7 +64,7 @@
 // A single fp32 chain of fp32 matrix steps over D=128 would leave ~3e-4 absolute
 // error in logZ on clustered data.
 
-#include "fgmm_common.hpp"
+#include "fgmm_screen.hpp"
 
 #include <float.h>
 #include <math.h>
@@ -125,6 +125,9 @@ __host__ inline int iso_padded_dim(int64_t D) {
   return D <= 128 ? (int)round_up(D < 1 ? 1 : D, 32) : (int)round_up(D, 64);
 }
 
+// Partials a slab of the gathering pass 2 leaves (two above D = 64: see make_plan).
+__host__ __device__ constexpr int gather_parts(int DP) { return DP <= 64 ? 1 : 2; }
+
 struct IsoPlan {
   int64_t N, K, D;
   int DP;       // D padded to a multiple of 32 (of 64 above 128)
@@ -133,6 +136,7 @@ struct IsoPlan {
   int cpg;      // component blocks per pass-2 workgroup
   int ncg;      // groups of cpg component blocks (pass 2)
   int nslab;    // row slabs (pass 2)
+  int spp;      // partials per slab (pass 2)
   int nslab_lj; // row slabs of the automatic stored branch's pass 2
   int64_t rows_per_slab_lj;
   int rgroups;  // row groups per slab (partials per slab)
@@ -152,69 +156,11 @@ struct IsoPlan {
   bool bfneed;  // bf16 contract up to D = 128: need masks from pass 1, iso_bf16_gather in pass 2
                 // (or iso_bf16_accum where most pairs are needed)
   bool screen;  // default plan up to D = 128, large calls: a probe selects the screened pass 1
-                // (iso_screen) on the device where most rows need one component block only
+                // (screen_pairs) on the device where most rows need one component block only
   size_t off_musw, off_mu3, off_kcblk, off_kclin, off_kcgat, off_rowstat, off_part_mu, off_part_nk,
       off_part_sig, off_lj, off_ljmax, off_ljmask, off_ljcount, off_xsplit, off_zpair, off_probe, off_scop,
-      off_sce, off_list, off_single, off_faint, off_nearnk, total;
+      off_sce, off_list, off_faint, off_state, total;
 };
-
-// The screened pass 1 (iso_screen): 16-dimension chunks of its approximate contraction
-// (the constants' chunk included), its LDS, and the calls it may take.
-constexpr int kScreenWaves = 4;     // waves per workgroup, 64 rows (two 32-row tiles) each
-constexpr int kScreenBlocks = 2;    // component blocks per LDS stage
-__host__ __device__ constexpr int screen_chunks(int DP) { return DP / 16 + 1; }
-__host__ __device__ constexpr int screen_rs(int DP) { return DP / 2 + 8; }   // bf16 row stride of the staging tile
-__host__ __device__ constexpr size_t screen_stage_bytes(int DP) {
-  return (size_t)kScreenBlocks * screen_chunks(DP) * 64 * 16;
-}
-// Per wave: half of a 32-row tile's columns in bf16 and their partial sums of squares.
-__host__ __device__ constexpr size_t screen_tile_bytes(int DP) {
-  return (size_t)32 * screen_rs(DP) * 2 + (size_t)32 * (DP / 8 + 1) * 4;
-}
-// The first stage's operands, then the staging tiles, which the second stage and the
-// rows' block bounds (bf16, 64 rows per wave) overlay once the rows are in registers.
-__host__ __device__ constexpr size_t screen_lds_bytes(int DP, int KB) {
-  const size_t a = kScreenWaves * screen_tile_bytes(DP);
-  const size_t b = screen_stage_bytes(DP) + (size_t)kScreenWaves * 64 * round_up(KB, 8) * 2;
-  return screen_stage_bytes(DP) + (a > b ? a : b);
-}
-// Calls whose pass 1 is worth screening: at least kScreenMinWork (32-row tile, block,
-// chunk) steps, below which the further launches cost more than the screening saves,
-// and at least 4 blocks (with one needed block a row, screening B blocks leaves 1/B of
-// the exact contraction); two workgroups per compute unit.
-constexpr int64_t kScreenMinWork = 500000;
-constexpr int64_t kMaxScreenLdx = (int64_t)4 << 20;   // 64 rows within 32-bit buffer offsets
-__host__ inline bool use_screen(int64_t N, int DP, int KB) {
-  return DP <= 128 && KB >= 4 && KB <= kProbeMaxKB && N < ((int64_t)1 << 31) - 256 &&
-         cdiv(N, 32) * KB * (DP / 16) >= kScreenMinWork && screen_lds_bytes(DP, KB) <= kMaxLds / 2;
-}
-
-// The screened pass 1 tells near pairs from faint ones.  A pair is near unless its
-// responsibility r provably has r, r ||x||, r ||x||^2 <= 2^-kNearGap; the faint pairs of
-// a component with Nk >= kNearNk then change none of its sums by a rounding (at most
-// N 2^-72 <= 2^-41, against 2^-24 of 2^-10), and a row's terms outside its near blocks
-// change no bit of its fp32 log-sum-exp (at most K 2^-72 of it).  So pass 2 takes the
-// near pairs, and then the faint ones of those blocks that hold a component with less.
-constexpr float kNearGap = 72.0f;
-constexpr float kNearNk = 0x1p-10f;
-
-// How a call's passes run.  The probe's last workgroup sums its counts and writes the
-// choice as one word, which every later kernel of the call reads with one scalar load
-// (each summing the counts for itself cost 0.5 us a kernel).
-enum IsoMode { kModeDefault = 0, kModeStored = 1, kModeScreen = 2 };
-__device__ __forceinline__ int iso_mode(const int* __restrict__ sel) { return sel ? *sel : kModeDefault; }
-// What the probe chooses from: up to max_multi sampled rows near several blocks, the
-// screened pass 1 (-1: never); else, from min_pairs needed pairs on, the stored branch if
-// the call has one.
-struct IsoRule {
-  int64_t max_multi, min_pairs;
-  int stored;
-};
-// The probe's part of the workspace: per sampled tile the needed pairs, then (from
-// kProbeTiles on) the rows near several blocks; then the choice and the count of
-// finished workgroups (zeroed by the prologue).
-constexpr int kProbeMode = 2 * kProbeTiles, kProbeDone = 2 * kProbeTiles + 1;
-constexpr size_t kIsoProbeBytes = (2 * kProbeTiles + 2) * sizeof(unsigned);
 
 // Pass 1 with need masks keeps a bf16 bound of each row's block maximum in LDS,
 // 2 bytes per (row, block) for its 4 waves, while the workgroup still fits twice in
@@ -273,12 +219,13 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   p.DP = iso_padded_dim(D);
   p.KB = (int)cdiv(K, 32);
   p.KP = p.KB * 32;
+  p.spp = 1;
   p.bf16 = bf16;
   p.lj = !bf16 && use_stored_lj(N, p.DP, p.KB, allow_lj);
   p.need = !bf16 && !p.lj;
   p.autolj = p.need && auto_lj && p.DP <= 128 && N > 0 && p.KB > 0 && p.KB <= kProbeMaxKB &&
              (size_t)round_up(cdiv(N, 32), 8) * (size_t)p.KB * kLjTile * sizeof(float) <= kMaxLjBytes;
-  p.screen = p.need && allow_screen && use_screen(N, p.DP, p.KB);
+  p.screen = p.need && allow_screen && use_screen(N, p.DP, false, p.KB);
   p.nprobe = (p.autolj || p.screen) ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
   p.ctile = p.need && p.DP > 128;
   p.rexact = (p.need || (p.lj && p.DP <= 128)) &&
@@ -328,10 +275,12 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   } else if (p.need && N > 0 && p.KB > 0) {
     // The gathering pass 2: one round of waves, two per SIMD up to D = 64, one above
     // (there, 64 slabs in two rounds took 0.266 ms at N=1M K=1024 D=128, 32 slabs take
-    // 0.247 ms).  The stored branch's pass 2 takes eight blocks per compute unit.
+    // 0.247 ms; their float32 sums go out in two partials each, so that they are no
+    // longer).  The stored branch's pass 2 takes eight blocks per compute unit.
+    p.spp = gather_parts(p.DP);
     const int64_t rounds = p.DP <= 64 ? 8 : 4;
     const int64_t want = gather_slab_count(cdiv(rounds * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
-    p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double2));
+    p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32 * p.spp), sizeof(double2)) / (32 * p.spp) * (32 * p.spp);
     p.nslab = (int)cdiv(N, p.rows_per_slab);
     if (p.DP <= 128) {   // its partials are laid out with or without the branch
       const int64_t wl = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
@@ -353,7 +302,7 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     p.rows_per_slab = tile_rows;
     p.nslab = 0;
   }
-  p.npart = std::max(p.nslab, p.nslab_lj) * p.rgroups;
+  p.npart = std::max(p.nslab * p.spp, p.nslab_lj) * p.rgroups;
   // The bf16 contract's need masks: each row's block maxima (bf16, 2 bytes per row and
   // block for the 4 waves of a pass-1 workgroup) must fit in LDS beside the stages.
   p.bfneed = bf16 && !p.bfw && p.DP <= 128 && p.KB > 0 &&
@@ -372,9 +321,10 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     // after it: the screening operands and error bounds, and the list of rows that need
     // several blocks (its length first).
     size_t so = off;
-    p.off_scop = so; so = align256(so + (size_t)p.KB * screen_chunks(p.DP) * 64 * 16);
+    p.off_scop = so; so = align256(so + (size_t)p.KB * screen_chunks(p.DP, false) * 64 * 16);
     p.off_sce = so;  so = align256(so + (size_t)p.KB * sizeof(float4));
     p.off_list = so; so = align256(so + 256 + (size_t)N * sizeof(int));
+    p.off_probe = so; so = align256(so + kProbeBytes);
     off = so;
   }
   off = std::max(off, align256(p.off_part_mu + (size_t)p.npart * p.KP * p.DP * sizeof(float)));
@@ -395,12 +345,10 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
   p.off_xsplit = off; off = align256(off + ptiles * ljt_xsplit_bytes(p.DP));
   p.off_zpair = off;  off = align256(off + ptiles * 32 * sizeof(float2));
   // The probe: sampled rows' block maxima, its counters and the selector word.
-  p.off_probe = off;  off = align256(off + (p.nprobe > 0 ? kIsoProbeBytes : 0));
-  // The screened pass 1: one bit per row, set where the row is near one block only; the
-  // faint pairs' words; and pass 2's Nk partials before it adds faint pairs.
-  p.off_single = off; off = align256(off + (p.screen ? (size_t)cdiv(N, 64) * 2 * sizeof(unsigned) : 0));
+  if (p.nprobe > 0 && !p.screen) { p.off_probe = off; off = align256(off + kProbeBytes); }
+  // The call's state words, and the screened pass 1's words of faint pairs.
+  p.off_state = off;  off = align256(off + (p.nprobe > 0 ? state_bytes(p.KB) : 0));
   p.off_faint = off;  off = align256(off + (p.screen ? ntile * sizeof(unsigned) : 0));
-  p.off_nearnk = off; off = align256(off + (p.screen ? (size_t)p.nslab * p.KP * sizeof(float) : 0));
   p.total = off;
   return p;
 }
@@ -419,7 +367,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
                                                double4* __restrict__ kc_gat, bf16x8* __restrict__ mu3,
                                                unsigned* __restrict__ ljcount, bf16x8* __restrict__ sc_op,
                                                float4* __restrict__ sc_e, unsigned* __restrict__ list_count,
-                                               unsigned* __restrict__ probe) {
+                                               unsigned* __restrict__ state) {
   __shared__ double sC[32], sB[32], sL[32], sO[kPrepChunks][32];
   const int kb = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
@@ -427,7 +375,10 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
   // Pass 1 counts the needed row pairs of the stored log-joint into these.
   if (ljcount && kb == 0 && wave == 0) ljcount[lane] = 0u;
   if (list_count && kb == 0 && tid == 0) *list_count = 0u;
-  if (probe && kb == 0 && tid == 0) probe[kProbeDone] = 0u;
+  if (state && tid == 0) {
+    if (kb == 0) state[kStateDone] = 0u;
+    state[kStateAlive + kb] = 0u;
+  }
   const int64_t comp = (int64_t)kb * 32 + c;
   const bool valid = comp < K;
   const int NQ = DP / 16;
@@ -515,9 +466,9 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
   if (sc_op) {
     // The screening's constants chunk, -b ||x||^2 + C as products of three-way bf16
-    // splits (iso_screen's row operand holds the matching splits of ||x||^2 and ones),
+    // splits (screen_pairs's row operand holds the matching splits of ||x||^2 and ones),
     // and the block's error bound |approximate - exact log-joint| <=
-    // sc_e.x ||x|| + sc_e.y ||x||^2 + sc_e.z (iso_screen).
+    // sc_e.x ||x|| + sc_e.y ||x||^2 + sc_e.z (screen_pairs).
     f32x4 lo = zero4();
     const double C = sL[c];
     lo.x = -(float)sB[c];
@@ -761,10 +712,7 @@ void iso_lse(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
 // ---------------------------------------------------------------------------
 constexpr int kPipeWaves = 8;
 constexpr int kPipeThreads = 64 * kPipeWaves;
-constexpr int kListBase = 64;   // ints before the first row of iso_screen's list (entry 0: its length)
-// Lists of up to this many 32-row workgroups per compute unit run one tile per workgroup
-// (a round of them takes about a quarter of a round of 256-row workgroups).
-constexpr int kFewRounds = 3;
+
 
 // iso_lse_pipe's grid: whole rounds of 8-tile workgroups (one per compute unit),
 // then the tiles left in groups of `small`, one group per compute unit.
@@ -815,8 +763,8 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, g = lane >> 5;
-  const int mode = iso_mode(sel);
-  // After the screening (iso_screen) only the rows on its list are left, the listed rows
+  const int mode = call_mode(sel);
+  // After the screening (screen_pairs) only the rows on its list are left, the listed rows
   // taking the place of rows 0 .. n - 1; it has written the need masks.
   const bool listed = mode == kModeScreen;
   const int64_t nrow = listed ? (int64_t)(unsigned)list[0] : N;
@@ -1129,14 +1077,13 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
                                                                     const bf16x8* __restrict__ mu3,
                                                                     const double2* __restrict__ kc_blk, int KB,
                                                                     const float4* __restrict__ sc_e, int ntile,
-                                                                    IsoRule rule, unsigned* __restrict__ count) {
+                                                                    ProbeRule rule, unsigned* __restrict__ count,
+                                                                    unsigned* __restrict__ state) {
   constexpr int NQ = DP / 16;
   constexpr int BLK = NQ * 4 * 64;
-  // The rows' block maxima and the screening's error bounds, the rows' maxima over the
-  // blocks (R, and R less its bound) by 32 threads each, and their kept blocks.
+  // The rows' block maxima and the screening's error bounds.
   __shared__ float rmax[kProbeMaxKB * 32], rerr[kProbeMaxKB * 32];
-  __shared__ float rowR[32][33], rowL[32][33];
-  __shared__ unsigned part[kProbeWaves], blocks[32];
+  __shared__ ProbeScratch sh;
   const int s = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1197,313 +1144,9 @@ __global__ __launch_bounds__(64 * kProbeWaves) void iso_store_probe(const float*
       rerr[kb * 32 + c] = sc_e ? fmaf(e.x, nx, fmaf(e.y, xs, e.z)) : 0.0f;
     }
   }
-  if (tid < 32) blocks[tid] = 0u;
-  __syncthreads();
-  // Each row's largest maximum R and largest lower bound L: 32 threads a row.
-  const int t32 = tid >> 5;
-  float R = -INFINITY, L = -INFINITY;
-  for (int kb = t32; kb < KB; kb += 32) {
-    const float r = rmax[kb * 32 + c];
-    R = fmaxf(R, r);
-    L = fmaxf(L, r - rerr[kb * 32 + c]);
-  }
-  rowR[t32][c] = R;
-  rowL[t32][c] = L;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 32; ++j) {
-    R = fmaxf(R, rowR[j][c]);
-    L = fmaxf(L, rowL[j][c]);
-  }
-  unsigned need = 0, kept = 0;
-  if (valid) {
-    const float near_gap = fminf(kLjNeedGap, kNearGap + 2.0f * log2f(1.0f + nx));
-    for (int kb = t32; kb < KB; kb += 32) {
-      const float r = rmax[kb * 32 + c];
-      need += (r - R >= -kLjNeedGap) ? 1u : 0u;
-      kept += !(r + rerr[kb * 32 + c] - L < -near_gap) ? 1u : 0u;   // iso_screen's near blocks
-    }
-    if (sc_e && kept != 0) atomicAdd(blocks + c, kept);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) need += __shfl_xor(need, o);
-  if (lane == 0) part[wave] = need;
-  __syncthreads();
-  if (tid == 0) {
-    unsigned tot = 0;
-    for (int w = 0; w < kProbeWaves; ++w) tot += part[w];
-    count[s] = tot;
-  }
-  if (wave != 0) return;
-  const uint64_t multi = __builtin_amdgcn_ballot_w64(sc_e != nullptr && lane < 32 && blocks[c] > 1u);
-  unsigned done = 0;
-  if (lane == 0) {
-    count[kProbeTiles + s] = (unsigned)__builtin_popcountll(multi);
-    __threadfence();
-    done = atomicAdd(count + kProbeDone, 1u);
-  }
-  if (__builtin_amdgcn_readfirstlane(done) != (unsigned)ntile - 1u) return;
-  // The last workgroup to finish: every count is visible to device-scope loads.
-  __threadfence();
-  uint64_t t = 0;
-  if (lane < ntile)
-    t = ((uint64_t)__hip_atomic_load(count + kProbeTiles + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) << 32) |
-        __hip_atomic_load(count + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);   // at most 2^20 pairs and 2^11 rows
-  if (lane == 0)
-    count[kProbeMode] = (int64_t)(t >> 32) <= rule.max_multi ? kModeScreen
-                        : rule.stored && (int64_t)(t & 0xffffffffu) >= rule.min_pairs ? kModeStored : kModeDefault;
+  probe_finish(rmax, rerr, sh, KB, valid, nx, sc_e != nullptr, s, ntile, rule, count, state);
 }
 
-
-// ---------------------------------------------------------------------------
-// The screened pass 1 (default plan up to D = 128, large calls, selected by the probe).
-//
-// Where clusters are separated, the exact contraction (seven bf16 steps per 16
-// dimensions) of nearly every (row, block) pair only proves that its responsibilities
-// are zero.  This kernel proves it with one step: the approximate log-joint
-//   a_nk = sum_d bf16(x_d) bf16(2 b_k mu_kd) - b_k ||x||^2 + C_k
-// comes straight out of the matrix cores (the constants are one more chunk of three-way
-// splits), a row's block maximum is a maximum of accumulators, and
-//   |a_nk - ll2_nk| <= E = sc_e.x ||x|| + sc_e.y ||x||^2 + sc_e.z   (iso_prep, per block):
-// each operand is rounded by at most 2^-9 of itself, so the products err by 2^-8 ||x||
-// ||2 b mu|| (Cauchy-Schwarz; 0x1.06p-8 with the second-order and accumulation terms),
-// the constants' dropped split products and fp32 sums by under 2^-14 (b ||x||^2 + |C|).
-// With L the largest a - E over all blocks (logZ2 >= L), a block with a + E < L -
-// kLjNeedGap holds only responsibilities that are exactly zero, as the need masks of the
-// exact pass 1 state; the other blocks get their need bit.  Not-finite values make E
-// or a infinite or NaN, and the comparison then keeps the block.
-// A row with one needed block needs no other block for logZ either: the gathering pass
-// 2 forms its log-sum-exp there (`single` bit).  The rest go on a list, which
-// iso_lse_pipe runs through the exact pass 1.
-//
-// Bound: matrix steps and VALU, which mostly add up on a SIMD: at D = 128, 9 matrix
-// steps (288 cycles) and about 25 VALU instructions per (32 rows, block); matrix steps
-// alone 51% of its cycles.  Each operand read from LDS serves two 32-row tiles.  Rows
-// are read in whole lines and transposed through LDS (the exact pass reads 16-byte
-// pieces of 32 rows per instruction, which at this kernel's length would bound it).
-// N=1M K=1024 D=128 clustered: 0.27 ms, and pass 1 and 2 with it 0.55 ms instead of
-// 1.73 ms (drop-in call 1.73 -> 0.58 ms); N=400K K=300 D=50: call 0.51 -> 0.28 ms.
-// ---------------------------------------------------------------------------
-template <int DP>
-__global__ __attribute__((amdgpu_flat_work_group_size(64 * kScreenWaves, 64 * kScreenWaves),
-                          amdgpu_waves_per_eu(3, 3)))
-void iso_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ sc_op,
-                const float4* __restrict__ sc_e, int KB, unsigned* __restrict__ need,
-                unsigned* __restrict__ faint, unsigned* __restrict__ single, int* __restrict__ list, const int* __restrict__ sel) {
-  constexpr int NC = screen_chunks(DP), NQ = DP / 16;
-  constexpr int BLK = NC * 64;                    // bf16x8 per block
-  constexpr int STG = kScreenBlocks * BLK;        // bf16x8 per stage
-  constexpr int RS = screen_rs(DP), V4 = DP / 8;  // float4 per half row
-  constexpr int LPT = 32 * V4 / 64;               // float4 per lane and half tile
-  if (iso_mode(sel) != kModeScreen) return;
-
-  extern __shared__ __align__(16) unsigned char lds_raw[];
-  bf16x8* const op0 = reinterpret_cast<bf16x8*>(lds_raw);
-  unsigned char* const rest = lds_raw + screen_stage_bytes(DP);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 31, g = lane >> 5;
-  unsigned short* const ub_l = reinterpret_cast<unsigned short*>(rest + screen_stage_bytes(DP)) +
-                               wave * 64 * ((KB + 7) & ~7) + lane;
-
-  // Stage st (blocks kScreenBlocks st ..) into operand buffer st & 1, in 1 KB pieces.
-  auto fetch = [&](int st) {
-    const int nb = KB - st * kScreenBlocks < kScreenBlocks ? KB - st * kScreenBlocks : kScreenBlocks;
-    const DmaSrc r = dma_src(sc_op + (int64_t)st * STG, (uint32_t)(nb * BLK * (int)sizeof(bf16x8)));
-    bf16x8* dst = (st & 1) ? reinterpret_cast<bf16x8*>(rest) : op0;
-    for (int p = wave; p < nb * NC; p += kScreenWaves)
-      lds_dma16(r, dst + p * 64, lane * (int)sizeof(bf16x8), p * 64 * (int)sizeof(bf16x8));
-  };
-  const int64_t row0 = (int64_t)blockIdx.x * (64 * kScreenWaves) + wave * 64;
-  const int64_t row = row0 + lane;
-  fetch(0);
-
-  // The wave's two 32-row tiles in halves of the columns: whole 128-byte lines per load,
-  // rounded to bf16 into the wave's staging tile and read back as B operands; ||x||^2
-  // from the fp32 values.  The next half's loads are in flight meanwhile.
-  __bf16* const xt = reinterpret_cast<__bf16*>(rest + wave * screen_tile_bytes(DP));
-  float* const sq = reinterpret_cast<float*>(xt + 32 * RS);
-  bf16x8 xb[2][NC];
-  float xs = 0.0f;   // of the lane's own row, row0 + lane
-  f32x4 raw[2][LPT];
-  // Rows past N lie past the resource and read zeros, as do columns from D on.
-  const int64_t rows = N - row0 < 64 ? (N - row0 > 0 ? N - row0 : 0) : 64;
-  const buf_rsrc xr = make_rsrc(X + (rows > 0 ? row0 * ldx : 0), (uint32_t)(rows * ldx * (int64_t)sizeof(float)));
-  const int rbytes = (int)ldx * (int)sizeof(float);
-  auto load = [&](int u, f32x4 (&r)[LPT]) __attribute__((always_inline)) {
-    if constexpr (64 % V4 == 0) {   // a lane's column is the same in every load
-      const int d0 = (u & 1) * (DP / 2) + 4 * (lane % V4);
-      int off = d0 < D ? (32 * (u >> 1) + lane / V4) * rbytes + d0 * 4 : kBufOob;
-#pragma unroll
-      for (int i = 0; i < LPT; ++i) {
-        r[i] = buf_load_f32x4(xr, buf_off(off));
-        off += (64 / V4) * rbytes;
-        if (d0 >= D) off = kBufOob;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < LPT; ++i) {
-        const int idx = i * 64 + lane, d0 = (u & 1) * (DP / 2) + 4 * (idx % V4);
-        r[i] = buf_load_f32x4(xr, buf_off(d0 < D ? (32 * (u >> 1) + idx / V4) * rbytes + d0 * 4 : kBufOob));
-      }
-    }
-    if (D & 3) {   // uniform: the columns past D inside the last vector
-#pragma unroll
-      for (int i = 0; i < LPT; ++i) {
-        const int d0 = (u & 1) * (DP / 2) + 4 * ((i * 64 + lane) % V4);
-        if (d0 + 1 >= D) r[i].y = 0.0f;
-        if (d0 + 2 >= D) r[i].z = 0.0f;
-        if (d0 + 3 >= D) r[i].w = 0.0f;
-      }
-    }
-  };
-  load(0, raw[0]);
-  float s = 0.0f;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int t = u >> 1, h = u & 1;
-    if (u < 3) load(u + 1, raw[(u + 1) & 1]);
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int idx = i * 64 + lane, rr = idx / V4, v = idx % V4;
-      const f32x4 x = raw[u & 1][i];
-      const uint2 w = {bf16_pair(f32x2{x.x, x.y}), bf16_pair(f32x2{x.z, x.w})};
-      *reinterpret_cast<uint2*>(xt + rr * RS + 4 * v) = w;
-      sq[rr * (V4 + 1) + v] = fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w)));
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (h == 0) s = 0.0f;
-#pragma unroll
-    for (int v = 0; v < V4; ++v) s += sq[c * (V4 + 1) + v];
-#pragma unroll
-    for (int q = 0; q < NQ / 2; ++q)
-      xb[t][h * (NQ / 2) + q] = *reinterpret_cast<const bf16x8*>(xt + c * RS + 16 * q + 8 * g);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (h == 1) {
-      if (g == t) xs = s;
-      // The constants' chunk: ||x||^2's splits in the first half, ones in the second.
-      f32x4 lo = zero4();
-      lo.x = s;
-      bf16x8 sp[3], a;
-      split3_bf16(lo, zero4(), sp);
-      const __bf16 one = (__bf16)1.0f, zero = (__bf16)0.0f;
-      a[0] = g == 0 ? sp[0][0] : one;
-      a[1] = g == 0 ? sp[1][0] : one;
-      a[2] = g == 0 ? sp[2][0] : one;
-      a[3] = g == 0 ? sp[0][0] : zero;
-      a[4] = g == 0 ? sp[1][0] : zero;
-      a[5] = g == 0 ? sp[0][0] : zero;
-      a[6] = zero;
-      a[7] = zero;
-      xb[t][NQ] = a;
-    }
-  }
-  const float nx = sqrtf(xs);
-  lds_barrier();   // every wave has read its staging tile: the second stage and the bounds may overwrite it
-
-  for (int kb = KB; kb < ((KB + 7) & ~7); ++kb) ub_l[kb * 64] = 0xff7f;   // the least finite bound
-
-  float L = -INFINITY;
-  const int nst = (KB + kScreenBlocks - 1) / kScreenBlocks;
-  for (int st = 0; st < nst; ++st) {
-    dma_barrier();   // stage st has landed, and every wave is done with stage st - 1
-    if (st + 1 < nst) fetch(st + 1);
-    const bf16x8* op = ((st & 1) ? reinterpret_cast<const bf16x8*>(rest) : op0) + lane;
-#pragma unroll
-    for (int j = 0; j < kScreenBlocks; ++j) {
-      const int kb = st * kScreenBlocks + j;
-      if (kb >= KB) break;
-      const float4 e = sc_e[kb];
-      // All of the block's operand reads in flight before the first is used.
-      bf16x8 a[NC];
-#pragma unroll
-      for (int q = 0; q < NC; ++q) a[q] = op[(j * NC + q) * 64];
-      __builtin_amdgcn_sched_barrier(0);
-      f32x16 acc[2] = {zero16(), zero16()};
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int q = 0; q < NC; ++q) acc[t] = mfma_bf16(a[q], xb[t][q], acc[t]);
-      }
-      float m[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        m[t] = acc[t][0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) m[t] = fmaxf(m[t], acc[t][i]);
-      }
-      // Lane l's own row is row l % 32 of tile l / 32; the other half-wave holds half of
-      // its block maximum.
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m[0]), __float_as_uint(m[1]), false, false);
-      const float am = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      const float E = fmaf(e.x, nx, fmaf(e.y, xs, e.z));
-      // The bound rounded up to bf16: truncation does it for negative values, and for
-      // positive ones after adding 2^-7 of them (one bf16 step or more).
-      const float ub = am + E;
-      ub_l[kb * 64] = (unsigned short)(__float_as_uint(fmaf(fmaxf(ub, 0.0f), 0x1p-7f, ub)) >> 16);
-      L = fmaxf(L, am - E);
-    }
-  }
-
-  // Need words of the two tiles (each lane reads back the bounds it wrote itself), 32
-  // blocks at a time, lane c of half g keeping block kb0 + c of tile g.
-  const bool valid = row < N;
-  if (!valid) L = INFINITY;   // a row past N (zeros: finite bounds) gets no bit
-  const float near_gap = fminf(kLjNeedGap, kNearGap + 2.0f * log2f(1.0f + nx));   // kLjNeedGap if nx is NaN
-  uint64_t once = 0, twice = 0;   // rows with at least one, two near blocks
-  const int64_t tile = (row0 >> 5) + g;
-  for (int kb0 = 0; kb0 < KB; kb0 += 32) {
-    unsigned w = 0, wf = 0;
-#pragma unroll 1
-    for (int j0 = 0; j0 < 32 && kb0 + j0 < KB; j0 += 8) {
-      // Eight bounds in flight together (past KB: the fill).
-      float ub[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ub[j] = bf16_bits_to_float(ub_l[(kb0 + j0 + j) * 64]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float u = ub[j] - L;
-        const uint64_t b = __builtin_amdgcn_ballot_w64(!(u < -near_gap));
-        const uint64_t f = __builtin_amdgcn_ballot_w64(!(u < -kLjNeedGap)) & ~b;
-        twice |= once & b;
-        once |= b;
-        if (c == j0 + j) {
-          w = g == 0 ? (unsigned)b : (unsigned)(b >> 32);
-          wf = g == 0 ? (unsigned)f : (unsigned)(f >> 32);
-        }
-      }
-    }
-    if (kb0 + c < KB && tile * 32 < N) {
-      need[tile * KB + kb0 + c] = w;
-      faint[tile * KB + kb0 + c] = wf;
-    }
-  }
-  const uint64_t one = once & ~twice;
-  const uint64_t many = __builtin_amdgcn_ballot_w64(valid) & ~one;
-  if (c == 0 && tile * 32 < N) single[tile] = g == 0 ? (unsigned)one : (unsigned)(one >> 32);
-  // The workgroup's listed rows: one atomic for all (one per wave, at N=400K
-  // K=300 D=50 where most waves have some, serialised on the counter: 110 us for the
-  // kernel, 48 us this way).
-  int* cnt_l = reinterpret_cast<int*>(lds_raw);   // the first stage's operands have been used
-  lds_barrier();
-  if (lane == 0) cnt_l[wave] = __builtin_popcountll(many);
-  lds_barrier();
-  int before = 0, total = 0;
-#pragma unroll
-  for (int v = 0; v < kScreenWaves; ++v) {
-    const int n = cnt_l[v];
-    before += v < wave ? n : 0;
-    total += n;
-  }
-  if (total == 0) return;
-  if (tid == 0) cnt_l[kScreenWaves] = (int)atomicAdd(reinterpret_cast<unsigned*>(list), (unsigned)total);
-  lds_barrier();
-  const int pos = cnt_l[kScreenWaves] + before +
-                  (int)__builtin_amdgcn_mbcnt_hi((unsigned)(many >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)many, 0u));
-  if ((many >> lane) & 1) list[kListBase + pos] = (int)row;
-}
 
 // ---------------------------------------------------------------------------
 // Pass 1 of the default plan above D = 128 (any D).  The split operands of a row
@@ -1816,19 +1459,20 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
                       const unsigned* __restrict__ needcount, int64_t dense_min, int nslab,
                       int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_nk,
                       float* __restrict__ part_sig, int dense, const int* __restrict__ sel,
-                      const unsigned* __restrict__ single, const double2* __restrict__ kc_blk,
-                      float* __restrict__ logZ, int lse_only, float* __restrict__ near_nk, int faint) {
+                      const unsigned* __restrict__ own_words, const double2* __restrict__ kc_blk,
+                      float* __restrict__ logZ, int lse_only, unsigned* __restrict__ alive, int faint) {
   constexpr int NQ = DP / 16;
   constexpr int NJ = DP / 32;
   constexpr int RS = gather_rs(DP);
   constexpr int BLK = NQ * 4 * 64;   // bf16x8 per component block
+  constexpr int PW = gather_parts(DP);
   // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO runs instead when selected; after
   // the screened pass 1 this kernel always runs, else with at least dense_min needed rows
   // iso_accum_tiles does (uniform exits).
-  const int mode = iso_mode(sel);
+  const int mode = call_mode(sel);
   if (mode == kModeStored) return;
   if (mode == kModeDefault && (lse_only || faint || need_total(needcount) >= dense_min)) return;
-  const bool fused = mode == kModeScreen && single != nullptr;
+  const bool fused = mode == kModeScreen && own_words != nullptr && !faint;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   unsigned char* lp = lds_raw;
@@ -1849,17 +1493,8 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   if (faint) {
     // The second run after the screened pass 1: the block's faint pairs, where one of its
     // components has too small an Nk to absorb them (one of zero weight has none).
-    float* nk_l = reinterpret_cast<float*>(lds_raw);   // [8][32]
-    float v = 0.0f;
-    for (int sl = tid >> 5; sl < nslab; sl += 8) v += near_nk[(int64_t)sl * KP + kb * 32 + c];
-    nk_l[tid] = v;
-    __syncthreads();
-    v = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v += nk_l[j * 32 + c];
     const bool none = kc_gat[(int64_t)kb * 32 + c].x == -INFINITY;
-    if (__builtin_amdgcn_ballot_w64(!(v >= kNearNk) && !none) == 0) return;
-    __syncthreads();
+    if (((unsigned)__builtin_amdgcn_ballot_w64(!none) & ~alive[kb]) == 0u) return;   // uniform
   }
   for (int idx = tid; idx < BLK; idx += 64 * kGatherWaves) mu_l[idx] = mu3[(int64_t)kb * BLK + idx];
   if (tid < 32) kb_l[tid] = kc_blk[(int64_t)kb * 32 + tid];
@@ -1878,12 +1513,14 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
-  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32);
+  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32), t_mid = (t_begin + t_end) / 2;
 
   // Need words of 64 tiles at a time, one per lane, the next batch in flight.
   auto words = [&](int64_t tb) -> unsigned {
     const int64_t t = tb + lane;
-    return t < t_end ? need[t * KB + kb] : 0u;
+    if (t >= t_end) return 0u;
+    // (The faint words hold the own pairs' bits too, which are near.)
+    return need[t * KB + kb] & (faint ? ~own_words[t * KB + kb] : ~0u);
   };
   int64_t tb = t_begin;
   unsigned mword = words(tb), mnext = words(tb + 64);
@@ -1906,7 +1543,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   // state.  Stage P holds the tile after next while tile P is computed.
   f32x4 raw[2][2 * NQ];
   double2 rst[2];
-  unsigned sgl[2] = {0u, 0u};   // the single-block word of the row's tile (fused)
+  unsigned sgl[2] = {0u, 0u};   // the own-pairs word of the row's tile (fused)
   int erow[2] = {0, 0};
   // The rows come through resources over the slab: a lane without a row reads zeros
   // and makes no access, and the loads of a tile issue back to back.  X so while the
@@ -1916,12 +1553,12 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const bool xfull = xbuf && D == DP;
   const buf_rsrc xres = slab_rsrc(X, ldx, r_begin, xbuf ? r_end : r_begin);
   const buf_rsrc rres = make_rsrc(rowstat + r_begin, (uint32_t)((r_end - r_begin) * sizeof(double2)));
-  const buf_rsrc sres = make_rsrc(fused ? single + t_begin : nullptr,
-                                  fused ? (uint32_t)((t_end - t_begin) * sizeof(unsigned)) : 0u);
+  const buf_rsrc sres = make_rsrc(fused ? own_words + t_begin * KB + kb : nullptr,
+                                  fused ? (uint32_t)((t_end - t_begin) * KB * sizeof(unsigned)) : 0u);
   auto issue = [&](int e, f32x4 (&rw)[2 * NQ], double2& rs, unsigned& sw, int& er) __attribute__((always_inline)) {
     const bool ok = e >= 0;
     er = e;
-    sw = buf_load_u32(sres, buf_off(ok ? (e >> 5) * (int)sizeof(unsigned) : kBufOob));
+    sw = buf_load_u32(sres, buf_off(ok ? (e >> 5) * KB * (int)sizeof(unsigned) : kBufOob));
     if (xfull) {
       const int off = buf_off(ok ? (int)((int64_t)e * ldx * (int64_t)sizeof(float)) + 32 * g : kBufOob);
 #pragma unroll
@@ -2061,40 +1698,56 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
     return cnt_ahead;
   };
 
+  // Partial p of the slab (the faint pass adds to the first), and the sums start again.
+  auto store = [&](int p) __attribute__((always_inline)) {
+    nk += __shfl_xor(nk, 32);
+    sig += __shfl_xor(sig, 32);
+    const int64_t kbase = (int64_t)(slab * PW + p) * KP + (int64_t)kb * 32;
+    float* pm = part_mu + kbase * DP + 4 * g * DP + c;
+    if (faint) {
+      nk += part_nk[kbase + c];
+      sig += part_sig[kbase + c];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[j][i] += pm[acc_row(i, 0) * DP + 32 * j];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) pm[acc_row(i, 0) * DP + 32 * j] = acc[j][i];
+      acc[j] = zero16();
+    }
+    if (g == 0) {
+      part_nk[kbase + c] = nk;
+      part_sig[kbase + c] = sig;
+    }
+    if (mode == kModeScreen && !faint) mark_alive(alive, kb, nk);
+    nk = sig = 0.0f;
+  };
+
   int e;
   int cnt0 = take(e);
   if (cnt0 > 0) issue(e, raw[0], rst[0], sgl[0], erow[0]);
   int cnt1 = cnt0 > 0 ? take(e) : 0;
   if (cnt1 > 0) issue(e, raw[1], rst[1], sgl[1], erow[1]);
-  while (cnt0 > 0) {
-    cnt0 = tile(std::integral_constant<int, 0>{});
-    if (cnt1 == 0) break;
-    cnt1 = tile(std::integral_constant<int, 1>{});
-  }
-  if (lse_only) return;
-
-  nk += __shfl_xor(nk, 32);
-  sig += __shfl_xor(sig, 32);
-  const int64_t kbase = (int64_t)slab * KP + (int64_t)kb * 32;
-  if (faint) {   // added to the near pairs' sums
-    if (qt == 0) return;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[j][i] += part_mu[(kbase + acc_row(i, g)) * DP + 32 * j + c];
+  // Above D = 64 a partial ends once half of the slab's tiles are queued.
+  const int parts = (lse_only || faint) ? 1 : PW;
+#pragma unroll 1
+  for (int p = 0; p < parts; ++p) {
+    while (cnt0 > 0) {
+      cnt0 = tile(std::integral_constant<int, 0>{});
+      if (cnt1 == 0) {
+        cnt0 = 0;
+        break;
+      }
+      cnt1 = tile(std::integral_constant<int, 1>{});
+      if (p + 1 < parts && tb >= t_mid) break;
     }
-    nk += part_nk[kbase + c];
-    sig += part_sig[kbase + c];
-  }
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) part_mu[(kbase + acc_row(i, g)) * DP + 32 * j + c] = acc[j][i];
-  }
-  if (g == 0) {
-    part_nk[kbase + c] = nk;
-    part_sig[kbase + c] = sig;
-    if (mode == kModeScreen && !faint) near_nk[kbase + c] = nk;
+    if (lse_only || (faint && qt == 0)) return;
+    store(p);
   }
 }
 
@@ -2135,7 +1788,7 @@ void iso_accum_tiles(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   constexpr int V4 = DP / 4;              // float4 per row
   constexpr int LPT = 32 * V4 / NT;       // float4 per thread per tile
   static_assert((32 * V4) % NT == 0, "tile split");
-  if (iso_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
+  if (call_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
   if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exits)
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -2170,6 +1823,7 @@ void iso_accum_tiles(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
+  if (r_end < r_begin) r_end = r_begin;   // a slab past N: no rows, a zero partial
   const int64_t t_begin = r_begin / 32, t_end = r_end > r_begin ? cdiv(r_end, 32) : t_begin;
 
   f32x4 st[LPT];
@@ -2340,7 +1994,7 @@ void iso_accum_tiles2(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   constexpr int NV = 32 * V4;              // float4 per tile
   constexpr int LPT = (NV + NT - 1) / NT;  // float4 per thread per tile
   static_assert(NQ % 2 == 0 && kIsoChains == 2, "one chain per wave of a pair");
-  if (iso_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
+  if (call_mode(sel) != kModeDefault) return;       // the stored branch or the gathering kernel runs
   if (need_total(needcount) < dense_min) return;   // the gathering kernel runs (uniform exits)
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -2378,6 +2032,7 @@ void iso_accum_tiles2(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
+  if (r_end < r_begin) r_end = r_begin;   // a slab past N: no rows, a zero partial
   const int64_t t_begin = r_begin / 32, t_end = r_end > r_begin ? cdiv(r_end, 32) : t_begin;
 
   f32x4 st[LPT];
@@ -3126,7 +2781,7 @@ void iso_accum_ljt(const float* __restrict__ lj, const __bf16* __restrict__ xspl
   // iso_accum_sparse takes the call when pass 1 found the masks sparse; with a
   // selector word, the recomputing kernels take it unless the word is set.
   if (sparse_max >= 0 && need_total(ljcount) <= sparse_max) return;
-  if (sel != nullptr && iso_mode(sel) != kModeStored) return;
+  if (sel != nullptr && call_mode(sel) != kModeStored) return;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
 
@@ -3555,15 +3210,6 @@ void iso_accum_sparse(const float* __restrict__ X, int64_t ldx, int64_t N, const
 // ---------------------------------------------------------------------------
 // Finish: fixed-order fp64 reduction over slabs (deterministic).
 // ---------------------------------------------------------------------------
-// The partials a call left: `stored` of them where the stored branch ran, else `n`.
-struct PartCount {
-  const int* sel;
-  int n, stored;
-};
-__device__ __forceinline__ int part_count(const PartCount& p) {
-  return iso_mode(p.sel) == kModeStored ? p.stored : p.n;
-}
-
 // A workgroup sums 256 / G consecutive output columns (mu_acc rows, then Nk, then
 // sig_acc, as one list): G threads a column take the partials in turn (G = 4, 16), so the
 // loads of a wave stay in whole lines, and their sums are added in order.  One wave per
@@ -3691,7 +3337,7 @@ hipError_t launch_ctile(const IsoPlan& pl, const float* X, int64_t ldx, unsigned
 
 // The word that holds the device's choice of the call's branches (nullptr: none to make).
 const int* iso_sel(const IsoPlan& pl, unsigned char* ws) {
-  return pl.nprobe > 0 ? reinterpret_cast<const int*>(ws + pl.off_probe) + kProbeMode : nullptr;
+  return pl.nprobe > 0 ? reinterpret_cast<const int*>(ws + pl.off_state) + kStateMode : nullptr;
 }
 
 // The default plan up to D = 128, the stored plan's passes up to D = 128 and its
@@ -3711,10 +3357,9 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
   // A dense call computes every pair, so it never screens.  Both phases of a split call
   // evaluate the same choice.
   const bool screen = pl.screen && !dense && ldx <= kMaxScreenLdx;
-  unsigned* single = screen ? reinterpret_cast<unsigned*>(ws + pl.off_single) : nullptr;
   int* list = screen ? reinterpret_cast<int*>(ws + pl.off_list) : nullptr;
   unsigned* faint = screen ? reinterpret_cast<unsigned*>(ws + pl.off_faint) : nullptr;
-  float* near_nk = screen ? reinterpret_cast<float*>(ws + pl.off_nearnk) : nullptr;
+  unsigned* alive = screen ? reinterpret_cast<unsigned*>(ws + pl.off_state) + kStateAlive : nullptr;
   const int* sel = iso_sel(pl, ws);
   if (run1) {
     if constexpr (DP <= 128) {
@@ -3726,18 +3371,19 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
           hipLaunchKernelGGL((iso_store_probe<DP>), dim3((unsigned)pl.nprobe), dim3(64 * kProbeWaves), 0, stream, X, ldx, pl.N,
                              (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3), kc_blk, pl.KB,
                              screen ? reinterpret_cast<const float4*>(ws + pl.off_sce) : nullptr, pl.nprobe,
-                             IsoRule{screen ? (int64_t)pl.nprobe * 32 / 2 : -1, probe_min_pairs(pl.N, pl.nprobe, pl.KB),
+                             ProbeRule{screen ? (int64_t)pl.nprobe * 32 / 2 : -1, probe_min_pairs(pl.N, pl.nprobe, pl.KB),
                                      pl.autolj ? 1 : 0},
-                             reinterpret_cast<unsigned*>(ws + pl.off_probe));
+                             reinterpret_cast<unsigned*>(ws + pl.off_probe),
+                             reinterpret_cast<unsigned*>(ws + pl.off_state));
         if (screen) {
-          const size_t lds = screen_lds_bytes(DP, pl.KB);
+          const size_t lds = screen_lds_bytes(DP, false, pl.KB);
           if (lds > 65536)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&iso_screen<DP>),
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&screen_pairs<DP, false>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
           if (e != hipSuccess) return e;
-          hipLaunchKernelGGL(iso_screen<DP>, dim3((unsigned)cdiv(pl.N, 64 * kScreenWaves)), dim3(64 * kScreenWaves), lds,
+          hipLaunchKernelGGL((screen_pairs<DP, false>), dim3((unsigned)cdiv(pl.N, 64 * kScreenWaves)), dim3(64 * kScreenWaves), lds,
                              stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_scop),
-                             reinterpret_cast<const float4*>(ws + pl.off_sce), pl.KB, ljmask, faint, single, list, sel);
+                             reinterpret_cast<const float4*>(ws + pl.off_sce), pl.KB, ljmask, faint, 1, list, sel);
         }
         const bool st = pl.lj || pl.autolj;
         const size_t lds1 = lse_pipe_lds_bytes<DP>() + (pl.rexact ? (size_t)kPipeWaves * 32 * pl.KB * 2 : 0) +
@@ -3793,8 +3439,8 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
                            reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
                            reinterpret_cast<const double4*>(ws + pl.off_kcgat), pl.KB, pl.KP, rowstat,
                            words, ljcount, dense_min, pl.nslab, pl.rows_per_slab, pmu, pnk, psig,
-                           dense ? 1 : 0, sel, run1 && !faint_pass ? single : nullptr, kc_blk, logZ, run2 ? 0 : 1,
-                           near_nk, faint_pass);
+                           dense ? 1 : 0, sel, faint_pass ? ljmask : run1 ? faint : nullptr, kc_blk, logZ,
+                           run2 ? 0 : 1, alive, faint_pass);
       };
       gather(ljmask, 0);
       if (!run2) return hipGetLastError();
@@ -3805,10 +3451,12 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
         hipError_t et = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_t);
         if (et != hipSuccess) return et;
-        hipLaunchKernelGGL(kern, dim3((unsigned)(pl.nslab * cdiv(pl.KB, kTileBlocks))), dim3(64 * waves), lds_t,
+        // Each slab as its spp partials, a slab of rows each.
+        hipLaunchKernelGGL(kern, dim3((unsigned)(pl.nslab * pl.spp * cdiv(pl.KB, kTileBlocks))), dim3(64 * waves), lds_t,
                            stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
                            reinterpret_cast<const double4*>(ws + pl.off_kcgat), pl.KB, pl.KP, rowstat, ljmask,
-                           ljcount, dense_min, pl.nslab, pl.rows_per_slab, pmu, pnk, psig, dense ? 1 : 0, sel);
+                           ljcount, dense_min, pl.nslab * pl.spp, pl.rows_per_slab / pl.spp, pmu, pnk, psig,
+                           dense ? 1 : 0, sel);
         return hipGetLastError();
       };
       if constexpr (DP > 64) {
@@ -5027,7 +4675,7 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
                        pl.screen ? reinterpret_cast<bf16x8*>(ws + pl.off_scop) : nullptr,
                        pl.screen ? reinterpret_cast<float4*>(ws + pl.off_sce) : nullptr,
                        pl.screen ? reinterpret_cast<unsigned*>(ws + pl.off_list) : nullptr,
-                       pl.nprobe > 0 ? reinterpret_cast<unsigned*>(ws + pl.off_probe) : nullptr);
+                       pl.nprobe > 0 ? reinterpret_cast<unsigned*>(ws + pl.off_state) : nullptr);
   if (N > 0) {
     auto run = [&](auto dp_tag) -> hipError_t {
       constexpr int DP = decltype(dp_tag)::value;
@@ -5060,7 +4708,7 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
   const float* pnk = reinterpret_cast<const float*>(ws + pl.off_part_nk);
   const float* psig = reinterpret_cast<const float*>(ws + pl.off_part_sig);
   const int64_t nout = K * (D + 2);
-  const PartCount parts{iso_sel(pl, ws), pl.nslab * pl.rgroups, pl.nslab_lj * pl.rgroups};
+  const PartCount parts{iso_sel(pl, ws), pl.nslab * pl.spp * pl.rgroups, pl.nslab_lj * pl.rgroups};
   if (atomic) {
     if (!accumulate) {
       hipLaunchKernelGGL(fill_f32, dim3((unsigned)cdiv(K, 256)), dim3(256), 0, stream, Nk, K, 0.0f);
