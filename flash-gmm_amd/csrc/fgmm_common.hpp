@@ -796,10 +796,12 @@ struct ProbeSel {
   const unsigned* count;
   int n;
   int64_t min_pairs;
+  int64_t max_screen;   // up to this many sampled pairs: the screened pass 1 (-1: never)
 };
-// The stored branch is selected (uniform; false without a probe).
-__device__ __forceinline__ bool probe_selects(const ProbeSel& p) {
-  if (p.count == nullptr) return false;
+// The branch the probe selects (uniform; the default without a probe).
+constexpr int kProbeDefault = 0, kProbeStored = 1, kProbeScreen = 2;
+__device__ __forceinline__ int probe_mode(const ProbeSel& p) {
+  if (p.count == nullptr) return kProbeDefault;
   const int lane = threadIdx.x & 63;
   unsigned v = lane < p.n ? p.count[lane] : 0u;
   uint64_t t = v;
@@ -807,8 +809,9 @@ __device__ __forceinline__ bool probe_selects(const ProbeSel& p) {
   for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
   const uint64_t tot = (uint64_t)__builtin_amdgcn_readfirstlane((unsigned)t) |
                        ((uint64_t)__builtin_amdgcn_readfirstlane((unsigned)(t >> 32)) << 32);
-  return (int64_t)tot >= p.min_pairs;
+  return (int64_t)tot <= p.max_screen ? kProbeScreen : (int64_t)tot >= p.min_pairs ? kProbeStored : kProbeDefault;
 }
+__device__ __forceinline__ bool probe_selects(const ProbeSel& p) { return probe_mode(p) == kProbeStored; }
 // The sampled tiles (tile s of ntile is s * tiles / ntile) and the probe's
 // threshold: half of the sampled (row, block) pairs.
 __host__ __device__ inline int64_t probe_tile(int s, int64_t N, int ntile) { return (int64_t)s * cdiv(N, 32) / ntile; }

@@ -65,9 +65,10 @@ struct FullPlan {
                 // (FGMM_FLAG_STORE_LOGJOINT_AUTO, D <= 64): pass 1 also keeps the log-joint, and
                 // full_accum_ljt reads r from it over the same slabs and partials
   int nprobe;   // the probe's sampled tiles
+  bool screen;  // the probe may also select the screened pass 1 (full_screen)
   size_t off_probe;
   size_t off_lop, off_bsw, off_ck, off_l3, off_esw, off_rowstat, off_part_sig, off_part_mu, off_part_nk,
-      off_lj, off_need, off_bound, total;
+      off_lj, off_need, off_bound, off_sc, total;
 };
 
 // One LDS stage holds SMB 32-coordinate blocks of one component: all of them up to
@@ -122,6 +123,30 @@ __host__ __device__ constexpr int full_list_spill(int DP, int K) {
 // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO runs up to D = 64 (sig_outer's
 // accumulators and split operands of one component fit a wave's registers).
 __host__ __device__ constexpr bool flj_applies(int DP) { return DP <= 64; }
+
+// The screened pass 1 (see full_screen): calls with the probe, up to kScreenMaxK
+// components (the probe's estimate is in pairs: fewer than 16 components leave too little
+// to screen out) and at least kScreenMinWork (32-row tile, component, 32-coordinate block)
+// steps, below which its launches cost what it saves.  The fp64 log-joint of the needed
+// pairs is indexed [row][component], 8 bytes a pair, within kMaxLjBytes.
+constexpr int kScreenMinK = 16;
+constexpr int64_t kScreenMinWork = 40000;
+constexpr int kScreenTpw = 4;      // 32-row tiles per wave
+constexpr int kScreenPieces = 16;  // 1 KB operand pieces per LDS stage
+constexpr int kScreenConsts = 16;  // floats after a component's -b: c (up, down), the error's A, F, B
+template <int DP>
+struct ScreenShape {
+  static constexpr int NMB = DP / 32, NQ = DP / 16;
+  static constexpr int CPS = kScreenPieces / (NMB * NQ);   // components per stage
+  static constexpr int SCF = DP + kScreenConsts;
+  static constexpr int SCB = CPS * SCF * 4;
+  static constexpr int STAGE = kScreenPieces * 1024 + SCB;
+};
+constexpr int64_t kScreenRows = (int64_t)kWaves * kScreenTpw * 32;   // rows per workgroup
+__host__ inline size_t screen_region_bytes(int64_t N, int KP) {
+  return std::max((size_t)N * KP * sizeof(double),
+                  (size_t)round_up(N, kScreenRows) * KP * sizeof(unsigned short));
+}
 
 // Stored log-joint of the full model: per (32-row tile, component) 32 floats, rows
 // contiguous, [tile][KP][32]; the tiles of the pass-1 grid (rounded up to 8, a
@@ -188,6 +213,8 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   p.keep_lj = p.need && p.DP > 128 && !p.wide && full_lj_bytes(N, p.KP) <= kMaxLjBytes;
   p.autolj = p.need && auto_lj && flj_applies(p.DP) && N > 0 && K <= kProbeMaxKB &&
              full_lj_bytes(N, p.KP) <= kMaxLjBytes;
+  p.screen = p.autolj && K >= kScreenMinK && cdiv(N, 32) * K * p.NMB >= kScreenMinWork &&
+             screen_region_bytes(N, p.KP) <= kMaxLjBytes;
   p.nprobe = p.autolj ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
   // A list entry holds the component in 16 bits (the LDS limit keeps K far below that).
   p.needmode = !p.need ? kNeedRunMax
@@ -258,7 +285,9 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   p.off_part_mu = off;  off = align256(off + (size_t)p.npart * p.KP * p.DP * sizeof(float));
   p.off_part_nk = off;  off = align256(off + (size_t)p.npart * p.KP * sizeof(float));
   p.off_lj = off;
-  if (p.lj || p.keep_lj || p.autolj) off = align256(off + full_lj_bytes(N, p.KP));
+  // The screened pass 1's bounds and then its fp64 log-joint take the same bytes.
+  if (p.lj || p.keep_lj || p.autolj)
+    off = align256(off + std::max(full_lj_bytes(N, p.KP), p.screen ? screen_region_bytes(N, p.KP) : (size_t)0));
   // Need masks: one word per (32-row tile of the pass-1 grid, component).
   p.grid1 = 0;
   p.off_need = off;
@@ -273,6 +302,8 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   }
   p.off_probe = off;
   if (p.autolj) off = align256(off + probe_bytes() + (size_t)p.nprobe * p.KP * 32 * sizeof(float));
+  p.off_sc = off;
+  if (p.screen) off = align256(off + (size_t)p.KP * (p.DP + kScreenConsts) * sizeof(float));
   p.total = off;
   return p;
 }
@@ -299,8 +330,10 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
 __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu, int64_t ldmu,
                                                     const float* __restrict__ L, int64_t K, int D, int DP,
                                                     const float* __restrict__ lpi, bf16x8* __restrict__ l3,
-                                                    double* __restrict__ esw, double* __restrict__ ck) {
+                                                    double* __restrict__ esw, double* __restrict__ ck,
+                                                    float* __restrict__ sc) {
   __shared__ double so[16][256];  // o_qj, DP <= 256
+  __shared__ double red[3][4];    // sc: per wave, the squares of L - bf16(L), of bf16(L) and of b
   __shared__ double se[256];      // e_j, then log |L_jj|
   const int64_t k = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -319,6 +352,7 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
   }
   __syncthreads();
   // e_j = sum_q fp32(o_qj) - b_j with b_j = sum_q o_qj, both summed in q order.
+  double bt = 0.0;
   if (tid < DP) {
     double b = 0.0, osum = 0.0;
     for (int q = 0; q < NQ; ++q) {
@@ -326,8 +360,10 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
       b += so[q][tid];
     }
     se[tid] = osum - b;
+    bt = b;
   }
   __syncthreads();
+  double da = 0.0, df = 0.0;
   // Operands: (mb, q) pairs dealt over the four waves.
   for (int pq = wave; pq < NMB * NQ; pq += 4) {
     const int mb = pq / NQ, q = pq % NQ;
@@ -344,6 +380,14 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
     bf16x8* dst = l3 + (((k * NMB + mb) * NQ + q) * 4) * 64 + lane;
 #pragma unroll
     for (int t = 0; t < 3; ++t) dst[t * 64] = sp[t];
+    if (sc != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const double h = (double)(float)sp[0][e], r = (double)(e < 4 ? lo[e & 3] : hi[e & 3]) - h;
+        da = fma(r, r, da);
+        df = fma(h, h, df);
+      }
+    }
     // Offset slot: -o_qj in k slots 0..2 (lane-half 0), against x6c_ones.
     const float mo = -(float)so[q][j];
     const f32x4 olo = {g == 0 ? mo : 0.0f, 0.0f, 0.0f, 0.0f};
@@ -362,6 +406,27 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
     esw[(k * NMB + mb) * 32 + gg * 16 + i] = se[32 * mb + acc_row(i, gg)];
   }
   __syncthreads();
+  if (sc != nullptr) {
+    // The screening's -b in the accumulator's order (so[0] passes b on) and its norms.
+    double db = bt * bt;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      da += __shfl_xor(da, o);
+      df += __shfl_xor(df, o);
+      db += __shfl_xor(db, o);
+    }
+    if (lane == 0) {
+      red[0][wave] = da;
+      red[1][wave] = df;
+      red[2][wave] = db;
+    }
+    if (tid < DP) so[0][tid] = bt;
+    __syncthreads();
+    if (tid < DP) {
+      const int mb = tid / 32, gg = (tid >> 4) & 1, i = tid & 15;
+      sc[k * (DP + kScreenConsts) + tid] = -(float)so[0][32 * mb + acc_row(i, gg)];
+    }
+  }
   // c_k, the log-determinant summed in d order.
   if (tid < D) se[tid] = valid ? log(fabs((double)Lk[(int64_t)tid * D + tid]) + 1e-30) : 0.0;
   __syncthreads();
@@ -373,6 +438,20 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
       c0 = ((double)lpi[k] + ld - 0.5 * (double)D * kLog2Pi) * kLog2e;
     }
     ck[k] = c0;
+    if (sc != nullptr) {
+      // The bound's constants (see full_screen), each rounded outwards.
+      const double a = sqrt(red[0][0] + red[0][1] + red[0][2] + red[0][3]) * 1.0001;
+      const double f = sqrt(red[1][0] + red[1][1] + red[1][2] + red[1][3]) * 1.0001;
+      const double b = sqrt(red[2][0] + red[2][1] + red[2][2] + red[2][3]) * 1.0001;
+      const double cd = (double)(D + 32) * 0x1p-22;
+      const bool fin = fabs(c0) < 1e38;
+      float* o = sc + k * (DP + kScreenConsts) + DP;
+      o[0] = (float)(fin ? c0 + fabs(c0) * 0x1p-20 : c0);
+      o[1] = (float)(fin ? c0 - fabs(c0) * 0x1p-20 : -INFINITY);
+      o[2] = (float)((a + cd * f) * 1.0001);
+      o[3] = (float)(f * 1.0001);
+      o[4] = (float)(cd * b * 1.0001);
+    }
   }
 }
 
@@ -408,7 +487,7 @@ void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
   constexpr bool MASKS = LJM == kLjmNeed && !(KEEP && flj_applies(DP));
   // FGMM_FLAG_STORE_LOGJOINT_AUTO launches both need-mask instances; the probe's
   // counts let the KEEP one (the stored branch) or the other run.
-  if (probe.count != nullptr && probe_selects(probe) != KEEP) return;
+  if (probe.count != nullptr && probe_mode(probe) != (KEEP ? kProbeStored : kProbeDefault)) return;
   constexpr int NMB = DP / 32, NQ = DP / 16;
   constexpr int SMB = full_x6_smb(DP);            // coordinate blocks per stage
   constexpr int NST = NMB / SMB;                  // stages per component
@@ -1005,7 +1084,8 @@ __host__ inline int64_t gather_grid(int nslab, int K) { return gather_item_grid(
 
 // LJR: r comes from the log-joint pass 1 stored (keep_lj plans) instead of a
 // whitening of the queued rows.
-template <int DP, int GRP, bool LJR = false>
+// LLO (screened calls, GRP 0): only the fp64 log-joint of the pairs, to llo.
+template <int DP, int GRP, bool LJR = false, bool LLO = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kGatherWaves, 64 * kGatherWaves),
                           amdgpu_waves_per_eu(gather_waves_per_eu(DP), gather_waves_per_eu(DP))))
 void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
@@ -1013,10 +1093,14 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
                        const double* __restrict__ ck, int K, int KP, const double* __restrict__ rowstat,
                        const unsigned* __restrict__ need, int nslab, int64_t rows_per_slab,
                        float* __restrict__ part_sig, float* __restrict__ part_mu, float* __restrict__ part_nk,
-                       int dense, const float* __restrict__ lj, ProbeSel sel) {
+                       int dense, const float* __restrict__ lj, ProbeSel sel, double* __restrict__ llo) {
   constexpr int NMB = DP / 32, NQ = DP / 16, NSB = NMB * (NMB + 1) / 2;
   constexpr int NGRP = gather_sig_groups(DP);
-  if (probe_selects(sel)) return;   // the stored branch's full_accum_ljt takes the call
+  if constexpr (LLO) {
+    if (probe_mode(sel) != kProbeScreen) return;
+  } else {
+    if (probe_selects(sel)) return;   // the stored branch's full_accum_ljt takes the call
+  }
   constexpr int NSBG = (NSB + NGRP - 1) / NGRP;              // blocks per group
   constexpr int SB0 = GRP * NSBG;                            // this group's blocks SB0 .. SB1 - 1
   constexpr int SB1 = SB0 + NSBG < NSB ? SB0 + NSBG : NSB;
@@ -1133,8 +1217,10 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     bf16x8 xb[LJR ? 1 : NQ][3];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      *reinterpret_cast<f32x4*>(xt + c * RS + 16 * q + 8 * g) = raw[2 * q];
-      *reinterpret_cast<f32x4*>(xt + c * RS + 16 * q + 8 * g + 4) = raw[2 * q + 1];
+      if constexpr (!LLO) {
+        *reinterpret_cast<f32x4*>(xt + c * RS + 16 * q + 8 * g) = raw[2 * q];
+        *reinterpret_cast<f32x4*>(xt + c * RS + 16 * q + 8 * g + 4) = raw[2 * q + 1];
+      }
       if constexpr (!LJR) split3_bf16(raw[2 * q], raw[2 * q + 1], xb[q]);
     }
     const double lz2 = rst;
@@ -1165,6 +1251,13 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       }
       maha += __shfl_xor(maha, 32);
       const double ll = e_l[DP] - hl * maha;
+      if constexpr (LLO) {
+        if (g == 0 && e >= 0) llo[(r_begin + e) * KP + k] = ll;
+        if (!PREFETCH) cnt_next = take(en);
+        e = en;
+        cnt = cnt_next;
+        continue;
+      }
       rv = fast_exp2((float)(ll - lz2));
     }
     if (g == 0) {
@@ -1224,6 +1317,7 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     cnt = cnt_next;
   }
 
+  if constexpr (LLO) return;
   const int64_t pbase = (int64_t)slab * KP + k;
   float* ps = part_sig + pbase * NSB * 1024;
 #pragma unroll
@@ -1500,6 +1594,242 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The screened pass 1 (calls with the probe where it estimates at most an eighth of the
+// pairs as needed: clustered rows).  The exact whitening, 7 bf16 steps per 16 dimensions,
+// of nearly every (row, component) pair only shows that its responsibility is zero.
+// full_screen shows it with one: with Lh = bf16(L), xh = bf16(x) and v' = Lh^T xh - b,
+//   ||v - v'|| <= ||L - Lh||_F ||x|| + ||Lh||_F ||x - xh|| + fp32 rounding
+//              <= A ||x|| + F ||x - xh|| + B = E
+// (A, F, B per component from the prologue; the accumulation's rounding is at most
+// (D + 32) 2^-22 (||Lh||_F ||xh|| + ||b||), every add at 2^-23 of its partial sum), so
+// the log-joint lies between c - hl (||v'|| + E)^2 and c - hl max(0, ||v'|| - E)^2, each
+// rounded outwards.  A pair whose upper bound is kLjNeedGap below the row's largest lower
+// bound has a responsibility of exactly 0 in fp32 and adds nothing to logZ2.  Anything not
+// finite stays needed.  Then full_accum_gather<.., LLO> forms the exact fp64 log-joint of
+// the needed pairs, and full_need_lse each row's logZ2 and the exact need bits
+// (need_put_masks' test): pass 2 is the default plan's.
+//
+// full_screen: each wave holds kScreenTpw 32-row tiles in bf16, so an operand read from LDS
+// serves 128 rows (with two tiles LDS reads alone take as long as the matrix steps); a
+// stage of 16 KB (the first split of pass 1's operands) is two components at D = 64.  The
+// two half-waves trade their partial sums so that each lane owns one row of a tile pair.
+// Upper bounds go to `ub` as bf16 ([workgroup][wave][tile pair][component][64 rows], 128
+// bytes a store); once the row's largest lower bound is final each lane reads its own
+// back.  Bound: matrix steps and the squares' VALU, about equal.
+// N=250K K=256 D=64, clustered: the drop-in call 2.635 -> 0.708 ms (exact pass 1 2.45 ms;
+// traced: full_screen 0.565, the gathered log-joint 0.075, full_need_lse 0.020).
+// ---------------------------------------------------------------------------
+template <int DP>
+__global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads), amdgpu_waves_per_eu(2, 2)))
+void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ l3,
+                 const float* __restrict__ sc, int K, int KP, unsigned short* __restrict__ ub,
+                 unsigned* __restrict__ need, ProbeSel sel) {
+  if (probe_mode(sel) != kProbeScreen) return;
+  using SH = ScreenShape<DP>;
+  constexpr int NMB = SH::NMB, NQ = SH::NQ, CPS = SH::CPS, SCF = SH::SCF, TPW = kScreenTpw;
+  __shared__ __align__(16) unsigned char lds[2][SH::STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, g = lane >> 5;
+  const int64_t slot = (int64_t)blockIdx.x * kWaves + wave;
+
+  auto fetch = [&](int s) {
+    const int64_t left = (int64_t)KP - (int64_t)s * CPS;   // components, at least 1
+    const int64_t n = left < CPS ? left : CPS;
+    unsigned char* dst = lds[s & 1];
+    const DmaSrc r = dma_src(l3 + (int64_t)s * kScreenPieces * 4 * 64, (uint32_t)(n * NMB * NQ * 4096));
+#pragma unroll
+    for (int p = 0; p < kScreenPieces / kWaves; ++p) {
+      const int piece = wave * (kScreenPieces / kWaves) + p;
+      if (piece < n * NMB * NQ) lds_dma16(r, dst + piece * 1024, lane * 16, piece * 4096);
+    }
+    const DmaSrc rs = dma_src(sc + (int64_t)s * CPS * SCF, (uint32_t)(n * SCF * 4));
+    static_assert(SH::SCB <= 2048 && SH::SCB % 16 == 0, "two waves copy a stage's constants");
+    if (wave < 2 && wave * 1024 + lane * 16 < (int)n * SCF * 4)
+      lds_dma16(rs, dst + kScreenPieces * 1024 + wave * 1024, wave * 1024 + lane * 16, 0);
+  };
+  fetch(0);
+  bf16x8 xh[TPW][NQ];
+  float xn[TPW / 2], xe[TPW / 2], M[TPW / 2];   // the lane's row of each tile pair: ||x||, ||x - xh||
+  {
+    float n2[TPW], e2[TPW];
+#pragma unroll
+    for (int u = 0; u < TPW; ++u) {
+      const int64_t row = (slot * TPW + u) * 32 + c;
+      n2[u] = 0.0f;
+      e2[u] = 0.0f;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int d0 = 16 * q + 8 * g;
+        const f32x4 lo = load_row4(X, ldx, row, d0, D, row < N), hi = load_row4(X, ldx, row, d0 + 4, D, row < N);
+        xh[u][q] = to_bf16x8(lo, hi);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = e < 4 ? lo[e & 3] : hi[e & 3], r = x - (float)xh[u][q][e];
+          n2[u] = fmaf(x, x, n2[u]);
+          e2[u] = fmaf(r, r, e2[u]);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TPW / 2; ++j) {
+      const float n = (g ? n2[2 * j + 1] : n2[2 * j]) + __shfl_xor(g ? n2[2 * j] : n2[2 * j + 1], 32);
+      const float e = (g ? e2[2 * j + 1] : e2[2 * j]) + __shfl_xor(g ? e2[2 * j] : e2[2 * j + 1], 32);
+      xn[j] = fmaf(sqrtf(n), 1.0001f, 1e-18f);   // 1e-18: squares that underflow
+      xe[j] = fmaf(sqrtf(e), 1.0001f, 1e-18f);
+      M[j] = -INFINITY;
+    }
+  }
+  unsigned short* ubw = ub + slot * (TPW / 2) * KP * 64 + lane;
+  dma_barrier();
+
+  const float hlo = (float)(0.5 * kLog2e * (1.0 - 0x1p-19)), hhi = (float)(0.5 * kLog2e * (1.0 + 0x1p-19));
+  const int nstage = (K + CPS - 1) / CPS;
+  for (int s = 0; s < nstage; ++s) {
+    if (s + 1 < nstage) fetch(s + 1);
+    const bf16x8* la = reinterpret_cast<const bf16x8*>(lds[s & 1]) + lane;
+    const float* lc = reinterpret_cast<const float*>(lds[s & 1] + kScreenPieces * 1024);
+#pragma unroll 1
+    for (int cc = 0; cc < CPS; ++cc) {
+      const int k = s * CPS + cc;
+      if (k >= K) break;   // uniform
+      float ss[TPW];
+#pragma unroll
+      for (int u = 0; u < TPW; ++u) ss[u] = 0.0f;
+#pragma unroll
+      for (int mb = 0; mb < NMB; ++mb) {
+        f32x16 b;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(lc + cc * SCF + mb * 32 + g * 16 + 4 * j);
+          b[4 * j] = v.x; b[4 * j + 1] = v.y; b[4 * j + 2] = v.z; b[4 * j + 3] = v.w;
+        }
+        f32x16 t[TPW];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const bf16x8 a = la[((cc * NMB + mb) * NQ + q) * 64];
+#pragma unroll
+          for (int u = 0; u < TPW; ++u) t[u] = mfma_bf16(a, xh[u][q], q == 0 ? b : t[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < TPW; ++u) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) ss[u] = fmaf(t[u][i], t[u][i], ss[u]);
+        }
+      }
+      const float* kc = lc + cc * SCF + DP;
+      const float cu = kc[0], cl = kc[1], ea = kc[2], ef = kc[3], eb = kc[4];
+#pragma unroll
+      for (int j = 0; j < TPW / 2; ++j) {
+        const float v2 = (g ? ss[2 * j + 1] : ss[2 * j]) + __shfl_xor(g ? ss[2 * j] : ss[2 * j + 1], 32);
+        // 2^-14 covers the squares' sum and the root, 1.0001 the bound's own rounding.
+        const float rt = __builtin_amdgcn_sqrtf(v2);
+        const float E = fmaf(ea, xn[j], fmaf(ef, xe[j], eb)) * 1.0001f;
+        const float lo = fmaxf(fmaf(rt, 1.0f - 0x1p-14f, -E), 0.0f), hi = fmaf(rt, 1.0f + 0x1p-14f, E);
+        float up = fmaf(-hlo * lo, lo, cu);
+        up = v2 < 3e38f ? up : INFINITY;
+        M[j] = fmaxf(M[j], fmaf(-hhi * hi, hi, cl));
+        ubw[((int64_t)j * KP + k) * 64] = bf16_bits_up(up);
+      }
+    }
+    dma_barrier();
+  }
+  // The lane's bounds against its row's largest lower bound; lane i collects the words of
+  // component k0 + i, so that 64 go out in one store.
+#pragma unroll
+  for (int j = 0; j < TPW / 2; ++j) {
+    const int64_t tile = slot * TPW + 2 * j;
+    if (tile * 32 >= N) break;
+    const bool valid = (tile + g) * 32 + c < N;
+    const float thr = M[j] - kLjNeedGap;
+    for (int k0 = 0; k0 < K; k0 += 64) {
+      unsigned w0 = 0u, w1 = 0u;
+#pragma unroll 8
+      for (int i = 0; i < 64; ++i) {
+        const int k = k0 + i < K ? k0 + i : K - 1;
+        const float R = bf16_bits_to_float(ubw[((int64_t)j * KP + k) * 64]);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(valid && !(R < thr));
+        w0 = lane == i ? (unsigned)m : w0;
+        w1 = lane == i ? (unsigned)(m >> 32) : w1;
+      }
+      if (k0 + lane < K) {
+        need[tile * KP + k0 + lane] = w0;
+        if ((tile + 1) * 32 < N) need[(tile + 1) * KP + k0 + lane] = w1;
+      }
+    }
+  }
+}
+
+// Each row's logZ2 from the log-joint of its needed pairs, in pass 1's component order
+// and arithmetic, then the exact need bits.  One wave per 32-row tile; eight components'
+// loads in flight.  Bound: latency.
+__global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, const double* __restrict__ ll,
+                                                     unsigned* __restrict__ need, double* __restrict__ rowstat,
+                                                     float* __restrict__ logZ, ProbeSel sel) {
+  if (probe_mode(sel) != kProbeScreen) return;
+  const int lane = threadIdx.x & 63, c = lane & 31;
+  const int64_t tile = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t row = tile * 32 + c;
+  if (tile * 32 >= N) return;   // uniform over the wave
+  const double* lr = ll + (row < N ? row : N - 1) * KP;
+  unsigned* nw = need + tile * KP;
+  // f(component, this lane's row needs it, its log-joint) over the tile's nonzero words.
+  auto pairs = [&](unsigned w, int k0, auto f) {
+    uint64_t bits = __builtin_amdgcn_ballot_w64(w != 0u);
+    while (bits != 0) {
+      int kk[8];
+      double v[8];
+      bool in[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        kk[j] = bits != 0 ? __builtin_ctzll(bits) : -1;
+        bits = bits != 0 ? bits & (bits - 1) : 0;
+        const unsigned word = kk[j] >= 0 ? (unsigned)__builtin_amdgcn_readlane((int)w, kk[j] & 63) : 0u;
+        in[j] = (word >> c) & 1u;
+        v[j] = 0.0;
+        if (in[j]) v[j] = lr[k0 + kk[j]];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (kk[j] >= 0) f(kk[j], in[j], v[j]);
+    }
+  };
+  double mx = -INFINITY;
+  float sm = 0.0f;
+  int n = 0;
+  for (int k0 = 0; k0 < K; k0 += 64) {
+    const unsigned w = k0 + lane < K ? nw[k0 + lane] : 0u;
+    pairs(w, k0, [&](int, bool in, double v) {
+      if (!in) return;
+      const double mn = fmax(mx, v);
+      const double ms = mn == -INFINITY ? 0.0 : mn;
+      sm = sm * fast_exp2((float)(mx - ms)) + fast_exp2((float)(v - ms));
+      mx = mn;
+      ++n;
+    });
+  }
+  const double lz2 = mx + (double)log2f(sm);
+  if (row < N && lane < 32) {
+    rowstat[row] = lz2;
+    if (logZ) logZ[row] = (float)(lz2 * kLn2);
+  }
+  // A row's only pair is needed.
+  if (__builtin_amdgcn_ballot_w64(n > 1) == 0) return;
+  const float zx = (float)lz2;
+  const float zy = (lz2 > -INFINITY && lz2 < INFINITY) ? (float)(lz2 - (double)zx) : 0.0f;
+  for (int k0 = 0; k0 < K; k0 += 64) {
+    const unsigned w = k0 + lane < K ? nw[k0 + lane] : 0u;
+    unsigned nwd = w;
+    pairs(w, k0, [&](int kk, bool in, double v) {
+      const float R = bf16_bits_to_float(bf16_bits_up((float)v));
+      const unsigned m = (unsigned)__builtin_amdgcn_ballot_w64(in && !(((R - zx) - zy) < -kLjNeedGap));
+      if (lane == kk) nwd = m;
+    });
+    if (nwd != w) nw[k0 + lane] = nwd;
+  }
+}
+
 template <int DP>
 hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsigned char* ws,
                          float* logZ, bool run1, bool run2, bool dense, hipStream_t stream) {
@@ -1512,8 +1842,10 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
   };
   // FGMM_FLAG_STORE_LOGJOINT_AUTO: the probe's counts select the branch in both passes.
   unsigned* probe = pl.autolj ? reinterpret_cast<unsigned*>(ws + pl.off_probe) : nullptr;
-  const ProbeSel psel = probe ? ProbeSel{probe, pl.nprobe, probe_min_pairs(pl.N, pl.nprobe, (int)pl.K)}
-                              : ProbeSel{nullptr, 0, 0};
+  // The screened pass 1 up to an eighth of the sampled pairs (a quarter of the stored
+  // branch's least, half of them).
+  const int64_t min_pairs = probe ? probe_min_pairs(pl.N, pl.nprobe, (int)pl.K) : 0;
+  const ProbeSel psel = {probe, pl.nprobe, min_pairs, pl.screen && !dense ? min_pairs / 4 : (int64_t)-1};
   if (run1) {
     if constexpr (flj_applies(DP)) {
       if (pl.autolj) {
@@ -1561,6 +1893,24 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                            lj, reinterpret_cast<unsigned*>(ws + pl.off_need),
                            reinterpret_cast<unsigned short*>(ws + pl.off_bound), dense ? 1 : 0, psel);
       }
+      if (pl.screen && !dense) {
+        unsigned* need = reinterpret_cast<unsigned*>(ws + pl.off_need);
+        double* ll = reinterpret_cast<double*>(ws + pl.off_lj);
+        hipLaunchKernelGGL((full_screen<DP>), dim3((unsigned)cdiv(pl.N, kScreenRows)), dim3(kThreads), 0, stream, X,
+                           ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
+                           reinterpret_cast<const float*>(ws + pl.off_sc), (int)pl.K, pl.KP,
+                           reinterpret_cast<unsigned short*>(ws + pl.off_lj), need, psel);
+        constexpr size_t ldsg = gather_lds_bytes<DP>();
+        auto kll = &full_accum_gather<DP, 0, false, true>;
+        e = set_lds(reinterpret_cast<const void*>(kll), ldsg);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kll, dim3((unsigned)gather_grid(pl.nslab, (int)pl.K)), dim3(64 * kGatherWaves), ldsg,
+                           stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
+                           reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat, need,
+                           pl.nslab, pl.rows_per_slab, nullptr, nullptr, nullptr, 0, nullptr, psel, ll);
+        hipLaunchKernelGGL(full_need_lse, dim3((unsigned)cdiv(pl.N, 128)), dim3(256), 0, stream, pl.N, (int)pl.K,
+                           pl.KP, ll, need, rowstat, logZ, psel);
+      }
     }
   }
   if (!run2) return hipGetLastError();
@@ -1583,7 +1933,7 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                              reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                              reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat,
                              reinterpret_cast<const unsigned*>(ws + pl.off_need), pl.nslab, pl.rows_per_slab,
-                             psig, pmu, pnk, dense ? 1 : 0, lj, psel);
+                             psig, pmu, pnk, dense ? 1 : 0, lj, psel, nullptr);
         }
         return hipSuccess;
       };
@@ -2589,7 +2939,8 @@ extern "C" int fgmm_full_estep_f32(const float* X, int64_t ldx, int64_t N, int64
   else if (run1)
     hipLaunchKernelGGL(full_x6_prep, dim3((unsigned)pl.KP), dim3(256), 0, stream, mu, ldmu, prec_chol, K,
                        (int)D, pl.DP, log_pi, reinterpret_cast<bf16x8*>(ws + pl.off_l3),
-                       reinterpret_cast<double*>(ws + pl.off_esw), reinterpret_cast<double*>(ws + pl.off_ck));
+                       reinterpret_cast<double*>(ws + pl.off_esw), reinterpret_cast<double*>(ws + pl.off_ck),
+                       pl.screen ? reinterpret_cast<float*>(ws + pl.off_sc) : nullptr);
   if (N > 0) {
     auto run = [&](auto dp_tag) -> hipError_t {
       constexpr int DP = decltype(dp_tag)::value;

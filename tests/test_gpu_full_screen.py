@@ -1,0 +1,67 @@
+"""The full model's screened pass 1 (the drop-in call on clustered rows): against the
+default plan, whose exact pass 1 sees every pair, and against the float64 oracle."""
+
+import math
+
+import pytest
+import torch
+
+from flash_gmm import data, full_estep_into
+from oracle import gmm_oracle as O
+from parity import assert_close_stats, assert_dense_agrees
+
+pytestmark = pytest.mark.gpu
+KEYS = ("X", "mu", "prec_chol", "log_pi")
+
+
+def call(inp, dev, store):
+    args = [inp[k].to(dev) for k in KEYS]
+    N, D = args[0].shape
+    K = args[1].shape[0]
+    out = [torch.full((N,), math.nan, device=dev), torch.empty(K, device=dev), torch.empty(K, D, device=dev),
+           torch.empty(K, D, D, device=dev)]
+    full_estep_into(*args, *out, store_log_joint=store)
+    torch.cuda.synchronize()
+    return out
+
+
+def same(got, want, what):
+    """logZ bit for bit; the sums, whose terms the default plan's wider masks may group
+    otherwise, as assert_dense_agrees takes two groupings; NaN where it is NaN."""
+    for name, u, v in zip(("logZ", "Nk", "mu_acc", "sig_outer"), got, want):
+        assert torch.equal(u.isnan(), v.isnan()), f"{what} {name}: NaN"
+    assert_dense_agrees([u.nan_to_num(0.0) for u in got], [v.nan_to_num(0.0) for v in want], bitwise=False)
+
+
+# Widths 32 and 64, a last stage of 1, 4 and all of its components, a last tile of 1 row, a
+# last workgroup of one tile, D that is no multiple of 4.
+@pytest.mark.parametrize("N,K,D", [(5_153, 256, 32), (9_217, 301, 64), (40_033, 100, 39), (90_001, 17, 50),
+                                   (30_001, 77, 17)])
+def test_screened_sizes(N, K, D, gpu_device):
+    print(f"full screen N={N} K={K} D={D}", flush=True)
+    inp = data.full_clustered(N, K, D, seed=K % 13)
+    got = call(inp, gpu_device, "auto")
+    same(got, call(inp, gpu_device, False), f"N={N} K={K} D={D}")
+    assert_close_stats(got, O.estep_full(*[inp[k] for k in KEYS]), f"full screen N={N} K={K} D={D}")
+
+
+def test_rows_of_several_and_special_components(gpu_device):
+    """Components in close pairs and far away, zero weights, then NaN, infinite and huge rows."""
+    inp = data.full_clustered(20_000, 128, 40, seed=5)
+    g = torch.Generator().manual_seed(1)
+    inp["mu"][64:100] = inp["mu"][:36] + 0.05 * torch.randn(36, 40, generator=g)
+    inp["prec_chol"][64:100] = inp["prec_chol"][:36]
+    inp["mu"][100:110] *= 50.0
+    inp["log_pi"][110:120] = -math.inf
+    print("full screen paired", flush=True)
+    got = call(inp, gpu_device, "auto")
+    same(got, call(inp, gpu_device, False), "paired")
+    assert (got[1][110:120] == 0).all()
+    inp["X"][7, 3] = math.nan
+    inp["X"][10_000, 39] = math.inf
+    inp["X"][19_999] = 1e-25
+    print("full screen special rows", flush=True)
+    same(call(inp, gpu_device, "auto"), call(inp, gpu_device, False), "special rows")
+    inp["X"][7] = inp["X"][10_000] = 1e18   # finite; the screening's squares are not all
+    print("full screen huge rows", flush=True)
+    same(call(inp, gpu_device, "auto"), call(inp, gpu_device, False), "huge rows")
