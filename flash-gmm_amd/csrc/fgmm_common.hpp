@@ -943,6 +943,20 @@ __host__ inline int64_t gather_slab_count(int64_t want, int64_t max_slabs, int W
   const int64_t n = g * W;
   return n < max_slabs ? n : max_slabs;
 }
+// Slabs of the gathering passes that hold one workgroup per compute unit (above D = 64,
+// two partials a slab): between half of `want` (its partials are then as long) and `want`,
+// the group count whose rounds of workgroups take least, rounds / groups, the smallest of
+// equals.  A fixed half took two rounds for 280 workgroups on 256 compute units:
+// diagonal N=554K K=202 D=101, N(0, I) rows: pass 2 2.06 ms; two fixed rounds of twice the
+// slabs 1.56 ms, and these whole rounds bring the call from 2.59 to 1.77 ms.
+__host__ inline int64_t gather_slab_rounds(int64_t want, int64_t max_slabs, int W, int64_t items, int64_t cus) {
+  const int64_t most = cdiv(gather_slab_count(want, INT64_MAX, W), W);
+  int64_t best = most;
+  for (int64_t g = most; 2 * g >= most && g >= 1; g = g > 8 ? g - 8 : g / 2)
+    if (cdiv(g * items, cus) * best <= cdiv(best * items, cus) * g) best = g;
+  const int64_t n = best * W;
+  return n < max_slabs ? n : max_slabs;
+}
 // The gathering passes read a slab's row state (logZ2, and ||x||^2 for the isotropic
 // model) through one buffer resource whose byte offsets are 32-bit: a slab holds at
 // most this many rows, so the offsets stay below 2^31 whatever N and K are (beyond

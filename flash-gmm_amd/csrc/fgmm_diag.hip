@@ -220,17 +220,20 @@ DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
   } else if (p.need && N > 0 && p.KB > 0) {
-    // The gathering pass 2: one round of waves, two per SIMD up to D = 64, one above.
+    // The gathering pass 2: one round of waves, two per SIMD, up to D = 64; whole rounds
+    // of one wave per SIMD above (gather_slab_rounds).
     // The stored branch's pass 2 takes eight blocks per compute unit; the partials are
     // laid out for it with or without the branch.
-    auto slabs = [&](int64_t waves, int64_t& rows) {
-      const int64_t want = gather_slab_count(cdiv(waves * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
+    auto slabs = [&](int64_t waves, int64_t& rows, bool one_round) {
+      const int64_t n = cdiv(waves * current_device_cus(), p.KB);
+      const int64_t want = one_round ? gather_slab_rounds(n, cdiv(N, 32), kGatherWaves, p.KB, current_device_cus())
+                                     : gather_slab_count(n, cdiv(N, 32), kGatherWaves);
       rows = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
       return (int)cdiv(N, rows);
     };
     p.spp = gather_parts(p.DP);
-    p.nslab = slabs(p.DP <= 64 ? 8 : 4, p.rows_per_slab);
-    p.nslab_lj = slabs(8, p.rows_per_slab_lj);
+    p.nslab = slabs(8, p.rows_per_slab, p.DP > 64);
+    p.nslab_lj = slabs(8, p.rows_per_slab_lj, false);
   } else if (N > 0 && p.ncg > 0) {
     int64_t want = (int64_t)current_device_cus() / p.ncg;
     if (want >= 8) want = (want / 8) * 8;

@@ -273,13 +273,15 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double2));
     p.nslab = (int)cdiv(N, p.rows_per_slab);
   } else if (p.need && N > 0 && p.KB > 0) {
-    // The gathering pass 2: one round of waves, two per SIMD up to D = 64, one above
+    // The gathering pass 2: one round of waves, two per SIMD, up to D = 64; whole rounds
+    // of one wave per SIMD above
     // (there, 64 slabs in two rounds took 0.266 ms at N=1M K=1024 D=128, 32 slabs take
     // 0.247 ms; their float32 sums go out in two partials each, so that they are no
     // longer).  The stored branch's pass 2 takes eight blocks per compute unit.
     p.spp = gather_parts(p.DP);
-    const int64_t rounds = p.DP <= 64 ? 8 : 4;
-    const int64_t want = gather_slab_count(cdiv(rounds * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
+    const int64_t cus = current_device_cus(), full = cdiv(8 * cus, p.KB);
+    const int64_t want = p.DP <= 64 ? gather_slab_count(full, cdiv(N, 32), kGatherWaves)
+                                    : gather_slab_rounds(full, cdiv(N, 32), kGatherWaves, p.KB, cus);
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32 * p.spp), sizeof(double2)) / (32 * p.spp) * (32 * p.spp);
     p.nslab = (int)cdiv(N, p.rows_per_slab);
     if (p.DP <= 128) {   // its partials are laid out with or without the branch
