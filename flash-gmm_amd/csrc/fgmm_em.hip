@@ -104,19 +104,30 @@ __global__ __launch_bounds__(256) void diag_mstep_kernel(const float* __restrict
 constexpr int kFullMstepMaxD = 4096;
 constexpr size_t kMstepScratchBytes = (size_t)1 << 30;
 
-__global__ __launch_bounds__(256) void full_mstep_kernel(const float* __restrict__ Nk,
-                                                         const float* __restrict__ mu_acc,
-                                                         const float* __restrict__ sig_outer, double N,
-                                                         int D, double reg, float* __restrict__ mu,
-                                                         int64_t ldmu, float* __restrict__ prec_chol,
-                                                         float* __restrict__ lpi, int* __restrict__ info) {
+// Bound: the D serial steps' latency.  One barrier a step: the Cholesky is right-looking on
+// unscaled columns (S_ab -= S_aj S_bj / d_j), and each step also adds its column's terms to
+// the inverse, whose accumulators lie below the diagonal: with U_aj = S_aj w_j, w_j =
+// 1/sqrt(d_j), row j of W is -S_cj w_j (c > j), so all elements (a < j, y) of a step are
+// S -= S_aj S_yj / d_j (y == j: S = S_aj / d_j), independent of one another.
+// kMstepRow threads take consecutive y; rows have an odd stride (the accumulators are
+// walked down a column).
+// K=32 D=39: 73 us before (three barriers a step, then one thread per column of the inverse);
+// a three-iteration fit at N=100K 1.00 -> 0.89 ms.
+constexpr int kMstepThreads = 512, kMstepRow = 32;
+__host__ __device__ constexpr int mstep_stride(int D) { return D | 1; }
+
+__global__ __launch_bounds__(kMstepThreads) void full_mstep_kernel(
+    const float* __restrict__ Nk, const float* __restrict__ mu_acc, const float* __restrict__ sig_outer, double N,
+    int D, double reg, float* __restrict__ mu, int64_t ldmu, float* __restrict__ prec_chol, float* __restrict__ lpi,
+    int* __restrict__ info) {
   extern __shared__ double lds_d[];
-  double* S = lds_d;            // D x D: U in the upper triangle, W^T below it
-  double* m = S + D * D;        // new mean
+  const int RS = mstep_stride(D);
+  double* S = lds_d;            // D x D
+  double* m = S + D * RS;       // new mean
   double* wd = m + D;           // diagonal of W
-  __shared__ double piv;
   const int64_t k = blockIdx.x;
-  const int t = threadIdx.x, nt = blockDim.x;
+  const int t = threadIdx.x, nt = kMstepThreads;
+  const int tx = t % kMstepRow, ty = t / kMstepRow, na = kMstepThreads / kMstepRow;
   const double nk = (double)Nk[k];
   if (!(nk > 0.0)) {
     if (t == 0) lpi[k] = -INFINITY;
@@ -125,50 +136,38 @@ __global__ __launch_bounds__(256) void full_mstep_kernel(const float* __restrict
   for (int i = t; i < D; i += nt) m[i] = (double)mu_acc[k * D + i] / nk;
   __syncthreads();
   const float* so = sig_outer + k * (int64_t)D * D;
-  for (int e = t; e < D * D; e += nt) {
-    const int i = e / D, j = e % D;
-    double v = 0.5 * ((double)so[i * D + j] + (double)so[j * D + i]) / nk - m[i] * m[j];
-    if (i == j) v += reg;
-    S[e] = v;
-  }
-  __syncthreads();
-  bool indefinite = false;   // thread 0 only
+  for (int i = ty; i < D; i += na)
+    for (int j = tx; j < D; j += kMstepRow) {
+      double v = 0.5 * ((double)so[i * D + j] + (double)so[j * D + i]) / nk - m[i] * m[j];
+      if (i == j) v += reg;
+      S[i * RS + j] = v;
+    }
+  bool indefinite = false;
   for (int j = D - 1; j >= 0; --j) {
-    if (t == 0) {
-      double d = S[j * D + j];
-      if (!(d > 0.0)) {
-        d = reg > 0.0 ? reg : 1e-30;
-        indefinite = true;
+    __syncthreads();
+    double d = S[j * RS + j];
+    if (!(d > 0.0)) {
+      d = reg > 0.0 ? reg : 1e-30;
+      indefinite = true;
+    }
+    if (t == 0) wd[j] = 1.0 / sqrt(d);
+    const double q = 1.0 / d;
+    for (int y = tx; y < D; y += kMstepRow) {
+      const double f = y == j ? -q : S[y * RS + j] * q;
+      const int last = y < j ? y : j - 1;   // above the diagonal: a <= y
+      for (int a = ty; a <= last; a += na) {
+        const double sa = S[a * RS + j];
+        double* e = y < j ? S + a * RS + y : S + y * RS + a;
+        *e = y == j ? -sa * f : *e - sa * f;
       }
-      piv = sqrt(d);
-      S[j * D + j] = piv;
     }
-    __syncthreads();
-    const double p = piv;
-    for (int i = t; i < j; i += nt) S[i * D + j] /= p;
-    __syncthreads();
-    for (int e = t; e < j * j; e += nt) {
-      const int a = e / j, b = e % j;
-      if (a <= b) S[a * D + b] -= S[a * D + j] * S[b * D + j];
-    }
-    __syncthreads();
   }
   if (t == 0 && indefinite && info) atomicAdd(info, 1);
-  // Column c of W = U^-1 by back substitution, stored transposed in row c below the diagonal.
-  for (int c = t; c < D; c += nt) {
-    wd[c] = 1.0 / S[c * D + c];
-    for (int i = c - 1; i >= 0; --i) {
-      double acc = S[i * D + c] * wd[c];
-      for (int l = i + 1; l < c; ++l) acc += S[i * D + l] * S[c * D + l];
-      S[c * D + i] = -acc / S[i * D + i];
-    }
-  }
   __syncthreads();
   float* L = prec_chol + k * (int64_t)D * D;
-  for (int e = t; e < D * D; e += nt) {
-    const int i = e / D, j = e % D;
-    L[e] = (float)(j < i ? S[i * D + j] : (j == i ? wd[i] : 0.0));
-  }
+  for (int i = ty; i < D; i += na)
+    for (int j = tx; j < D; j += kMstepRow)
+      L[i * D + j] = (float)(j < i ? -S[i * RS + j] * wd[j] : (j == i ? wd[i] : 0.0));
   for (int i = t; i < D; i += nt) mu[k * ldmu + i] = (float)m[i];
   if (t == 0) lpi[k] = (float)log(nk / N);
 }
@@ -403,13 +402,13 @@ extern "C" int fgmm_full_mstep_f32(const float* Nk, const float* mu_acc, const f
     const hipError_t fe = hipFreeAsync(scratch, (hipStream_t)stream);
     return le == hipSuccess && fe == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
   }
-  const size_t lds = ((size_t)D * D + 2 * (size_t)D) * sizeof(double);
+  const size_t lds = ((size_t)D * mstep_stride((int)D) + 2 * (size_t)D) * sizeof(double);
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&full_mstep_kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return FGMM_ERR_HIP;
   }
-  hipLaunchKernelGGL(full_mstep_kernel, dim3((unsigned)K), dim3(256), lds, (hipStream_t)stream, Nk,
+  hipLaunchKernelGGL(full_mstep_kernel, dim3((unsigned)K), dim3(kMstepThreads), lds, (hipStream_t)stream, Nk,
                      mu_acc, sig_outer, (double)N, (int)D, reg_covar, mu, ldmu, prec_chol, log_pi, info);
   return hipGetLastError() == hipSuccess ? FGMM_OK : FGMM_ERR_HIP;
 }
