@@ -386,6 +386,9 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
         const double h = (double)(float)sp[0][e], r = (double)(e < 4 ? lo[e & 3] : hi[e & 3]) - h;
         da = fma(r, r, da);
         df = fma(h, h, df);
+        // The screening leaves out the blocks above L's diagonal; a component with
+        // anything there (NaN too) gets no bound.
+        if (q < 2 * mb && !(h + r == 0.0)) da = INFINITY;
       }
     }
     // Offset slot: -o_qj in k slots 0..2 (lane-half 0), against x6c_ones.
@@ -1616,8 +1619,11 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // two half-waves trade their partial sums so that each lane owns one row of a tile pair.
 // Upper bounds go to `ub` as bf16 ([workgroup][wave][tile pair][component][64 rows], 128
 // bytes a store); once the row's largest lower bound is final each lane reads its own
-// back.  Bound: matrix steps and the squares' VALU, about equal.
-// N=250K K=256 D=64, clustered: the drop-in call 2.635 -> 0.708 ms (exact pass 1 2.45 ms;
+// back.  Bound: matrix steps and the squares' VALU, about equal.  The steps of the blocks
+// above L's diagonal (2 of 8 at D = 64) are left out: a component with a nonzero there
+// has A = infinity, so nothing of it is screened.
+// N=250K K=256 D=64, clustered: the drop-in call 2.670 -> 0.655 ms (0.705 with all eight
+// steps; exact pass 1 2.45 ms;
 // traced: full_screen 0.565, the gathered log-joint 0.075, full_need_lse 0.020).
 // ---------------------------------------------------------------------------
 template <int DP>
@@ -1642,7 +1648,8 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
 #pragma unroll
     for (int p = 0; p < kScreenPieces / kWaves; ++p) {
       const int piece = wave * (kScreenPieces / kWaves) + p;
-      if (piece < n * NMB * NQ) lds_dma16(r, dst + piece * 1024, lane * 16, piece * 4096);
+      const bool upper = piece % NQ < 2 * (piece / NQ % NMB);
+      if (piece < n * NMB * NQ && !upper) lds_dma16(r, dst + piece * 1024, lane * 16, piece * 4096);
     }
     const DmaSrc rs = dma_src(sc + (int64_t)s * CPS * SCF, (uint32_t)(n * SCF * 4));
     static_assert(SH::SCB <= 2048 && SH::SCB % 16 == 0, "two waves copy a stage's constants");
@@ -1707,10 +1714,10 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
         }
         f32x16 t[TPW];
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
+        for (int q = 2 * mb; q < NQ; ++q) {   // L is lower-triangular
           const bf16x8 a = la[((cc * NMB + mb) * NQ + q) * 64];
 #pragma unroll
-          for (int u = 0; u < TPW; ++u) t[u] = mfma_bf16(a, xh[u][q], q == 0 ? b : t[u]);
+          for (int u = 0; u < TPW; ++u) t[u] = mfma_bf16(a, xh[u][q], q == 2 * mb ? b : t[u]);
         }
 #pragma unroll
         for (int u = 0; u < TPW; ++u) {

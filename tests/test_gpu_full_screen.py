@@ -53,6 +53,7 @@ def test_rows_of_several_and_special_components(gpu_device):
     inp["prec_chol"][64:100] = inp["prec_chol"][:36]
     inp["mu"][100:110] *= 50.0
     inp["log_pi"][110:120] = -math.inf
+    inp["prec_chol"][120:124, 3, 37] = 5.0   # above the diagonal: taken as it is
     print("full screen paired", flush=True)
     got = call(inp, gpu_device, "auto")
     same(got, call(inp, gpu_device, False), "paired")
