@@ -66,6 +66,7 @@ struct FullPlan {
                 // full_accum_ljt reads r from it over the same slabs and partials
   int nprobe;   // the probe's sampled tiles
   bool screen;  // the probe may also select the screened pass 1 (full_screen)
+  int screen_cap;   // its pool of log-joints per tile
   size_t off_probe;
   size_t off_lop, off_bsw, off_ck, off_l3, off_esw, off_rowstat, off_part_sig, off_part_mu, off_part_nk,
       off_lj, off_need, off_bound, off_sc, total;
@@ -127,8 +128,9 @@ __host__ __device__ constexpr bool flj_applies(int DP) { return DP <= 64; }
 // The screened pass 1 (see full_screen): calls with the probe, up to kScreenMaxK
 // components (the probe's estimate is in pairs: fewer than 16 components leave too little
 // to screen out) and at least kScreenMinWork (32-row tile, component, 32-coordinate block)
-// steps, below which its launches cost what it saves.  The fp64 log-joint of the needed
-// pairs is indexed [row][component], 8 bytes a pair, within kMaxLjBytes.
+// steps, below which its launches cost what it saves.  In the stored branch's log-joint
+// space: the bounds, 2 bytes a pair, then per tile a pool of screen_cap doubles (about a
+// quarter of its pairs) for the needed pairs' fp64 log-joint.
 constexpr int kScreenMinK = 16;
 constexpr int64_t kScreenMinWork = 40000;
 constexpr int kScreenTpw = 4;      // 32-row tiles per wave
@@ -143,9 +145,8 @@ struct ScreenShape {
   static constexpr int STAGE = kScreenPieces * 1024 + SCB;
 };
 constexpr int64_t kScreenRows = (int64_t)kWaves * kScreenTpw * 32;   // rows per workgroup
-__host__ inline size_t screen_region_bytes(int64_t N, int KP) {
-  return std::max((size_t)N * KP * sizeof(double),
-                  (size_t)round_up(N, kScreenRows) * KP * sizeof(unsigned short));
+__host__ inline size_t screen_ub_bytes(int64_t N, int KP) {
+  return (size_t)round_up(N, kScreenRows) * KP * sizeof(unsigned short);
 }
 
 // Stored log-joint of the full model: per (32-row tile, component) 32 floats, rows
@@ -213,8 +214,12 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   p.keep_lj = p.need && p.DP > 128 && !p.wide && full_lj_bytes(N, p.KP) <= kMaxLjBytes;
   p.autolj = p.need && auto_lj && flj_applies(p.DP) && N > 0 && K <= kProbeMaxKB &&
              full_lj_bytes(N, p.KP) <= kMaxLjBytes;
-  p.screen = p.autolj && K >= kScreenMinK && cdiv(N, 32) * K * p.NMB >= kScreenMinWork &&
-             screen_region_bytes(N, p.KP) <= kMaxLjBytes;
+  p.screen_cap = 0;
+  if (p.autolj && K >= kScreenMinK && cdiv(N, 32) * K * p.NMB >= kScreenMinWork &&
+      full_lj_bytes(N, p.KP) > screen_ub_bytes(N, p.KP))
+    p.screen_cap = (int)std::min<size_t>(
+        65535, (full_lj_bytes(N, p.KP) - screen_ub_bytes(N, p.KP)) / sizeof(double) / (size_t)cdiv(N, 32));
+  p.screen = p.screen_cap >= 4 * p.KP;   // an eighth of a tile's pairs
   p.nprobe = p.autolj ? (int)std::min<int64_t>(kProbeTiles, cdiv(N, 32)) : 0;
   // A list entry holds the component in 16 bits (the LDS limit keeps K far below that).
   p.needmode = !p.need ? kNeedRunMax
@@ -285,9 +290,7 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   p.off_part_mu = off;  off = align256(off + (size_t)p.npart * p.KP * p.DP * sizeof(float));
   p.off_part_nk = off;  off = align256(off + (size_t)p.npart * p.KP * sizeof(float));
   p.off_lj = off;
-  // The screened pass 1's bounds and then its fp64 log-joint take the same bytes.
-  if (p.lj || p.keep_lj || p.autolj)
-    off = align256(off + std::max(full_lj_bytes(N, p.KP), p.screen ? screen_region_bytes(N, p.KP) : (size_t)0));
+  if (p.lj || p.keep_lj || p.autolj) off = align256(off + full_lj_bytes(N, p.KP));
   // Need masks: one word per (32-row tile of the pass-1 grid, component).
   p.grid1 = 0;
   p.off_need = off;
@@ -302,8 +305,7 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   }
   p.off_probe = off;
   if (p.autolj) off = align256(off + probe_bytes() + (size_t)p.nprobe * p.KP * 32 * sizeof(float));
-  p.off_sc = off;
-  if (p.screen) off = align256(off + (size_t)p.KP * (p.DP + kScreenConsts) * sizeof(float));
+  p.off_sc = p.off_part_sig;   // read by pass 1 only; pass 2 writes the partials
   p.total = off;
   return p;
 }
@@ -459,6 +461,13 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
 }
 
 
+// The branch, the default one where a screened call found a tile with more needed pairs
+// than its pool holds (full_screen).
+__device__ __forceinline__ int full_mode(const ProbeSel& p) {
+  const int m = probe_mode(p);
+  return m == kProbeScreen && *p.over != 0u ? kProbeDefault : m;
+}
+
 // What pass 1 leaves for pass 2 besides logZ2.
 constexpr int kLjmStore = 1;   // the stored log-joint
 constexpr int kLjmNeed = 2;    // need masks only (the default plan)
@@ -490,7 +499,7 @@ void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
   constexpr bool MASKS = LJM == kLjmNeed && !(KEEP && flj_applies(DP));
   // FGMM_FLAG_STORE_LOGJOINT_AUTO launches both need-mask instances; the probe's
   // counts let the KEEP one (the stored branch) or the other run.
-  if (probe.count != nullptr && probe_mode(probe) != (KEEP ? kProbeStored : kProbeDefault)) return;
+  if (probe.count != nullptr && full_mode(probe) != (KEEP ? kProbeStored : kProbeDefault)) return;
   constexpr int NMB = DP / 32, NQ = DP / 16;
   constexpr int SMB = full_x6_smb(DP);            // coordinate blocks per stage
   constexpr int NST = NMB / SMB;                  // stages per component
@@ -761,7 +770,7 @@ __global__ __launch_bounds__(64 * kProbeWaves) void full_probe_ll(const float* _
 
 __global__ __launch_bounds__(256) void full_probe_count(int64_t N, int K, int KP, int ntile,
                                                         const float* __restrict__ lls,
-                                                        unsigned* __restrict__ count) {
+                                                        unsigned* __restrict__ count, unsigned* over) {
   __shared__ float mrow[8][32];
   __shared__ unsigned part[4];
   const int s = blockIdx.x;
@@ -785,6 +794,8 @@ __global__ __launch_bounds__(256) void full_probe_count(int64_t N, int K, int KP
   if (lane == 0) part[wave] = need;
   __syncthreads();
   if (tid == 0) count[s] = part[0] + part[1] + part[2] + part[3];
+  // full_screen's flag takes the first word of tile 0's log-joints, read above.
+  if (s == 0 && tid == 0) *over = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -1096,11 +1107,12 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
                        const double* __restrict__ ck, int K, int KP, const double* __restrict__ rowstat,
                        const unsigned* __restrict__ need, int nslab, int64_t rows_per_slab,
                        float* __restrict__ part_sig, float* __restrict__ part_mu, float* __restrict__ part_nk,
-                       int dense, const float* __restrict__ lj, ProbeSel sel, double* __restrict__ llo) {
+                       int dense, const float* __restrict__ lj, ProbeSel sel, double* __restrict__ llo,
+                       const unsigned short* __restrict__ rank, int cap) {
   constexpr int NMB = DP / 32, NQ = DP / 16, NSB = NMB * (NMB + 1) / 2;
   constexpr int NGRP = gather_sig_groups(DP);
   if constexpr (LLO) {
-    if (probe_mode(sel) != kProbeScreen) return;
+    if (full_mode(sel) != kProbeScreen) return;
   } else {
     if (probe_selects(sel)) return;   // the stored branch's full_accum_ljt takes the call
   }
@@ -1255,7 +1267,10 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       maha += __shfl_xor(maha, 32);
       const double ll = e_l[DP] - hl * maha;
       if constexpr (LLO) {
-        if (g == 0 && e >= 0) llo[(r_begin + e) * KP + k] = ll;
+        if (g == 0 && e >= 0) {
+          const int64_t row = r_begin + e;
+          llo[(row >> 5) * cap + rank[((row >> 6) * KP + k) * 64 + (row & 63)]] = ll;
+        }
         if (!PREFETCH) cnt_next = take(en);
         e = en;
         cnt = cnt_next;
@@ -1619,7 +1634,8 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // two half-waves trade their partial sums so that each lane owns one row of a tile pair.
 // Upper bounds go to `ub` as bf16 ([workgroup][wave][tile pair][component][64 rows], 128
 // bytes a store); once the row's largest lower bound is final each lane reads its own
-// back.  Bound: matrix steps and the squares' VALU, about equal.  The steps of the blocks
+// back, counts the needed pairs and leaves each its place in its tile's pool instead; a tile
+// with more than the pool holds sets `over`, and the exact pass 1 takes the call.  Bound: matrix steps and the squares' VALU, about equal.  The steps of the blocks
 // above L's diagonal (2 of 8 at D = 64) are left out: a component with a nonzero there
 // has A = infinity, so nothing of it is screened.
 // N=250K K=256 D=64, clustered: the drop-in call 2.670 -> 0.655 ms (0.705 with all eight
@@ -1630,7 +1646,7 @@ template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads), amdgpu_waves_per_eu(2, 2)))
 void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ l3,
                  const float* __restrict__ sc, int K, int KP, unsigned short* __restrict__ ub,
-                 unsigned* __restrict__ need, ProbeSel sel) {
+                 unsigned* __restrict__ need, int cap, unsigned* __restrict__ over, ProbeSel sel) {
   if (probe_mode(sel) != kProbeScreen) return;
   using SH = ScreenShape<DP>;
   constexpr int NMB = SH::NMB, NQ = SH::NQ, CPS = SH::CPS, SCF = SH::SCF, TPW = kScreenTpw;
@@ -1750,21 +1766,32 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
     if (tile * 32 >= N) break;
     const bool valid = (tile + g) * 32 + c < N;
     const float thr = M[j] - kLjNeedGap;
+    unsigned n = 0;   // needed pairs of the lane's tile so far
     for (int k0 = 0; k0 < K; k0 += 64) {
       unsigned w0 = 0u, w1 = 0u;
-#pragma unroll 8
-      for (int i = 0; i < 64; ++i) {
-        const int k = k0 + i < K ? k0 + i : K - 1;
-        const float R = bf16_bits_to_float(ubw[((int64_t)j * KP + k) * 64]);
-        const uint64_t m = __builtin_amdgcn_ballot_w64(valid && !(R < thr));
-        w0 = lane == i ? (unsigned)m : w0;
-        w1 = lane == i ? (unsigned)(m >> 32) : w1;
+      for (int i0 = 0; i0 < 64 && k0 + i0 < K; i0 += 8) {
+        unsigned short* p = ubw + ((int64_t)j * KP + k0 + i0) * 64;
+        float R[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) R[i] = bf16_bits_to_float(p[(k0 + i0 + i < K ? i : 0) * 64]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const bool mine = valid && k0 + i0 + i < K && !(R[i] < thr);
+          const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+          w0 = lane == i0 + i ? (unsigned)m : w0;
+          w1 = lane == i0 + i ? (unsigned)(m >> 32) : w1;
+          const unsigned mt = g ? (unsigned)(m >> 32) : (unsigned)m;
+          // The pair's place in the tile's pool, component by component.
+          if (mine) p[i * 64] = (unsigned short)(n + __popc(mt & ((1u << c) - 1u)));
+          n += __popc(mt);
+        }
       }
       if (k0 + lane < K) {
         need[tile * KP + k0 + lane] = w0;
         if ((tile + 1) * 32 < N) need[(tile + 1) * KP + k0 + lane] = w1;
       }
     }
+    if (n > (unsigned)cap) atomicOr(over, 1u);
   }
 }
 
@@ -1773,16 +1800,16 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
 // loads in flight.  Bound: latency.
 __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, const double* __restrict__ ll,
                                                      unsigned* __restrict__ need, double* __restrict__ rowstat,
-                                                     float* __restrict__ logZ, ProbeSel sel) {
-  if (probe_mode(sel) != kProbeScreen) return;
+                                                     float* __restrict__ logZ, int cap, ProbeSel sel) {
+  if (full_mode(sel) != kProbeScreen) return;
   const int lane = threadIdx.x & 63, c = lane & 31;
   const int64_t tile = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t row = tile * 32 + c;
   if (tile * 32 >= N) return;   // uniform over the wave
-  const double* lr = ll + (row < N ? row : N - 1) * KP;
+  const double* lt = ll + tile * cap;   // the tile's pool, component by component
   unsigned* nw = need + tile * KP;
   // f(component, this lane's row needs it, its log-joint) over the tile's nonzero words.
-  auto pairs = [&](unsigned w, int k0, auto f) {
+  auto pairs = [&](unsigned w, unsigned& at, auto f) {
     uint64_t bits = __builtin_amdgcn_ballot_w64(w != 0u);
     while (bits != 0) {
       int kk[8];
@@ -1795,7 +1822,8 @@ __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, c
         const unsigned word = kk[j] >= 0 ? (unsigned)__builtin_amdgcn_readlane((int)w, kk[j] & 63) : 0u;
         in[j] = (word >> c) & 1u;
         v[j] = 0.0;
-        if (in[j]) v[j] = lr[k0 + kk[j]];
+        if (in[j]) v[j] = lt[at + __popc(word & ((1u << c) - 1u))];
+        at += __popc(word);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -1805,9 +1833,10 @@ __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, c
   double mx = -INFINITY;
   float sm = 0.0f;
   int n = 0;
+  unsigned at = 0;
   for (int k0 = 0; k0 < K; k0 += 64) {
     const unsigned w = k0 + lane < K ? nw[k0 + lane] : 0u;
-    pairs(w, k0, [&](int, bool in, double v) {
+    pairs(w, at, [&](int, bool in, double v) {
       if (!in) return;
       const double mn = fmax(mx, v);
       const double ms = mn == -INFINITY ? 0.0 : mn;
@@ -1821,6 +1850,7 @@ __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, c
     rowstat[row] = lz2;
     if (logZ) logZ[row] = (float)(lz2 * kLn2);
   }
+  at = 0;
   // A row's only pair is needed.
   if (__builtin_amdgcn_ballot_w64(n > 1) == 0) return;
   const float zx = (float)lz2;
@@ -1828,7 +1858,7 @@ __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, c
   for (int k0 = 0; k0 < K; k0 += 64) {
     const unsigned w = k0 + lane < K ? nw[k0 + lane] : 0u;
     unsigned nwd = w;
-    pairs(w, k0, [&](int kk, bool in, double v) {
+    pairs(w, at, [&](int kk, bool in, double v) {
       const float R = bf16_bits_to_float(bf16_bits_up((float)v));
       const unsigned m = (unsigned)__builtin_amdgcn_ballot_w64(in && !(((R - zx) - zy) < -kLjNeedGap));
       if (lane == kk) nwd = m;
@@ -1852,7 +1882,8 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
   // The screened pass 1 up to an eighth of the sampled pairs (a quarter of the stored
   // branch's least, half of them).
   const int64_t min_pairs = probe ? probe_min_pairs(pl.N, pl.nprobe, (int)pl.K) : 0;
-  const ProbeSel psel = {probe, pl.nprobe, min_pairs, pl.screen && !dense ? min_pairs / 4 : (int64_t)-1};
+  unsigned* over = probe ? reinterpret_cast<unsigned*>(ws + pl.off_probe + probe_bytes()) : nullptr;
+  const ProbeSel psel = {probe, pl.nprobe, min_pairs, pl.screen && !dense ? min_pairs / 4 : (int64_t)-1, over};
   if (run1) {
     if constexpr (flj_applies(DP)) {
       if (pl.autolj) {
@@ -1862,7 +1893,14 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                            stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                            reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, pl.nprobe, lls);
         hipLaunchKernelGGL(full_probe_count, dim3((unsigned)pl.nprobe), dim3(256), 0, stream, pl.N, (int)pl.K, pl.KP,
-                           pl.nprobe, lls, probe);
+                           pl.nprobe, lls, probe, reinterpret_cast<unsigned*>(lls));
+      if (pl.screen && !dense) {
+        unsigned* need = reinterpret_cast<unsigned*>(ws + pl.off_need);
+        hipLaunchKernelGGL((full_screen<DP>), dim3((unsigned)cdiv(pl.N, kScreenRows)), dim3(kThreads), 0, stream, X,
+                           ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
+                           reinterpret_cast<const float*>(ws + pl.off_sc), (int)pl.K, pl.KP,
+                           reinterpret_cast<unsigned short*>(ws + pl.off_lj), need, pl.screen_cap, over, psel);
+      }
       }
     }
     const size_t lds1 = full_x6_lds_bytes(DP) + (pl.needmode == kNeedLists ? full_list_lds_bytes(DP, pl.KP) : 0);
@@ -1902,11 +1940,8 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
       }
       if (pl.screen && !dense) {
         unsigned* need = reinterpret_cast<unsigned*>(ws + pl.off_need);
-        double* ll = reinterpret_cast<double*>(ws + pl.off_lj);
-        hipLaunchKernelGGL((full_screen<DP>), dim3((unsigned)cdiv(pl.N, kScreenRows)), dim3(kThreads), 0, stream, X,
-                           ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
-                           reinterpret_cast<const float*>(ws + pl.off_sc), (int)pl.K, pl.KP,
-                           reinterpret_cast<unsigned short*>(ws + pl.off_lj), need, psel);
+        const unsigned short* ub = reinterpret_cast<const unsigned short*>(ws + pl.off_lj);
+        double* ll = reinterpret_cast<double*>(ws + pl.off_lj + screen_ub_bytes(pl.N, pl.KP));
         constexpr size_t ldsg = gather_lds_bytes<DP>();
         auto kll = &full_accum_gather<DP, 0, false, true>;
         e = set_lds(reinterpret_cast<const void*>(kll), ldsg);
@@ -1914,9 +1949,9 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
         hipLaunchKernelGGL(kll, dim3((unsigned)gather_grid(pl.nslab, (int)pl.K)), dim3(64 * kGatherWaves), ldsg,
                            stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                            reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat, need,
-                           pl.nslab, pl.rows_per_slab, nullptr, nullptr, nullptr, 0, nullptr, psel, ll);
+                           pl.nslab, pl.rows_per_slab, nullptr, nullptr, nullptr, 0, nullptr, psel, ll, ub, pl.screen_cap);
         hipLaunchKernelGGL(full_need_lse, dim3((unsigned)cdiv(pl.N, 128)), dim3(256), 0, stream, pl.N, (int)pl.K,
-                           pl.KP, ll, need, rowstat, logZ, psel);
+                           pl.KP, ll, need, rowstat, logZ, pl.screen_cap, psel);
       }
     }
   }
@@ -1940,7 +1975,7 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                              reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                              reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat,
                              reinterpret_cast<const unsigned*>(ws + pl.off_need), pl.nslab, pl.rows_per_slab,
-                             psig, pmu, pnk, dense ? 1 : 0, lj, psel, nullptr);
+                             psig, pmu, pnk, dense ? 1 : 0, lj, psel, nullptr, nullptr, 0);
         }
         return hipSuccess;
       };

@@ -66,3 +66,6 @@ def test_rows_of_several_and_special_components(gpu_device):
     inp["X"][7] = inp["X"][10_000] = 1e18   # finite; the screening's squares are not all
     print("full screen huge rows", flush=True)
     same(call(inp, gpu_device, "auto"), call(inp, gpu_device, False), "huge rows")
+    inp["X"][64:96] = math.nan   # a tile of which every pair is needed: the exact pass 1
+    print("full screen full tile", flush=True)
+    same(call(inp, gpu_device, "auto"), call(inp, gpu_device, False), "full tile")
