@@ -62,13 +62,7 @@ WORKLOADS = {
 # (FETCH_SIZE KiB, WRITE_SIZE KiB); the commands and tables are in profiles/.
 TRAFFIC_KIB = {
     # (workload, plan, precision): {kernel: (fetch KiB, write KiB)}; "phase1" names pass 1's
-    # The drop-in's mode (store_log_joint="auto"): on this clustered data the probe keeps
-    # the default plan, and iso_accum_ljt returns at once.
-    ("iso_n1m_k1024_d128", "default", "fp32"): {
-        "phase1": "iso_lse_pipe<128, 1>",
-        "iso_prep": (311, 1_104), "iso_store_probe<128>": (2_680, 2), "iso_lse_pipe<128, 1>": (310_281, 24_414),
-        "iso_accum_ljt<128>": (18, 0), "iso_accum_gather<128>": (268_569, 33_280),
-        "iso_accum_tiles2<128>": (16, 0), "iso_reduce": (20_842, 664)},
+    # The screened calls (clustered data, SCREENED) are not listed: their pass 1 is several kernels.
     # The reference's N(0, I) data: the probe selects the stored branch (pass 1 writes the
     # log-joint, the X parts and the logZ pairs; iso_accum_ljt reads them back).
     ("iso_ref_n1m_k1024_d128", "default", "fp32"): {
@@ -76,18 +70,6 @@ TRAFFIC_KIB = {
         "iso_prep": (310, 1_104), "iso_store_probe<128>": (2_679, 2),
         "iso_lse_pipe<128, 1>": (316_772, 4_534_764), "iso_accum_ljt<128>": (2_289_322, 33_280),
         "iso_accum_gather<128>": (22, 0), "iso_accum_tiles2<128>": (13, 0), "iso_reduce": (20_835, 664)},
-    ("diag_n1m_k1024_d96", "default", "fp32"): {
-        "phase1": "diag_lse_x6<96, 2, 0>",
-        "diag_x6_prep": (457, 1_552), "diag_lse_x6<96, 2, 0>": (193_991, 19_532),
-        "diag_accum_gather<96>": (207_844, 49_408), "diag_reduce": (25_823, 780)},
-    # The drop-in's mode: on this clustered data the probe keeps the default plan, and
-    # the stored branch's pass-1 instance and full_accum_ljt return at once.
-    ("full_n250k_k256_d64", "default", "fp32"): {
-        "phase1": "full_lse_x6<64, 2, 0, 2>",
-        "full_x6_prep": (2_134, 8_328), "full_probe_ll<64>": (5_285, 2_048), "full_probe_count": (1_045, 2),
-        "full_lse_x6<64, 2, 0, 2>": (177_976, 67_765), "full_lse_x6<64, 2, 1, 0>": (17, 0),
-        "full_accum_ljt<64>": (23, 0), "full_accum_gather<64, 0, 0>": (68_174, 25_150),
-        "full_reduce_sig": (12_328, 4_096), "full_reduce": (286, 65)},
     # N(0, I) data: the probe selects the stored branch.
     ("full_ref_n250k_k256_d64", "default", "fp32"): {
         "phase1": "full_lse_x6<64, 2, 1, 0>",
@@ -179,6 +161,19 @@ def pass1_executed(kind, N, K, D, precision, stored):
         return per * float(N) * K, "bf16", PEAK_BF16_MFMA_TFLOPS
     per = {"iso": 14 * DP, "diag": 28 * DP, "full": 14 * DP * DP}[kind]
     return per * float(N) * K, "bf16", PEAK_BF16_MFMA_TFLOPS
+
+
+# Clustered workloads whose drop-in call takes the screened pass 1.
+SCREENED = ("iso_n1m_k1024_d128", "diag_n1m_k1024_d96", "full_n250k_k256_d64")
+
+
+def screen_executed(kind, N, K, D):
+    """bf16 matrix flops of the screening (one step per product, the constants' chunk, and
+    for full only the blocks on and below the factor's diagonal).  The exact steps for the
+    few pairs it leaves are not counted."""
+    DP = padded_dim(kind, D)
+    per = {"iso": 2 * (DP + 16), "diag": 2 * (2 * DP + 16), "full": sum(64 * (DP - d) for d in range(0, DP, 32))}[kind]
+    return per * float(N) * K
 
 
 def iso_need_pairs(inp, logZ, chunk=65536):
@@ -368,7 +363,8 @@ def time_dropin(kind, inp, steps, warmup, stream):
 KERNELS = {
     # (kind, plan) -> (pass-1 kernel, pass-2 kernel)
     ("iso", "default"): ("iso_lse_pipe (need masks)", "iso_accum_gather / iso_accum_tiles (by the needed-pair count)"),
-    ("iso", "auto"): ("iso_store_probe, iso_lse_pipe (need masks; stores the log-joint where the probe selects it)",
+    ("iso", "auto"): ("iso_store_probe, then as the probe selects screen_pairs and iso_lse_pipe on the rows it lists, "
+                      "or iso_lse_pipe (need masks, or storing the log-joint)",
                       "iso_accum_ljt where the probe selected the stored branch, else iso_accum_gather / "
                       "iso_accum_tiles2 (by the needed-pair count)"),
     ("iso", "default_wide"): ("iso_lse_ctile (need masks)", "iso_accum_drange"),
@@ -376,15 +372,15 @@ KERNELS = {
                         "iso_accum_sparse / iso_accum_ljt (by the needed-pair count)"),
     ("iso", "stored_wide"): ("iso_lse_ctile (stores the log-joint)", "iso_accum_lj"),
     ("diag", "default"): ("diag_lse_x6 (need masks)", "diag_accum_gather"),
-    ("diag", "auto"): ("diag_store_probe, diag_lse_x6 (need masks; the instance that also stores the "
-                       "log-joint, the rows' feature parts and logZ pairs runs where the probe selects it)",
+    ("diag", "auto"): ("diag_store_probe, then as the probe selects screen_pairs and diag_lse_x6 on the rows it lists, "
+                       "or diag_lse_x6 (need masks, or storing the log-joint, feature parts and logZ pairs)",
                        "diag_accum_ljt where the probe selected the stored branch, else diag_accum_gather"),
     ("diag", "default_wide"): ("diag_lse_ctile (need masks)", "diag_accum_drange"),
     ("diag", "stored"): ("diag_lse_x6 (stores the log-joint)", "diag_accum_sparse / diag_accum_lj2"),
     ("diag", "stored_wide"): ("diag_lse_ctile (stores the log-joint)", "diag_accum_lj"),
     ("full", "default"): ("full_lse_x6 (need masks)", "full_accum_gather"),
-    ("full", "auto"): ("full_probe_ll, full_probe_count, full_lse_x6 (need masks; the instance that also keeps the "
-                       "log-joint runs where the probe selects it)",
+    ("full", "auto"): ("full_probe_ll, full_probe_count, then as the probe selects full_screen, the gathered "
+                       "log-joint and full_need_lse, or full_lse_x6 (need masks, or keeping the log-joint)",
                        "full_accum_ljt where the probe selected the stored branch, else full_accum_gather"),
     ("full", "stored"): ("full_lse_x6 (stores the log-joint)", "full_accum"),
 }
@@ -459,6 +455,8 @@ def main_workload(args):
     (flop, f1, f2), alg_bytes = algorithmic(kind, N, K, D)
     k1, k2 = kernel_names(kind, D, args.precision, mode)
     ex1, unit1, peak1 = pass1_executed(kind, N, K, D, args.precision, args.store_log_joint)
+    if mode == "auto" and workload in SCREENED:
+        ex1 = screen_executed(kind, N, K, D)
     phases = {
         "phase1": {"kernel": k1 + " + prologue", "ms": p1, "fp32_algorithmic_flop": f1,
                    "fp32_equivalent_tflops": f1 / (p1 * 1e-3) / 1e12,
