@@ -1638,8 +1638,8 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // with more than the pool holds sets `over`, and the exact pass 1 takes the call.  Bound: matrix steps and the squares' VALU, about equal.  The steps of the blocks
 // above L's diagonal (2 of 8 at D = 64) are left out: a component with a nonzero there
 // has A = infinity, so nothing of it is screened.
-// N=250K K=256 D=64, clustered: the drop-in call 2.670 -> 0.655 ms (0.705 with all eight
-// steps; exact pass 1 2.45 ms;
+// N=250K K=256 D=64, clustered: the drop-in call 2.641 -> 0.618 ms (0.705 with all eight
+// steps and a log-joint of every pair; exact pass 1 2.45 ms;
 // traced: full_screen 0.565, the gathered log-joint 0.075, full_need_lse 0.020).
 // ---------------------------------------------------------------------------
 template <int DP>
