@@ -364,6 +364,8 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
   const int NQ = DP / 8, NC = DP / 8 + 1;   // NC: the screening's chunks (16 x, then 16 x^2, then constants)
   const float* mrow = mu + (valid ? comp : 0) * ldmu;
   const float* lrow = lss + (valid ? comp : 0) * ldlss;
+  const double lp = valid ? (double)lpi[comp] : 0.0;
+  const BlockLive live(valid && lp != -INFINITY);
   double osum = 0.0, qs = 0.0, lsum = 0.0, w2 = 0.0, v2 = 0.0;
   for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
     const int q1 = q0 + kPrepChunks < NQ ? q0 + kPrepChunks : NQ;
@@ -403,8 +405,8 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
         // The screening's lanes take 8 dimensions: chunk q is half of its chunk q / 2.
         unsigned* po = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
         unsigned* pw = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + NQ / 2 + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
-        *reinterpret_cast<uint2*>(po) = uint2{bf16_pair(f32x2{fv.x, fv.y}), bf16_pair(f32x2{fv.z, fv.w})};
-        *reinterpret_cast<uint2*>(pw) = uint2{bf16_pair(f32x2{fw.x, fw.y}), bf16_pair(f32x2{fw.z, fw.w})};
+        *reinterpret_cast<uint2*>(po) = live.copy(uint2{bf16_pair(f32x2{fv.x, fv.y}), bf16_pair(f32x2{fv.z, fv.w})});
+        *reinterpret_cast<uint2*>(pw) = live.copy(uint2{bf16_pair(f32x2{fw.x, fw.y}), bf16_pair(f32x2{fw.z, fw.w})});
       }
       f32x4 ov = zero4();
       if (g == 0) ov.x = -(float)o;
@@ -441,12 +443,14 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
   double C0 = -INFINITY;   // C'_k without the centring offsets
   double eW = 0.0, eV = 0.0, eC = 0.0;   // the component's part of the screening's error bound
   if (g == 0) {
-    if (valid) C0 = ((double)lpi[comp] - 0.5 * ((double)D * kLog2Pi + lsum)) * kLog2e - qs;
+    if (valid) C0 = (lp - 0.5 * ((double)D * kLog2Pi + lsum)) * kLog2e - qs;
     sC[c] = valid ? C0 + osum : C0;
     if (valid) {
       eW = sqrt(w2);
       eV = sqrt(v2);
-      eC = C0 == -INFINITY ? 0.0 : fabs(C0);
+      eC = fabs(C0);
+      if (lp == -INFINITY && C0 == -INFINITY && eW < 1e30 && eV < 1e30)
+        eW = eV = eC = 0.0;   // weighs nothing: not in the screening's operands
       // A component whose constants are not ordinary numbers gets no finite bound: every
       // row then needs its block, and the exact passes see it.
       if (!(eW < 1e30) || !(eV < 1e30) || !(eC < 1e30)) eC = INFINITY;
@@ -455,9 +459,8 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
   if (sc_op) {
     // The constants' chunk: C in three parts against screen_pairs' ones (second half).
-    const double C = __shfl(C0, c);
     f32x4 lo = zero4();
-    lo.x = !valid || C == -INFINITY ? -1e30f : (float)C;
+    lo.x = (float)__shfl(C0, c);
     bf16x8 sp[3], a;
     split3_bf16(lo, zero4(), sp);
 #pragma unroll
@@ -467,7 +470,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
       a[1] = sp[1][0];
       a[2] = sp[2][0];
     }
-    sc_op[((int64_t)kb * NC + NC - 1) * 64 + lane] = a;
+    sc_op[((int64_t)kb * NC + NC - 1) * 64 + lane] = live.constants(a, g);
 #pragma unroll
     for (int o = 16; o >= 1; o >>= 1) {
       eW = fmax(eW, __shfl_xor(eW, o));

@@ -388,6 +388,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
   const double l = valid ? (double)lss[comp] : 0.0, lp = valid ? (double)lpi[comp] : 0.0;
   const double b = valid ? 0.5 * exp(-l) * kLog2e : 0.0;
   const float w2 = (float)(2.0 * b);
+  const BlockLive live(valid && lp != -INFINITY);
   double musq = 0.0, osum = 0.0;
   for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
     // Three-way bf16 splits for the split-bf16 contraction, mu3[kb][q][s][lane] = split s
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
       split3_bf16(lo, hi, sp);
 #pragma unroll
       for (int t = 0; t < 3; ++t) mu3[(((int64_t)kb * NQ + q) * 4 + t) * 64 + lane] = sp[t];
-      if (sc_op) sc_op[((int64_t)kb * (NQ + 1) + q) * 64 + lane] = to_bf16x8(lo * w2, hi * w2);
+      if (sc_op) sc_op[((int64_t)kb * (NQ + 1) + q) * 64 + lane] = live.copy(to_bf16x8(lo * w2, hi * w2));
       f32x4 olo = zero4();
       if (g == 0) olo.x = -(float)o;
       bf16x8 so[3];
@@ -459,7 +460,9 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
     if (valid) {
       eW = 2.0 * b * sqrt(musq);
       eB = b;
-      eC = C == -INFINITY ? 0.0 : fabs(C);
+      eC = fabs(C);
+      if (lp == -INFINITY && C == -INFINITY && eW < 1e30 && eB < 1e30)
+        eW = eB = eC = 0.0;   // weighs nothing: not in the screening's operands
       // A component whose constants are not ordinary numbers gets no finite bound: every
       // row then needs its block, and the exact passes see it.
       if (!(eW < 1e30) || !(eB < 1e30) || !(eC < 1e30)) eC = INFINITY;
@@ -474,7 +477,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
     f32x4 lo = zero4();
     const double C = sL[c];
     lo.x = -(float)sB[c];
-    lo.y = !valid || C == -INFINITY ? -1e30f : (float)C;
+    lo.y = (float)C;
     bf16x8 sp[3], a;
     split3_bf16(lo, zero4(), sp);
 #pragma unroll
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
     } else {
       a[0] = sp[0][1]; a[1] = sp[1][1]; a[2] = sp[2][1];
     }
-    sc_op[((int64_t)kb * (NQ + 1) + NQ) * 64 + lane] = a;
+    sc_op[((int64_t)kb * (NQ + 1) + NQ) * 64 + lane] = live.constants(a, g);
 #pragma unroll
     for (int o = 16; o >= 1; o >>= 1) {
       eW = fmax(eW, __shfl_xor(eW, o));

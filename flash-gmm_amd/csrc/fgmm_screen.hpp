@@ -63,6 +63,40 @@ __device__ __forceinline__ void mark_alive(unsigned* __restrict__ alive, int kb,
   if ((threadIdx.x & 63) == 0 && m != 0u) atomicOr(alive + kb, m);
 }
 
+// The components of a block that weigh something (log_pi > -inf, or NaN) in the screening's
+// operands, for the models' prologues (lane c of a half-wave is component c).  A component
+// without weight, padding included, repeats the block's first one with weight, so that it
+// does not change the row's block maximum; a block of such components only gets the
+// constant -inf: it raises no row's lower bound and gets a bit only where no block has one.
+// (A finite constant in their place wins once a row's log-joints are all below it.)
+struct BlockLive {
+  unsigned mask;
+  int src;   // the lane to copy from
+  __device__ explicit BlockLive(bool live) {
+    const int lane = threadIdx.x & 63;
+    mask = (unsigned)__builtin_amdgcn_ballot_w64(live);   // the half-waves agree
+    src = live || mask == 0u ? lane : (lane & 32) + __builtin_ctz(mask);
+  }
+  __device__ __forceinline__ uint2 copy(uint2 v) const {
+    if (mask == ~0u) return v;   // uniform
+    return make_uint2(__shfl(v.x, src), __shfl(v.y, src));
+  }
+  __device__ __forceinline__ bf16x8 copy(const bf16x8& a) const {
+    uint4 w = __builtin_bit_cast(uint4, a);
+    const uint2 lo = copy(make_uint2(w.x, w.y)), hi = copy(make_uint2(w.z, w.w));
+    return __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+  }
+  // The same for the constants' chunk, whose second half (g == 1) starts with the constant
+  // against the row operand's ones.
+  __device__ __forceinline__ bf16x8 constants(bf16x8 a, int g) const {
+    if (mask != 0u) return copy(a);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = (__bf16)0.0f;
+    if (g == 1) a[0] = (__bf16)(-INFINITY);
+    return a;
+  }
+};
+
 // How a call's passes run.  The probe's last workgroup sums its counts and writes the
 // choice as one word, which every later kernel of the call reads with one scalar load
 // (each summing the counts for itself cost 0.5 us a kernel).

@@ -1,0 +1,69 @@
+"""The screened pass 1 over the range of its inputs' values: logZ bit for bit the dense run's
+(the unscreened exact passes), the sums per component to 1e-5."""
+
+import math
+
+import pytest
+import torch
+
+from flash_gmm import data, diag_estep_into, iso_estep_into
+from parity import assert_dense_agrees
+
+pytestmark = pytest.mark.gpu
+KEYS = ("X", "mu", "log_sigma_sq", "log_pi")
+
+
+def call(model, inp, dev, **kw):
+    args = [inp[k].to(dev) for k in KEYS]
+    N, D = args[0].shape
+    K = args[1].shape[0]
+    out = [torch.full((N,), math.nan, device=dev), torch.empty(K, device=dev), torch.empty(K, D, device=dev),
+           torch.empty(K, device=dev) if model == "iso" else torch.empty(K, D, device=dev)]
+    (iso_estep_into if model == "iso" else diag_estep_into)(*args, *out, **kw)
+    torch.cuda.synchronize()
+    return out
+
+
+def check(model, inp, dev, what):
+    print(what, flush=True)
+    got, dense = call(model, inp, dev), call(model, inp, dev, dense=True)
+    bad = (got[0] != dense[0]).nonzero().flatten()
+    assert bad.numel() == 0, f"{what}: logZ of rows {bad[:8].tolist()}: {got[0][bad[:8]]} not {dense[0][bad[:8]]}"
+    assert_dense_agrees(got[:2], dense[:2], bitwise=False)
+    for u, v in zip(got[2:], dense[2:]):
+        u, v = u.double().reshape(u.shape[0], -1), v.double().reshape(v.shape[0], -1)
+        top = v.abs().max(dim=1).values
+        assert bool(((u - v).abs().max(dim=1).values <= 1e-5 * top).all()), what
+
+
+# A last block of 12 and of 8 components (the second with scattered zero weights too), and
+# whole blocks of which one has no weight.
+@pytest.mark.parametrize("N,K,D", [(400_031, 300, 64), (63_009, 1000, 128), (63_009, 1024, 128)])
+def test_iso_rows_below_any_sentinel(N, K, D, gpu_device):
+    """Finite rows whose every log-joint is below -1e28, beside components that weigh nothing
+    (log_pi = -inf, or the padding of the last block)."""
+    inp = data.iso_clustered(N, K, D, seed=K % 11)
+    if K == 1024:
+        inp["log_pi"][64:96] = -math.inf
+    elif K == 1000:
+        inp["log_pi"][5::37] = -math.inf
+    for i, v in enumerate((1e14, 2e15, -2e15, 1e17, -9.22e18)):
+        inp["X"][1000 * i + 17, 3 * i] = v
+    check("iso", inp, gpu_device, f"iso range N={N} K={K} D={D}")
+
+
+@pytest.mark.parametrize("N,K,D", [(42_017, 1000, 96), (42_017, 1024, 96)])
+def test_diag_rows_below_any_sentinel(N, K, D, gpu_device):
+    """Data in units of 1e-10 with outliers, beside components that weigh nothing."""
+    inp = data.diag_clustered(N, K, D, seed=K % 11)
+    if K == 1024:
+        inp["log_pi"][64:96] = -math.inf
+    elif K == 1000:
+        inp["log_pi"][5::37] = -math.inf
+    unit = 1e-10
+    inp["X"] *= unit
+    inp["mu"] *= unit
+    inp["log_sigma_sq"] += 2.0 * math.log(unit)
+    for i, v in enumerate((1e3, 1e5, -1e6, 1e7, -1e8)):
+        inp["X"][1000 * i + 17, 3 * i] = v
+    check("diag", inp, gpu_device, f"diag range N={N} K={K} D={D}")
