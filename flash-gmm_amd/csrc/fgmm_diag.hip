@@ -871,7 +871,7 @@ __global__ __launch_bounds__(64 * kProbeWaves) void diag_store_probe(const float
     xs += sq[(c * (V4 + 1) + v) * 2];
     xq += sq[(c * (V4 + 1) + v) * 2 + 1];
   }
-  const float nx = sqrtf(xs), ny = sqrtf(xq);
+  const float nx = sqrtf(xs), ny = squares_norm(xs, xq);
   __syncthreads();   // the rows are read: rerr may be written
   const bf16x8 ones = x6c_ones(lane);
   for (int kb = wave; kb < KB; kb += kProbeWaves) {

@@ -63,6 +63,11 @@ __device__ __forceinline__ void mark_alive(unsigned* __restrict__ alive, int kb,
   if ((threadIdx.x & 63) == 0 && m != 0u) atomicOr(alive + kb, m);
 }
 
+// The norm of the vector of squares, sqrt(sum x^4), from the fp32 sums xs = ||x||^2 and xq =
+// sum x^4.  Where fourth powers may have underflowed it is bounded by xs; what xs loses
+// itself (x^2 below 2^-126) is under 2^-19 of log-joint for weights up to 1e30.
+__device__ __forceinline__ float squares_norm(float xs, float xq) { return xq < 0x1p-100f ? xs : sqrtf(xq); }
+
 // The components of a block that weigh something (log_pi > -inf, or NaN) in the screening's
 // operands, for the models' prologues (lane c of a half-wave is component c).  A component
 // without weight, padding included, repeats the block's first one with weight, so that it
@@ -216,7 +221,7 @@ __device__ __forceinline__ void probe_finish(const float* rmax, const float* rer
 // splits), a row's block maximum is a maximum of accumulators, and per block (the models'
 // prologues form sc_e)
 //   |a_nk - ll2_nk| <= E = sc_e.x ||x|| + sc_e.y s + sc_e.z,
-// s = ||x||^2 (iso) or the norm of the vector of squares (diag): each operand is rounded
+// s = ||x||^2 (iso) or the norm of the vector of squares (diag, squares_norm): each operand is rounded
 // by at most 2^-9 of itself, so the products err by 2^-8 ||x|| ||2 b mu|| (diag: 2^-8
 // (||x|| ||2 v|| + s ||w||); Cauchy-Schwarz; 0x1.06p-8 with the second-order and
 // accumulation terms), the constants' dropped split products and fp32 sums by under
@@ -369,7 +374,7 @@ void screen_pairs(const float* __restrict__ X, int64_t ldx, int64_t N, int D, co
       xb[t][NC - 1] = a;
     }
   }
-  const float nx = sqrtf(xs), ny = DIAG ? sqrtf(xq) : xs;
+  const float nx = sqrtf(xs), ny = DIAG ? squares_norm(xs, xq) : xs;
   lds_barrier();   // every wave has read its staging tile: the second stage and the bounds may overwrite it
 
   uint2* const words_l = reinterpret_cast<uint2*>(ub_l - lane);   // 32 blocks' words take 4 blocks' bounds

@@ -67,3 +67,21 @@ def test_diag_rows_below_any_sentinel(N, K, D, gpu_device):
     for i, v in enumerate((1e3, 1e5, -1e6, 1e7, -1e8)):
         inp["X"][1000 * i + 17, 3 * i] = v
     check("diag", inp, gpu_device, f"diag range N={N} K={K} D={D}")
+
+
+@pytest.mark.parametrize("unit", [1e-14, 1e-12, 1.0])
+def test_diag_squares_of_squares_that_underflow(unit, gpu_device):
+    """Small units: the fourth powers of the rows' elements are 0 in float32.  Half of the
+    components have one variance each, whose rounding to bf16 adds up over the dimensions,
+    and a tenth of the rows is far out, nearest to those."""
+    N, K, D = 42_017, 1024, 96
+    inp = data.diag_clustered(N, K // 2, D, seed=3)
+    g = torch.Generator().manual_seed(3)
+    inp["mu"] = torch.cat([inp["mu"], 6.0 * torch.randn(K // 2, D, generator=g)])
+    inp["log_sigma_sq"] = torch.cat([inp["log_sigma_sq"], (0.6 + 0.8 * torch.rand(K // 2, 1, generator=g)).expand(-1, D)])
+    inp["log_pi"] = torch.full((K,), -math.log(K))
+    inp["X"][::10] *= 50.0
+    inp["X"] *= unit
+    inp["mu"] *= unit
+    inp["log_sigma_sq"] += 2.0 * math.log(unit)
+    check("diag", inp, gpu_device, f"diag unit {unit}")
