@@ -348,7 +348,9 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
                                                    unsigned* __restrict__ ljcount, bf16x8* __restrict__ sc_op,
                                                    float4* __restrict__ sc_e, unsigned* __restrict__ list_count,
                                                    unsigned* __restrict__ state) {
-  __shared__ double sC[32], sO[kPrepChunks][32], sL[kPrepChunks][32], sW[kPrepChunks][32], sV[kPrepChunks][32];
+  __shared__ double sC[32], sO[kPrepChunks][32], sL[kPrepChunks][32];
+  // The screening's operands: w's and v's squared rounding errors and squares.
+  __shared__ double sS[4][kPrepChunks][32];
   const int kb = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -366,7 +368,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
   const float* lrow = lss + (valid ? comp : 0) * ldlss;
   const double lp = valid ? (double)lpi[comp] : 0.0;
   const BlockLive live(valid && lp != -INFINITY);
-  double osum = 0.0, qs = 0.0, lsum = 0.0, w2 = 0.0, v2 = 0.0;
+  double osum = 0.0, qs = 0.0, lsum = 0.0, sums[4] = {0.0, 0.0, 0.0, 0.0};
   for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
     const int q1 = q0 + kPrepChunks < NQ ? q0 + kPrepChunks : NQ;
     for (int q = q0 + wave; q < q1; q += kPrepWaves) {
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
         fl[e] = lrow[d];
       }
       f32x4 fw = zero4(), fv = zero4();
-      double o = 0.0, ls = 0.0, sw = 0.0, sv = 0.0;
+      double o = 0.0, ls = 0.0, dw[4], dv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const bool in = valid && d0 + e < D;
@@ -387,15 +389,13 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
         const double w = in ? 0.5 * exp(-l) * kLog2e : 0.0, v = 2.0 * m * w;
         o = fma(m * m, w, o);
         ls += l;
-        sw = fma(w, w, sw);
-        sv = fma(v, v, sv);
+        dw[e] = -w;
+        dv[e] = v;
         fw[e] = (float)(-w);
         fv[e] = (float)v;
       }
       o += __shfl_xor(o, 32);   // both halves' dimensions (the sum commutes)
       ls += __shfl_xor(ls, 32);
-      sw += __shfl_xor(sw, 32);
-      sv += __shfl_xor(sv, 32);
       bf16x8 s[3];
       split3_bf16(fw, fv, s);
       bf16x8* dst = mu3 + ((int64_t)kb * NQ + q) * 4 * 64 + lane;
@@ -405,8 +405,25 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
         // The screening's lanes take 8 dimensions: chunk q is half of its chunk q / 2.
         unsigned* po = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
         unsigned* pw = reinterpret_cast<unsigned*>(sc_op + ((int64_t)kb * NC + NQ / 2 + q / 2) * 64 + 32 * (q & 1) + c) + 2 * g;
-        *reinterpret_cast<uint2*>(po) = live.copy(uint2{bf16_pair(f32x2{fv.x, fv.y}), bf16_pair(f32x2{fv.z, fv.w})});
-        *reinterpret_cast<uint2*>(pw) = live.copy(uint2{bf16_pair(f32x2{fw.x, fw.y}), bf16_pair(f32x2{fw.z, fw.w})});
+        const uint2 hv = {bf16_pair(f32x2{fv.x, fv.y}), bf16_pair(f32x2{fv.z, fv.w})};
+        const uint2 hw = {bf16_pair(f32x2{fw.x, fw.y}), bf16_pair(f32x2{fw.z, fw.w})};
+        *reinterpret_cast<uint2*>(po) = live.copy(hv);
+        *reinterpret_cast<uint2*>(pw) = live.copy(hw);
+        double p[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x2 pv = bf16_pair_widen(e < 2 ? hv.x : hv.y), pw2 = bf16_pair_widen(e < 2 ? hw.x : hw.y);
+          const double bv = (double)((e & 1) ? pv.y : pv.x), bw = (double)((e & 1) ? pw2.y : pw2.x);
+          p[0] = fma(dw[e] - bw, dw[e] - bw, p[0]);
+          p[1] = fma(bw, bw, p[1]);
+          p[2] = fma(dv[e] - bv, dv[e] - bv, p[2]);
+          p[3] = fma(bv, bv, p[3]);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          p[t] += __shfl_xor(p[t], 32);
+          if (g == 0) sS[t][q - q0][c] = p[t];
+        }
       }
       f32x4 ov = zero4();
       if (g == 0) ov.x = -(float)o;
@@ -422,8 +439,6 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
       if (g == 0) {
         sO[q - q0][c] = o;
         sL[q - q0][c] = ls;
-        sW[q - q0][c] = sw;
-        sV[q - q0][c] = sv;
       }
     }
     __syncthreads();
@@ -433,8 +448,10 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
         qs += o;
         osum += (double)(float)o;
         lsum += sL[q][c];
-        w2 += sW[q][c];
-        v2 += sV[q][c];
+        if (sc_op) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) sums[t] += sS[t][q][c];
+        }
       }
     }
     if (q1 < NQ) __syncthreads();
@@ -446,14 +463,14 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
     if (valid) C0 = (lp - 0.5 * ((double)D * kLog2Pi + lsum)) * kLog2e - qs;
     sC[c] = valid ? C0 + osum : C0;
     if (valid) {
-      eW = sqrt(w2);
-      eV = sqrt(v2);
+      eW = screen_weight_error(sums[0], sums[1]);
+      eV = screen_weight_error(sums[2], sums[3]);
       eC = fabs(C0);
       if (lp == -INFINITY && C0 == -INFINITY && eW < 1e30 && eV < 1e30)
         eW = eV = eC = 0.0;   // weighs nothing: not in the screening's operands
       // A component whose constants are not ordinary numbers gets no finite bound: every
       // row then needs its block, and the exact passes see it.
-      if (!(eW < 1e30) || !(eV < 1e30) || !(eC < 1e30)) eC = INFINITY;
+      if (!(sums[1] < 1e60) || !(sums[3] < 1e60) || !(eW < 1e30) || !(eV < 1e30) || !(eC < 1e30)) eC = INFINITY;
     }
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
@@ -478,7 +495,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void diag_x6_prep(const float* __r
       eC = fmax(eC, __shfl_xor(eC, o));
     }
     if (lane == 0)
-      sc_e[kb] = make_float4((float)(eV * 0x1.06p-8), (float)(eW * 0x1.06p-8), (float)(eC * 0x1p-14 + 1.0), 0.0f);
+      sc_e[kb] = make_float4((float)eV, (float)eW, (float)(eC * 0x1p-14 + 1.0), 0.0f);
   }
   if (lane < 32) {
     const int i = lane & 15, gg = lane >> 4;

@@ -371,6 +371,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
                                                float4* __restrict__ sc_e, unsigned* __restrict__ list_count,
                                                unsigned* __restrict__ state) {
   __shared__ double sC[32], sB[32], sL[32], sO[kPrepChunks][32];
+  __shared__ double sR[kPrepChunks][32], sH[kPrepChunks][32];   // the screening's operands: squared rounding errors, squares
   const int kb = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
   const double b = valid ? 0.5 * exp(-l) * kLog2e : 0.0;
   const float w2 = (float)(2.0 * b);
   const BlockLive live(valid && lp != -INFINITY);
-  double musq = 0.0, osum = 0.0;
+  double musq = 0.0, osum = 0.0, rsq = 0.0, hsq = 0.0;
   for (int q0 = 0; q0 < NQ; q0 += kPrepChunks) {
     // Three-way bf16 splits for the split-bf16 contraction, mu3[kb][q][s][lane] = split s
     // of mu[comp][16q + 8g .. 16q + 8g + 7] (s < 3), and slot 3 = the splits of the
@@ -419,7 +420,23 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
       split3_bf16(lo, hi, sp);
 #pragma unroll
       for (int t = 0; t < 3; ++t) mu3[(((int64_t)kb * NQ + q) * 4 + t) * 64 + lane] = sp[t];
-      if (sc_op) sc_op[((int64_t)kb * (NQ + 1) + q) * 64 + lane] = live.copy(to_bf16x8(lo * w2, hi * w2));
+      if (sc_op) {
+        const bf16x8 h = to_bf16x8(lo * w2, hi * w2);
+        sc_op[((int64_t)kb * (NQ + 1) + q) * 64 + lane] = live.copy(h);
+        double dr = 0.0, dh = 0.0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const double hv = (double)(float)h[e], rv = 2.0 * b * (double)(e < 4 ? lo[e & 3] : hi[e & 3]) - hv;
+          dr = fma(rv, rv, dr);
+          dh = fma(hv, hv, dh);
+        }
+        dr += __shfl_xor(dr, 32);
+        dh += __shfl_xor(dh, 32);
+        if (g == 0) {
+          sR[q - q0][c] = dr;
+          sH[q - q0][c] = dh;
+        }
+      }
       f32x4 olo = zero4();
       if (g == 0) olo.x = -(float)o;
       bf16x8 so[3];
@@ -440,12 +457,16 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
         const double o = sO[q - q0][c];
         musq += o;
         osum += (double)(float)o;
+        if (sc_op) {
+          rsq += sR[q - q0][c];
+          hsq += sH[q - q0][c];
+        }
       }
     }
     if (q1 < NQ) __syncthreads();
   }
   if (wave != 0) return;
-  double eW = 0.0, eB = 0.0, eC = 0.0;   // the component's part of the screening's error bound
+  double eW = 0.0, eB = 0.0, eC = 0.0;   // the component's part of the screening's error bound (screen_pairs)
   if (g == 0) {
     const double C = valid ? (lp - 0.5 * (double)D * (kLog2Pi + l)) * kLog2e - b * musq : -INFINITY;
     // The split-bf16 passes contract the centred cross term x.mu - sum_q o_q, so
@@ -458,14 +479,14 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
     // ||x - mu||^2 = ||x||^2 - 2 (x.mu - sum_q o_q) + (||mu||^2 - 2 sum_q o_q), the last term.
     kc_gat[comp] = make_double4(sC[c], b, musq - 2.0 * osum, 0.0);
     if (valid) {
-      eW = 2.0 * b * sqrt(musq);
+      eW = screen_weight_error(rsq, hsq);
       eB = b;
       eC = fabs(C);
       if (lp == -INFINITY && C == -INFINITY && eW < 1e30 && eB < 1e30)
         eW = eB = eC = 0.0;   // weighs nothing: not in the screening's operands
       // A component whose constants are not ordinary numbers gets no finite bound: every
       // row then needs its block, and the exact passes see it.
-      if (!(eW < 1e30) || !(eB < 1e30) || !(eC < 1e30)) eC = INFINITY;
+      if (!(hsq < 1e60) || !(eW < 1e30) || !(eB < 1e30) || !(eC < 1e30)) eC = INFINITY;
     }
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // one wave from here on
@@ -496,7 +517,7 @@ __global__ __launch_bounds__(64 * kPrepWaves) void iso_prep(const float* __restr
       eC = fmax(eC, __shfl_xor(eC, o));
     }
     if (lane == 0)
-      sc_e[kb] = make_float4((float)(eW * 0x1.06p-8), (float)(eB * 0x1p-14), (float)(eC * 0x1p-14 + 1.0), 0.0f);
+      sc_e[kb] = make_float4((float)eW, (float)(eB * 0x1p-14), (float)(eC * 0x1p-14 + 1.0), 0.0f);
   }
   // Constants in accumulator-register order: entry (g, i) is component acc_row(i, g).
   {

@@ -68,6 +68,12 @@ __device__ __forceinline__ void mark_alive(unsigned* __restrict__ alive, int kb,
 // itself (x^2 below 2^-126) is under 2^-19 of log-joint for weights up to 1e30.
 __device__ __forceinline__ float squares_norm(float xs, float xq) { return xq < 0x1p-100f ? xs : sqrtf(xq); }
 
+// The factor of the row's norm in the screening's error bound (screen_pairs): from an operand
+// row's sums of squares, of its rounding errors and of its rounded values.
+__device__ __forceinline__ double screen_weight_error(double err_sq, double rounded_sq) {
+  return sqrt(err_sq) + 0x1.06p-8 * sqrt(rounded_sq);
+}
+
 // The components of a block that weigh something (log_pi > -inf, or NaN) in the screening's
 // operands, for the models' prologues (lane c of a half-wave is component c).  A component
 // without weight, padding included, repeats the block's first one with weight, so that it
@@ -221,18 +227,20 @@ __device__ __forceinline__ void probe_finish(const float* rmax, const float* rer
 // splits), a row's block maximum is a maximum of accumulators, and per block (the models'
 // prologues form sc_e)
 //   |a_nk - ll2_nk| <= E = sc_e.x ||x|| + sc_e.y s + sc_e.z,
-// s = ||x||^2 (iso) or the norm of the vector of squares (diag, squares_norm): each operand is rounded
-// by at most 2^-9 of itself, so the products err by 2^-8 ||x|| ||2 b mu|| (diag: 2^-8
-// (||x|| ||2 v|| + s ||w||); Cauchy-Schwarz; 0x1.06p-8 with the second-order and
-// accumulation terms), the constants' dropped split products and fp32 sums by under
-// 2^-14 (b ||x||^2 + |C|).
+// s = ||x||^2 (iso) or the norm of the vector of squares (diag, squares_norm).  With w an
+// operand's row and h its rounding to bf16, |x.w - bf16(x).h| <= ||x|| ||w - h|| +
+// ||x - bf16(x)|| ||h||, the second of at most 2^-8 ||x|| ||h|| (8 significant bits), so
+// ||x||'s factor is ||w - h|| + 0x1.06p-8 ||h|| (screen_weight_error; 0x1.06 for the
+// second-order terms and the sum's roundings), s's likewise (diag); the constants' dropped
+// split products and their fp32 sums err by under 2^-14 (b ||x||^2 + |C|).  (Bounding
+// ||w - h|| by 2^-8 ||w|| too lists a fifth more of the rows at K=300 D=50.)
 // With L the largest a - E over all blocks (logZ2 >= L), a block with a + E < L -
 // kLjNeedGap holds only responsibilities that are exactly zero, as the need masks of the
 // exact pass 1 state; the other blocks get their need bit.  Not-finite values make E
 // or a infinite or NaN, and the comparison then keeps the block.
 // A row with one near block needs no other block for logZ either: the gathering pass 2
-// forms its log-sum-exp there (the pair's bit is set in both words, near and faint).  The rest go on a list, which
-// the exact pass 1 then runs.
+// forms its log-sum-exp there (the pair's bit is set in both words, near and faint).  The
+// rest go on a list, which the exact pass 1 then runs.
 //
 // Bound: matrix steps and VALU, which mostly add up on a SIMD: at D = 128, 9 matrix
 // steps (288 cycles) and about 25 VALU instructions per (32 rows, block); matrix steps

@@ -10,6 +10,7 @@ from flash_gmm import data, diag_estep_into, iso_estep_into
 from parity import assert_dense_agrees
 
 pytestmark = pytest.mark.gpu
+LOG2_E = math.log2(math.e)
 KEYS = ("X", "mu", "log_sigma_sq", "log_pi")
 
 
@@ -34,6 +35,7 @@ def check(model, inp, dev, what):
         u, v = u.double().reshape(u.shape[0], -1), v.double().reshape(v.shape[0], -1)
         top = v.abs().max(dim=1).values
         assert bool(((u - v).abs().max(dim=1).values <= 1e-5 * top).all()), what
+    return got
 
 
 # A last block of 12 and of 8 components (the second with scattered zero weights too), and
@@ -85,3 +87,24 @@ def test_diag_squares_of_squares_that_underflow(unit, gpu_device):
     inp["mu"] *= unit
     inp["log_sigma_sq"] += 2.0 * math.log(unit)
     check("diag", inp, gpu_device, f"diag unit {unit}")
+
+
+@pytest.mark.parametrize("model,N,D", [("iso", 63_009, 128), ("diag", 42_017, 96)])
+def test_roundings_to_bf16_that_add_up(model, N, D, gpu_device):
+    """Rows whose products with their component's operands are all rounded down by nearly 2^-7,
+    and a second component, 20 (log2) behind, whose operands are 0: the first one's block must
+    stay.  The other components are tight, so far behind."""
+    K, e = 1024, 2.0 ** -8
+    inp = (data.iso_clustered if model == "iso" else data.diag_clustered)(N, K, D, seed=8)
+    inp["X"] *= 0.25
+    inp["mu"] *= 0.25
+    inp["log_sigma_sq"] -= 2.0 * math.log(4.0)
+    for k, m in ((100, 64.0 * (1.0 + 0.97 * e)), (900, 0.0)):
+        block = slice(k // 32 * 32, k // 32 * 32 + 32)
+        inp["log_pi"][block] = -math.inf   # the block's bound is the component's
+        inp["log_pi"][k] = -7.0
+        inp["mu"][k] = m
+        inp["log_sigma_sq"][k] = math.log(LOG2_E)   # exp(-lss) log2 e = 1: the operands are the mean's elements
+    inp["X"][[33, 5000, N - 1]] = 32.0 * (1.0 + 0.99 * e)
+    out = check(model, inp, gpu_device, f"{model} rounded down")
+    assert abs(float(out[1][100]) - 3.0) < 1e-4
