@@ -1878,7 +1878,8 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
-  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32), t_mid = (t_begin + t_end) / 2;
+  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32);
+  const int last_lo = (int)((t_end - t_begin) / 2) * 32 - 1;   // last row of the slab's first half
 
   auto words = [&](int64_t tb) -> unsigned {
     const int64_t t = tb + lane;
@@ -1977,7 +1978,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   int e;
   int cnt = take(e);
   if (cnt > 0) issue(e);
-  // Above D = 64 a partial ends once half of the slab's tiles are queued.
+  // Above D = 64 the first partial ends with the tile that reaches the slab's second half.
   const int parts = (lse_only || faint) ? 1 : PW;
 #pragma unroll 1
   for (int part = 0; part < parts; ++part) {
@@ -1986,6 +1987,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
 #pragma unroll
     for (int q = 0; q < NQ; ++q) *reinterpret_cast<f32x4*>(xt + c * RS + 8 * q + 4 * g) = raw[q];
     if (g == 0) rs_l[c] = rst;
+    const bool past_lo = PW > 1 && __builtin_amdgcn_ballot_w64(erow >= last_lo) != 0;
     const bool own = fused && erow >= 0 && ((sgl >> (erow & 31)) & 1u);
     const bool owns = fused && __builtin_amdgcn_ballot_w64(own) != 0;
     const int64_t orow = r_begin + erow;
@@ -2103,7 +2105,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       }
     }
     cnt = cnt_next;
-    if (part + 1 < parts && tb >= t_mid) break;
+    if (part + 1 < parts && past_lo) break;
   }
   if (lse_only || (faint && qt == 0)) return;
   store(part);

@@ -1539,7 +1539,8 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   const int64_t r_begin = (int64_t)slab * rows_per_slab;
   int64_t r_end = r_begin + rows_per_slab;
   if (r_end > N) r_end = N;
-  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32), t_mid = (t_begin + t_end) / 2;
+  const int64_t t_begin = r_begin / 32, t_end = cdiv(r_end, 32);
+  const int last_lo = (int)((t_end - t_begin) / 2) * 32 - 1;   // last row of the slab's first half
 
   // Need words of 64 tiles at a time, one per lane, the next batch in flight.
   auto words = [&](int64_t tb) -> unsigned {
@@ -1571,6 +1572,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   double2 rst[2];
   unsigned sgl[2] = {0u, 0u};   // the own-pairs word of the row's tile (fused)
   int erow[2] = {0, 0};
+  bool past_lo = false;   // the tile last computed reaches the slab's second half (uniform)
   // The rows come through resources over the slab: a lane without a row reads zeros
   // and makes no access, and the loads of a tile issue back to back.  X so while the
   // slab spans under 2 GiB (uniform; with one offset per lane where D fills whole
@@ -1621,6 +1623,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   // issued into the same stage once its registers are free.  Returns that tile's count.
   auto tile = [&](auto par) __attribute__((always_inline)) -> int {
     constexpr int P = decltype(par)::value;
+    if (PW > 1) past_lo = __builtin_amdgcn_ballot_w64(erow[P] >= last_lo) != 0;
     // This tile's rows: bf16 splits in registers, x1 and x2 to LDS, row state to LDS.
     // A row whose one needed block is this one (fused) has no row state yet: its ||x||^2
     // is formed here as pass 1 does, its logZ2 below.
@@ -1759,7 +1762,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   if (cnt0 > 0) issue(e, raw[0], rst[0], sgl[0], erow[0]);
   int cnt1 = cnt0 > 0 ? take(e) : 0;
   if (cnt1 > 0) issue(e, raw[1], rst[1], sgl[1], erow[1]);
-  // Above D = 64 a partial ends once half of the slab's tiles are queued.
+  // Above D = 64 the first partial ends with the tile that reaches the slab's second half.
   const int parts = (lse_only || faint) ? 1 : PW;
 #pragma unroll 1
   for (int p = 0; p < parts; ++p) {
@@ -1770,7 +1773,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
         break;
       }
       cnt1 = tile(std::integral_constant<int, 1>{});
-      if (p + 1 < parts && tb >= t_mid) break;
+      if (p + 1 < parts && past_lo) break;
     }
     if (lse_only || (faint && qt == 0)) return;
     store(p);
