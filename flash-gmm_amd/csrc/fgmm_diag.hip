@@ -228,7 +228,8 @@ DiagPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
       const int64_t n = cdiv(waves * current_device_cus(), p.KB);
       const int64_t want = one_round ? gather_slab_rounds(n, cdiv(N, 32), kGatherWaves, p.KB, current_device_cus())
                                      : gather_slab_count(n, cdiv(N, 32), kGatherWaves);
-      rows = cap_slab_rows(round_up(cdiv(N, want), 32), sizeof(double));
+      const size_t row_bytes = p.screen ? std::max(sizeof(double), screen_word_bytes(p.KB, sizeof(uint2))) : sizeof(double);
+      rows = cap_slab_rows(round_up(cdiv(N, want), 32), row_bytes);
       return (int)cdiv(N, rows);
     };
     p.spp = gather_parts(p.DP);
@@ -2721,7 +2722,7 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
                            sel, pl.autolj ? reinterpret_cast<float*>(ws + pl.off_lj) : nullptr,
                            reinterpret_cast<__bf16*>(ws + pl.off_xsplit),
                            reinterpret_cast<float2*>(ws + pl.off_zpair), list,
-                           std::min<int64_t>((int64_t)kFewRounds * 32 * current_device_cus(), (int64_t)nblk1 * 32));
+                           few_rows(nblk1));
         return hipSuccess;
       };
       hipError_t e1 = launch1(pl.lj ? &diag_lse_x6<DP, kLjmStore> : &diag_lse_x6<DP, kLjmNeed>);
@@ -3955,6 +3956,16 @@ extern "C" size_t fgmm_diag_workspace_bytes_ex(int64_t N, int64_t K, int64_t D, 
   if (N < 0 || K < 0 || D < 1) return 0;
   const int64_t rows = diag_bw_call(D, flags) ? std::min(N, diag_bw_chunk_rows(K)) : N;
   return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags)).total;
+}
+
+// For the tests, as fgmm_iso_plan_info (not declared in flashgmm.h).
+extern "C" void fgmm_diag_plan_info(int64_t N, int64_t K, int64_t D, unsigned flags, int64_t* info) {
+  const DiagPlan pl = make_plan(N, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags));
+  const int64_t v[6] = {pl.screen ? 1 : 0,
+                        pl.nprobe > 0 ? (int64_t)(pl.off_state + kStateMode * sizeof(int)) : -1,
+                        pl.screen ? (int64_t)pl.off_list : -1, few_rows(cdiv(N, 32 * kWaves)), pl.rows_per_slab,
+                        pl.nslab};
+  std::copy(v, v + 6, info);
 }
 
 extern "C" int fgmm_diag_estep_f32(const float* X, int64_t ldx, int64_t N, int64_t D, const float* mu,

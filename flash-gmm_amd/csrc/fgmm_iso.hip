@@ -282,7 +282,8 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     const int64_t cus = current_device_cus(), full = cdiv(8 * cus, p.KB);
     const int64_t want = p.DP <= 64 ? gather_slab_count(full, cdiv(N, 32), kGatherWaves)
                                     : gather_slab_rounds(full, cdiv(N, 32), kGatherWaves, p.KB, cus);
-    p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32 * p.spp), sizeof(double2)) / (32 * p.spp) * (32 * p.spp);
+    const size_t row_bytes = p.screen ? std::max(sizeof(double2), screen_word_bytes(p.KB, sizeof(unsigned))) : sizeof(double2);
+    p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32 * p.spp), row_bytes) / (32 * p.spp) * (32 * p.spp);
     p.nslab = (int)cdiv(N, p.rows_per_slab);
     if (p.DP <= 128) {   // its partials are laid out with or without the branch
       const int64_t wl = gather_slab_count(cdiv((int64_t)8 * current_device_cus(), p.KB), cdiv(N, 32), kGatherWaves);
@@ -758,6 +759,9 @@ __host__ inline PipeGrid pipe_grid(int64_t N) {
   }
   return pg;
 }
+
+// Listed rows up to which iso_lse_pipe runs the list one tile per workgroup.
+__host__ inline int64_t iso_few_rows(int64_t N) { return few_rows(pipe_grid(N).grid); }
 
 template <int DP>
 constexpr size_t lse_pipe_lds_bytes() {
@@ -3428,7 +3432,7 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
                            pl.KB, logZ, rowstat, ljmask, ljcount, dense ? 1 : 0, lj, sel,
                            reinterpret_cast<__bf16*>(ws + pl.off_xsplit), reinterpret_cast<float2*>(ws + pl.off_zpair),
                            pg.full, pg.small, list,
-                           std::min<int64_t>((int64_t)kFewRounds * 32 * current_device_cus(), pg.grid * 32));
+                           iso_few_rows(pl.N));
       }
     } else {
       return hipErrorInvalidValue;   // launch_ctile runs pass 1 above D = 128
@@ -4620,6 +4624,18 @@ extern "C" size_t fgmm_iso_workspace_bytes_ex(int64_t N, int64_t K, int64_t D, u
   if (N < 0 || K < 0 || D < 1) return 0;
   const int64_t rows = iso_bw_call(D, flags) ? std::min(N, iso_bw_chunk_rows(K)) : N;
   return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags)).total;
+}
+
+// For the tests (not declared in flashgmm.h): what the plan of a call may choose and where its
+// workspace keeps the choice.  info: 1 if the probe may select the screened pass 1; byte offsets
+// of the word that holds the choice (CallMode) and of the list's length; listed rows up to
+// which the list runs a tile per workgroup; rows per slab; slabs.
+extern "C" void fgmm_iso_plan_info(int64_t N, int64_t K, int64_t D, unsigned flags, int64_t* info) {
+  const IsoPlan pl = make_plan(N, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags));
+  const int64_t v[6] = {pl.screen ? 1 : 0,
+                        pl.nprobe > 0 ? (int64_t)(pl.off_state + kStateMode * sizeof(int)) : -1,
+                        pl.screen ? (int64_t)pl.off_list : -1, iso_few_rows(N), pl.rows_per_slab, pl.nslab};
+  std::copy(v, v + 6, info);
 }
 
 // The least workspace fgmm_iso_estep_f32 takes for the call (without the screened pass

@@ -2,6 +2,8 @@
 // the device-side choice of a call's branches.
 #pragma once
 
+#include <algorithm>
+
 #include "fgmm_common.hpp"
 
 namespace fgmm {
@@ -46,6 +48,12 @@ constexpr int kListBase = 64;   // ints before the first row of the list (entry 
 // Lists of up to this many 32-row workgroups per compute unit run one tile per workgroup
 // (a round of them takes about a quarter of a round of whole workgroups).
 constexpr int kFewRounds = 3;
+__host__ inline int64_t few_rows(int64_t grid) {
+  return 32 * std::min<int64_t>((int64_t)kFewRounds * current_device_cus(), grid);
+}
+// Bytes of a row's share of its tile's need words, rounded up: the gathering pass 2 after the
+// screening reads them through a resource over its slab (cap_slab_rows).
+__host__ constexpr size_t screen_word_bytes(int KB, size_t word) { return ((size_t)KB * word + 31) / 32; }
 
 // The screened pass 1 tells near pairs from faint ones.  A pair is near unless its
 // responsibility r provably has r, r ||x||, r ||x||^2 <= 2^-kNearGap; the faint pairs of
