@@ -797,7 +797,6 @@ struct ProbeSel {
   int n;
   int64_t min_pairs;
   int64_t max_screen;   // up to this many sampled pairs: the screened pass 1 (-1: never)
-  const unsigned* over; // set by a screened call that goes back to the exact pass 1
 };
 // The branch the probe selects (uniform; the default without a probe).
 constexpr int kProbeDefault = 0, kProbeStored = 1, kProbeScreen = 2;

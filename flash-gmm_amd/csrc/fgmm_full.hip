@@ -69,7 +69,7 @@ struct FullPlan {
   int screen_cap;   // its pool of log-joints per tile
   size_t off_probe;
   size_t off_lop, off_bsw, off_ck, off_l3, off_esw, off_rowstat, off_part_sig, off_part_mu, off_part_nk,
-      off_lj, off_need, off_bound, off_sc, total;
+      off_lj, off_need, off_bound, off_sc, off_over, total;
 };
 
 // One LDS stage holds SMB 32-coordinate blocks of one component: all of them up to
@@ -305,7 +305,12 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   }
   p.off_probe = off;
   if (p.autolj) off = align256(off + probe_bytes() + (size_t)p.nprobe * p.KP * 32 * sizeof(float));
-  p.off_sc = p.off_part_sig;   // read by pass 1 only; pass 2 writes the partials
+  // Read by pass 1 only, so in the space of the partials pass 2 writes: the screening's
+  // constants, then a word that says whether any tile's byte is set and these bytes
+  // (full_screen).
+  p.off_sc = p.off_part_sig;
+  p.off_over = align256(p.off_sc + (size_t)p.KP * (p.DP + kScreenConsts) * sizeof(float));
+  if (p.off_over + sizeof(unsigned) + (size_t)cdiv(N, 32) > p.off_lj) p.screen = false;
   p.total = off;
   return p;
 }
@@ -333,12 +338,13 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
                                                     const float* __restrict__ L, int64_t K, int D, int DP,
                                                     const float* __restrict__ lpi, bf16x8* __restrict__ l3,
                                                     double* __restrict__ esw, double* __restrict__ ck,
-                                                    float* __restrict__ sc) {
+                                                    float* __restrict__ sc, unsigned* __restrict__ any_over) {
   __shared__ double so[16][256];  // o_qj, DP <= 256
   __shared__ double red[3][4];    // sc: per wave, the squares of L - bf16(L), of bf16(L) and of b
   __shared__ double se[256];      // e_j, then log |L_jj|
   const int64_t k = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (any_over && k == 0 && tid == 0) *any_over = 0u;
   const int c = lane & 31, g = lane >> 5;
   const bool valid = k < K;
   const float* Lk = L + k * (int64_t)D * D;
@@ -461,13 +467,6 @@ __global__ __launch_bounds__(256) void full_x6_prep(const float* __restrict__ mu
 }
 
 
-// The branch, the default one where a screened call found a tile with more needed pairs
-// than its pool holds (full_screen).
-__device__ __forceinline__ int full_mode(const ProbeSel& p) {
-  const int m = probe_mode(p);
-  return m == kProbeScreen && *p.over != 0u ? kProbeDefault : m;
-}
-
 // What pass 1 leaves for pass 2 besides logZ2.
 constexpr int kLjmStore = 1;   // the stored log-joint
 constexpr int kLjmNeed = 2;    // need masks only (the default plan)
@@ -489,7 +488,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads),
 void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ l3,
                  const double* __restrict__ esw, const double* __restrict__ ck, int K, int KP,
                  float* __restrict__ logZ, double* __restrict__ rowstat, float* __restrict__ lj,
-                 unsigned* __restrict__ need, unsigned short* __restrict__ bound, int dense, ProbeSel probe) {
+                 unsigned* __restrict__ need, unsigned short* __restrict__ bound, int dense, ProbeSel probe,
+                 const unsigned* __restrict__ any_over) {
   constexpr int needmode = NM;
   constexpr bool LJ = LJM == kLjmStore || KEEP;
   static_assert(!KEEP || LJM == kLjmNeed, "KEEP adds the log-joint to the need masks");
@@ -498,8 +498,13 @@ void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
   // gathering pass 2 reads both.
   constexpr bool MASKS = LJM == kLjmNeed && !(KEEP && flj_applies(DP));
   // FGMM_FLAG_STORE_LOGJOINT_AUTO launches both need-mask instances; the probe's
-  // counts let the KEEP one (the stored branch) or the other run.
-  if (probe.count != nullptr && full_mode(probe) != (KEEP ? kProbeStored : kProbeDefault)) return;
+  // counts let the KEEP one (the stored branch) or the other run, after the screened pass 1
+  // over the tile groups that hold a tile whose byte is set (full_screen).
+  const int mode = probe_mode(probe);
+  if (probe.count != nullptr && KEEP != (mode == kProbeStored)) return;
+  const bool only_over = mode == kProbeScreen;
+  if (only_over && *any_over == 0u) return;
+  const unsigned char* over = reinterpret_cast<const unsigned char*>(any_over + 1);
   constexpr int NMB = DP / 32, NQ = DP / 16;
   constexpr int SMB = full_x6_smb(DP);            // coordinate blocks per stage
   constexpr int NST = NMB / SMB;                  // stages per component
@@ -534,6 +539,10 @@ void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
   const int64_t tw_step = LJM == kLjmNeed ? (int64_t)gridDim.x : ntw;
 
   for (int64_t tw = blockIdx.x; tw < ntw; tw += tw_step) {
+  if (only_over) {   // uniform over the workgroup
+    const int64_t t = tw * kWaves * TPW + lane;
+    if (__builtin_amdgcn_ballot_w64(lane < kWaves * TPW && t * 32 < N && over[t] != 0) == 0) continue;
+  }
   int64_t tile[TPW];   // the wave's 32-row tiles
   bool valid[TPW];     // this lane's row of each
   int ncand[TPW];      // the row's listed candidates (kNeedLists; lanes of half-wave 0)
@@ -770,7 +779,7 @@ __global__ __launch_bounds__(64 * kProbeWaves) void full_probe_ll(const float* _
 
 __global__ __launch_bounds__(256) void full_probe_count(int64_t N, int K, int KP, int ntile,
                                                         const float* __restrict__ lls,
-                                                        unsigned* __restrict__ count, unsigned* over) {
+                                                        unsigned* __restrict__ count) {
   __shared__ float mrow[8][32];
   __shared__ unsigned part[4];
   const int s = blockIdx.x;
@@ -794,8 +803,6 @@ __global__ __launch_bounds__(256) void full_probe_count(int64_t N, int K, int KP
   if (lane == 0) part[wave] = need;
   __syncthreads();
   if (tid == 0) count[s] = part[0] + part[1] + part[2] + part[3];
-  // full_screen's flag takes the first word of tile 0's log-joints, read above.
-  if (s == 0 && tid == 0) *over = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -1112,7 +1119,7 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   constexpr int NMB = DP / 32, NQ = DP / 16, NSB = NMB * (NMB + 1) / 2;
   constexpr int NGRP = gather_sig_groups(DP);
   if constexpr (LLO) {
-    if (full_mode(sel) != kProbeScreen) return;
+    if (probe_mode(sel) != kProbeScreen) return;
   } else {
     if (probe_selects(sel)) return;   // the stored branch's full_accum_ljt takes the call
   }
@@ -1269,7 +1276,8 @@ void full_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       if constexpr (LLO) {
         if (g == 0 && e >= 0) {
           const int64_t row = r_begin + e;
-          llo[(row >> 5) * cap + rank[((row >> 6) * KP + k) * 64 + (row & 63)]] = ll;
+          const int at = rank[((row >> 6) * KP + k) * 64 + (row & 63)];
+          if (at < cap) llo[(row >> 5) * cap + at] = ll;   // (a tile with more is full_lse_x6's)
         }
         if (!PREFETCH) cnt_next = take(en);
         e = en;
@@ -1634,10 +1642,13 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // two half-waves trade their partial sums so that each lane owns one row of a tile pair.
 // Upper bounds go to `ub` as bf16 ([workgroup][wave][tile pair][component][64 rows], 128
 // bytes a store); once the row's largest lower bound is final each lane reads its own
-// back, counts the needed pairs and leaves each its place in its tile's pool instead; a tile
-// with more than the pool holds sets `over`, and the exact pass 1 takes the call.  Bound: matrix steps and the squares' VALU, about equal.  The steps of the blocks
-// above L's diagonal (2 of 8 at D = 64) are left out: a component with a nonzero there
-// has A = infinity, so nothing of it is screened.
+// back, counts the needed pairs and leaves each its place in its tile's pool instead.  A tile
+// with more than the pool holds (nine rows of NaN, of whose pairs none can be left out) sets
+// its byte after `any_over`: full_lse_x6 runs the tile groups that hold such a byte, the
+// others keep the screening's results (N=250K K=256 D=64, one such tile: 1.61 ms, 3.25 ms
+// with the exact pass 1 over all).  Bound: matrix steps and the squares' VALU, about equal.
+// The steps of the blocks above L's diagonal (2 of 8 at D = 64) are left out: a component
+// with a nonzero there has A = infinity, so nothing of it is screened.
 // N=250K K=256 D=64, clustered: the drop-in call 2.641 -> 0.618 ms (0.705 with all eight
 // steps and a log-joint of every pair; exact pass 1 2.45 ms;
 // traced: full_screen 0.565, the gathered log-joint 0.075, full_need_lse 0.020).
@@ -1646,7 +1657,7 @@ template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads), amdgpu_waves_per_eu(2, 2)))
 void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, const bf16x8* __restrict__ l3,
                  const float* __restrict__ sc, int K, int KP, unsigned short* __restrict__ ub,
-                 unsigned* __restrict__ need, int cap, unsigned* __restrict__ over, ProbeSel sel) {
+                 unsigned* __restrict__ need, int cap, unsigned* __restrict__ any_over, ProbeSel sel) {
   if (probe_mode(sel) != kProbeScreen) return;
   using SH = ScreenShape<DP>;
   constexpr int NMB = SH::NMB, NQ = SH::NQ, CPS = SH::CPS, SCF = SH::SCF, TPW = kScreenTpw;
@@ -1791,7 +1802,10 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
         if ((tile + 1) * 32 < N) need[(tile + 1) * KP + k0 + lane] = w1;
       }
     }
-    if (n > (unsigned)cap) atomicOr(over, 1u);
+    if (c == 0 && (tile + g) * 32 < N) {
+      reinterpret_cast<unsigned char*>(any_over + 1)[tile + g] = n > (unsigned)cap;
+      if (n > (unsigned)cap) atomicOr(any_over, 1u);
+    }
   }
 }
 
@@ -1800,12 +1814,14 @@ void full_screen(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
 // loads in flight.  Bound: latency.
 __global__ __launch_bounds__(256) void full_need_lse(int64_t N, int K, int KP, const double* __restrict__ ll,
                                                      unsigned* __restrict__ need, double* __restrict__ rowstat,
-                                                     float* __restrict__ logZ, int cap, ProbeSel sel) {
-  if (full_mode(sel) != kProbeScreen) return;
+                                                     float* __restrict__ logZ, int cap,
+                                                     const unsigned* __restrict__ any_over, ProbeSel sel) {
+  if (probe_mode(sel) != kProbeScreen) return;
+  const unsigned char* over = reinterpret_cast<const unsigned char*>(any_over + 1);
   const int lane = threadIdx.x & 63, c = lane & 31;
   const int64_t tile = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t row = tile * 32 + c;
-  if (tile * 32 >= N) return;   // uniform over the wave
+  if (tile * 32 >= N || over[tile] != 0) return;   // uniform over the wave
   const double* lt = ll + tile * cap;   // the tile's pool, component by component
   unsigned* nw = need + tile * KP;
   // f(component, this lane's row needs it, its log-joint) over the tile's nonzero words.
@@ -1882,8 +1898,9 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
   // The screened pass 1 up to an eighth of the sampled pairs (a quarter of the stored
   // branch's least, half of them).
   const int64_t min_pairs = probe ? probe_min_pairs(pl.N, pl.nprobe, (int)pl.K) : 0;
-  unsigned* over = probe ? reinterpret_cast<unsigned*>(ws + pl.off_probe + probe_bytes()) : nullptr;
-  const ProbeSel psel = {probe, pl.nprobe, min_pairs, pl.screen && !dense ? min_pairs / 4 : (int64_t)-1, over};
+  const bool screen = pl.screen && !dense;
+  const ProbeSel psel = {probe, pl.nprobe, min_pairs, screen ? min_pairs / 4 : (int64_t)-1};
+  unsigned* over = screen ? reinterpret_cast<unsigned*>(ws + pl.off_over) : nullptr;
   if (run1) {
     if constexpr (flj_applies(DP)) {
       if (pl.autolj) {
@@ -1893,14 +1910,26 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                            stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                            reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, pl.nprobe, lls);
         hipLaunchKernelGGL(full_probe_count, dim3((unsigned)pl.nprobe), dim3(256), 0, stream, pl.N, (int)pl.K, pl.KP,
-                           pl.nprobe, lls, probe, reinterpret_cast<unsigned*>(lls));
-      if (pl.screen && !dense) {
+                           pl.nprobe, lls, probe);
+      }
+      if (screen) {
         unsigned* need = reinterpret_cast<unsigned*>(ws + pl.off_need);
+        unsigned short* ub = reinterpret_cast<unsigned short*>(ws + pl.off_lj);
+        double* ll = reinterpret_cast<double*>(ws + pl.off_lj + screen_ub_bytes(pl.N, pl.KP));
         hipLaunchKernelGGL((full_screen<DP>), dim3((unsigned)cdiv(pl.N, kScreenRows)), dim3(kThreads), 0, stream, X,
                            ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                            reinterpret_cast<const float*>(ws + pl.off_sc), (int)pl.K, pl.KP,
-                           reinterpret_cast<unsigned short*>(ws + pl.off_lj), need, pl.screen_cap, over, psel);
-      }
+                           ub, need, pl.screen_cap, over, psel);
+        constexpr size_t ldsg = gather_lds_bytes<DP>();
+        auto kll = &full_accum_gather<DP, 0, false, true>;
+        const hipError_t el = set_lds(reinterpret_cast<const void*>(kll), ldsg);
+        if (el != hipSuccess) return el;
+        hipLaunchKernelGGL(kll, dim3((unsigned)gather_grid(pl.nslab, (int)pl.K)), dim3(64 * kGatherWaves), ldsg,
+                           stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
+                           reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat, need,
+                           pl.nslab, pl.rows_per_slab, nullptr, nullptr, nullptr, 0, nullptr, psel, ll, ub, pl.screen_cap);
+        hipLaunchKernelGGL(full_need_lse, dim3((unsigned)cdiv(pl.N, 128)), dim3(256), 0, stream, pl.N, (int)pl.K,
+                           pl.KP, ll, need, rowstat, logZ, pl.screen_cap, over, psel);
       }
     }
     const size_t lds1 = full_x6_lds_bytes(DP) + (pl.needmode == kNeedLists ? full_list_lds_bytes(DP, pl.KP) : 0);
@@ -1924,7 +1953,7 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                        pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                        reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, logZ,
                        rowstat, lj, reinterpret_cast<unsigned*>(ws + pl.off_need),
-                       reinterpret_cast<unsigned short*>(ws + pl.off_bound), dense ? 1 : 0, psel);
+                       reinterpret_cast<unsigned short*>(ws + pl.off_bound), dense ? 1 : 0, psel, over);
     if constexpr (flj_applies(DP)) {
       if (pl.autolj) {
         // The stored branch's instance: the same pass, keeping the log-joint and no need
@@ -1936,22 +1965,7 @@ hipError_t launch_passes(const FullPlan& pl, const float* X, int64_t ldx, unsign
                            reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
                            reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, logZ, rowstat,
                            lj, reinterpret_cast<unsigned*>(ws + pl.off_need),
-                           reinterpret_cast<unsigned short*>(ws + pl.off_bound), dense ? 1 : 0, psel);
-      }
-      if (pl.screen && !dense) {
-        unsigned* need = reinterpret_cast<unsigned*>(ws + pl.off_need);
-        const unsigned short* ub = reinterpret_cast<const unsigned short*>(ws + pl.off_lj);
-        double* ll = reinterpret_cast<double*>(ws + pl.off_lj + screen_ub_bytes(pl.N, pl.KP));
-        constexpr size_t ldsg = gather_lds_bytes<DP>();
-        auto kll = &full_accum_gather<DP, 0, false, true>;
-        e = set_lds(reinterpret_cast<const void*>(kll), ldsg);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kll, dim3((unsigned)gather_grid(pl.nslab, (int)pl.K)), dim3(64 * kGatherWaves), ldsg,
-                           stream, X, ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_l3),
-                           reinterpret_cast<const double*>(ws + pl.off_esw), ck, (int)pl.K, pl.KP, rowstat, need,
-                           pl.nslab, pl.rows_per_slab, nullptr, nullptr, nullptr, 0, nullptr, psel, ll, ub, pl.screen_cap);
-        hipLaunchKernelGGL(full_need_lse, dim3((unsigned)cdiv(pl.N, 128)), dim3(256), 0, stream, pl.N, (int)pl.K,
-                           pl.KP, ll, need, rowstat, logZ, pl.screen_cap, psel);
+                           reinterpret_cast<unsigned short*>(ws + pl.off_bound), dense ? 1 : 0, psel, nullptr);
       }
     }
   }
@@ -2914,6 +2928,17 @@ extern "C" size_t fgmm_full_workspace_bytes_ex(int64_t N, int64_t K, int64_t D, 
   return make_plan(rows, K, D, wants_stored_lj(flags), bf16, wants_auto_lj(flags)).total;
 }
 
+// For the tests (not declared in flashgmm.h).  info: 1 if the probe may select the screened
+// pass 1; byte offset of the probe's counts, their number and the largest sum at which it is
+// selected; byte offset of the tiles' bytes (full_screen); log-joints a tile's pool holds.
+extern "C" void fgmm_full_plan_info(int64_t N, int64_t K, int64_t D, unsigned flags, int64_t* info) {
+  const FullPlan pl = make_plan(N, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags));
+  const int64_t v[6] = {pl.screen ? 1 : 0, (int64_t)pl.off_probe, pl.nprobe,
+                        pl.autolj ? probe_min_pairs(N, pl.nprobe, (int)K) / 4 : -1, (int64_t)(pl.off_over + sizeof(unsigned)),
+                        pl.screen_cap};
+  std::copy(v, v + 6, info);
+}
+
 extern "C" int fgmm_full_estep_f32(const float* X, int64_t ldx, int64_t N, int64_t D, const float* mu,
                                    int64_t ldmu, int64_t K, const float* prec_chol, const float* log_pi,
                                    float* logZ, float* Nk, float* mu_acc, float* sig_outer,
@@ -2982,7 +3007,8 @@ extern "C" int fgmm_full_estep_f32(const float* X, int64_t ldx, int64_t N, int64
     hipLaunchKernelGGL(full_x6_prep, dim3((unsigned)pl.KP), dim3(256), 0, stream, mu, ldmu, prec_chol, K,
                        (int)D, pl.DP, log_pi, reinterpret_cast<bf16x8*>(ws + pl.off_l3),
                        reinterpret_cast<double*>(ws + pl.off_esw), reinterpret_cast<double*>(ws + pl.off_ck),
-                       pl.screen ? reinterpret_cast<float*>(ws + pl.off_sc) : nullptr);
+                       pl.screen ? reinterpret_cast<float*>(ws + pl.off_sc) : nullptr,
+                       pl.screen ? reinterpret_cast<unsigned*>(ws + pl.off_over) : nullptr);
   if (N > 0) {
     auto run = [&](auto dp_tag) -> hipError_t {
       constexpr int DP = decltype(dp_tag)::value;

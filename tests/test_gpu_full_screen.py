@@ -6,9 +6,10 @@ import math
 import pytest
 import torch
 
-from flash_gmm import data, full_estep_into
+from flash_gmm import _lib, data, full_estep_into
 from oracle import gmm_oracle as O
 from parity import assert_close_stats, assert_dense_agrees
+from routes import SCREEN, call_mode, overflowed_tiles
 
 pytestmark = pytest.mark.gpu
 KEYS = ("X", "mu", "prec_chol", "log_pi")
@@ -69,3 +70,24 @@ def test_rows_of_several_and_special_components(gpu_device):
     inp["X"][64:96] = math.nan   # a tile of which every pair is needed: the exact pass 1
     print("full screen full tile", flush=True)
     same(call(inp, gpu_device, "auto"), call(inp, gpu_device, False), "full tile")
+
+
+def test_a_tile_past_its_pool_costs_only_its_group(gpu_device):
+    """Tiles whose needed pairs exceed their pool (every pair of NaN rows is needed): the call
+    stays screened, and those tiles get the exact pass 1's results."""
+    dev, N, K, D = gpu_device, 40_033, 100, 39
+    inp = data.full_clustered(N, K, D, seed=2)
+    inp["X"][64:80] = math.nan
+    inp["X"][20_000] = math.nan   # alone in its tile: within the pool
+    inp["X"][40_010:] = math.nan   # 22 rows of the last tile but one, and the last one's only row
+    args = [inp[k].to(dev) for k in KEYS]
+    out = [torch.empty(N, device=dev), torch.empty(K, device=dev), torch.empty(K, D, device=dev),
+           torch.empty(K, D, D, device=dev)]
+    nbytes = _lib.lib().fgmm_full_workspace_bytes_ex(N, K, D, _lib.FLAG_STORE_LOGJOINT_AUTO)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    print("full screen pools", flush=True)
+    full_estep_into(*args, *out, store_log_joint="auto", workspace=ws, phase=1)
+    assert call_mode("full", ws, N, K, D, _lib.FLAG_STORE_LOGJOINT_AUTO) == SCREEN
+    assert overflowed_tiles(ws, N, K, D) == [2, 1250]
+    full_estep_into(*args, None, *out[1:], store_log_joint="auto", workspace=ws, phase=2)
+    same(out, call(inp, dev, False), "pools")

@@ -1,21 +1,8 @@
 """Plans of the E-steps, queried without a GPU."""
 
-import ctypes
-
 import pytest
 
-from flash_gmm import _lib
-
-
-def plan_info(model, N, K, D, flags=0):
-    """(may screen, offset of the choice, offset of the list's length, short list's rows, rows
-    per slab, slabs)."""
-    info = (ctypes.c_int64 * 6)()
-    fn = getattr(_lib.lib(), f"fgmm_{model}_plan_info")
-    fn.restype = None
-    fn.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_uint, ctypes.POINTER(ctypes.c_int64)]
-    fn(N, K, D, flags, info)
-    return list(info)
+from routes import plan_info
 
 
 # The widest plans that screen (the rows' block bounds fill LDS), and ordinary ones.
