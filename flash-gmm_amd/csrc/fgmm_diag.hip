@@ -1805,10 +1805,11 @@ __host__ size_t x6_lds_bytes_rt(int DP) {
 __host__ __device__ constexpr int gather_rs(int DP) { return DP + 4; }
 constexpr int kGatherSt = 20;   // row stride (floats) of half an S tile in LDS
 
-__host__ __device__ constexpr size_t gather_lds_bytes(int DP) {
+__host__ __device__ constexpr size_t gather_lds_bytes(int DP, bool SCR) {
   return (size_t)(DP / 8) * 4 * 64 * 16                          // mu block (bf16x8 operands)
-         + (size_t)32 * sizeof(double)                            // its constants
-         + (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float)  // half an S tile per wave
+         + (SCR ? (size_t)32 * sizeof(double)                              // its constants
+                  + (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float)  // half an S tile per wave
+                : 0)
          + (size_t)kGatherWaves * 32 * gather_rs(DP) * 4          // X tile per wave
          + (size_t)kGatherWaves * 32 * sizeof(double)              // logZ2 per wave
          + (size_t)kGatherWaves * 64 * sizeof(int);                // row queue per wave
@@ -1821,7 +1822,13 @@ __host__ inline int64_t gather_grid(int nslab, int KB) { return gather_item_grid
 // matrix steps.
 __host__ __device__ constexpr int gather_waves_per_simd(int DP) { return DP <= 64 ? 2 : 1; }
 
-template <int DP>
+// SCR: the pass after the screened pass 1, over the near pairs (screen_pairs); with own_lse
+// it forms the logZ2 of the rows near one block only, and with lse_only nothing else.  The
+// other instance is the default plan's pass, and after SCR the screened call's second, over
+// the faint pairs.  (As one kernel with both, the default plan's pass spilled at D = 64:
+// N=800K K=300 D=48 on N(0, I) rows 1.41 ms, 1.29 ms as two; D = 32 1.16 and 1.11 ms at
+// N=500K K=1024.)
+template <int DP, bool SCR>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kGatherWaves, 64 * kGatherWaves),
                           amdgpu_waves_per_eu(gather_waves_per_simd(DP), gather_waves_per_simd(DP))))
 void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
@@ -1829,8 +1836,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
                        double* __restrict__ rowstat, const uint2* __restrict__ need, int nslab,
                        int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_sq,
                        float* __restrict__ part_nk, int dense, const int* __restrict__ sel,
-                       float* __restrict__ logZ, int own_lse, int lse_only, unsigned* __restrict__ alive,
-                       int faint) {
+                       float* __restrict__ logZ, int own_lse, int lse_only, unsigned* __restrict__ alive) {
   constexpr int NQ = DP / 8;      // chunks of 8 dimensions (16 features)
   constexpr int NQH = NQ / 2;
   constexpr int NJ = DP / 32;
@@ -1840,16 +1846,14 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   static_assert(NQ % 2 == 0, "two halves of chunks");
   // The stored branch's diag_accum_ljt takes the call when the probe selects it.
   const int mode = call_mode(sel);
-  if (mode == kModeStored || (mode == kModeDefault && (lse_only || faint))) return;
-  // After the screened pass 1 the rows near one block only (the pairs in both words) have
-  // no logZ2 yet: it is formed here.
-  const bool screened = mode == kModeScreen, fused = screened && own_lse;
+  if (SCR ? mode != kModeScreen : mode == kModeStored) return;
+  const bool faint = !SCR && mode == kModeScreen;
 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   unsigned char* lp = lds_raw;
   bf16x8* mu_l = reinterpret_cast<bf16x8*>(lp);  lp += (size_t)BLK * sizeof(bf16x8);
-  double* kc_l = reinterpret_cast<double*>(lp);  lp += 32 * sizeof(double);
-  float* st_all = reinterpret_cast<float*>(lp);  lp += (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float);
+  double* kc_l = reinterpret_cast<double*>(lp);  lp += SCR ? 32 * sizeof(double) : 0;
+  float* st_all = reinterpret_cast<float*>(lp);  lp += !SCR ? 0 : (size_t)kGatherWaves * 32 * kGatherSt * sizeof(float);
   float* xt_all = reinterpret_cast<float*>(lp);  lp += (size_t)kGatherWaves * 32 * RS * 4;
   double* rs_all = reinterpret_cast<double*>(lp); lp += (size_t)kGatherWaves * 32 * sizeof(double);
   int* q_all = reinterpret_cast<int*>(lp);
@@ -1860,13 +1864,12 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   int sg, kb;
   if (!gather_item(blockIdx.x, gather_groups(nslab), KB, sg, kb)) return;   // uniform over the workgroup
   if (faint) {
-    // The second run after the screened pass 1: the block's faint pairs, where one of its
-    // components has too small an Nk to absorb them (one of zero weight has none).
+    // The block's faint pairs, where one of its components has too small an Nk to absorb them (one of zero weight has none).
     const bool none = kc_x6[(int64_t)kb * 32 + kc_x6_index(c)] == -INFINITY;
     if (((unsigned)__builtin_amdgcn_ballot_w64(!none) & ~alive[kb]) == 0u) return;   // uniform
   }
   for (int idx = tid; idx < BLK; idx += 64 * kGatherWaves) mu_l[idx] = mu3[(int64_t)kb * BLK + idx];
-  if (tid < 32) kc_l[tid] = kc_x6[(int64_t)kb * 32 + tid];
+  if (SCR && tid < 32) kc_l[tid] = kc_x6[(int64_t)kb * 32 + tid];
   __syncthreads();
   const int slab = sg * kGatherWaves + wave;
   if (slab >= nslab) return;   // no barrier follows
@@ -1887,7 +1890,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     if (t >= t_end) return 0u;
     const uint2 w = need[t * KB + kb];
     // The halves of the block, or (screened) its near and its faint pairs.
-    return !screened ? w.x | w.y : faint ? w.y & ~w.x : w.x;
+    return SCR ? w.x : faint ? w.y & ~w.x : w.x | w.y;
   };
   int64_t tb = t_begin;
   unsigned mword = words(tb), mnext = words(tb + 64);
@@ -1908,18 +1911,18 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   // the slab spans under 2 GiB (uniform), else load_row4.
   f32x4 raw[NQ];
   double rst;
-  unsigned sgl = 0u;   // the own-pairs word of the row's tile (fused)
+  unsigned sgl = 0u;   // the own-pairs word of the row's tile (SCR)
   int erow = -1;
   const int64_t slab_bytes = (r_end - r_begin) * ldx * (int64_t)sizeof(float);
   const bool xbuf = D == DP && slab_bytes <= ((int64_t)1 << 31) - 256;
   const buf_rsrc xres = make_rsrc(X + r_begin * ldx, xbuf ? (uint32_t)slab_bytes : 0u);
   const buf_rsrc rres = make_rsrc(rowstat + r_begin, (uint32_t)((r_end - r_begin) * sizeof(double)));
-  const buf_rsrc sres = make_rsrc(fused ? need + t_begin * KB + kb : nullptr,
-                                  fused ? (uint32_t)((t_end - t_begin) * KB * sizeof(uint2)) : 0u);
+  const buf_rsrc sres = make_rsrc(SCR && own_lse ? need + t_begin * KB + kb : nullptr,
+                                  SCR && own_lse ? (uint32_t)((t_end - t_begin) * KB * sizeof(uint2)) : 0u);
   auto issue = [&](int e) {
     const bool ok = e >= 0;
     erow = e;
-    sgl = buf_load_u32(sres, buf_off(ok ? (e >> 5) * KB * (int)sizeof(uint2) + 4 : kBufOob));
+    if constexpr (SCR) sgl = buf_load_u32(sres, buf_off(ok ? (e >> 5) * KB * (int)sizeof(uint2) + 4 : kBufOob));
     if (xbuf) {
       const int off = buf_off(ok ? (int)((int64_t)e * ldx * (int64_t)sizeof(float)) + 16 * g : kBufOob);
 #pragma unroll
@@ -1972,7 +1975,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       accq[j] = zero16();
     }
     if (g == 0) part_nk[kbase + c] = nk;
-    if (screened && !faint) mark_alive(alive, kb, nk);
+    if constexpr (SCR) mark_alive(alive, kb, nk);
     nk = 0.0f;
   };
 
@@ -1980,7 +1983,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
   int cnt = take(e);
   if (cnt > 0) issue(e);
   // Above D = 64 the first partial ends with the tile that reaches the slab's second half.
-  const int parts = (lse_only || faint) ? 1 : PW;
+  const int parts = ((SCR && lse_only) || faint) ? 1 : PW;
 #pragma unroll 1
   for (int part = 0; part < parts; ++part) {
   while (cnt > 0) {
@@ -1989,8 +1992,8 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     for (int q = 0; q < NQ; ++q) *reinterpret_cast<f32x4*>(xt + c * RS + 8 * q + 4 * g) = raw[q];
     if (g == 0) rs_l[c] = rst;
     const bool past_lo = PW > 1 && __builtin_amdgcn_ballot_w64(erow >= last_lo) != 0;
-    const bool own = fused && erow >= 0 && ((sgl >> (erow & 31)) & 1u);
-    const bool owns = fused && __builtin_amdgcn_ballot_w64(own) != 0;
+    const bool own = SCR && erow >= 0 && ((sgl >> (erow & 31)) & 1u);
+    const bool owns = SCR && __builtin_amdgcn_ballot_w64(own) != 0;
     const int64_t orow = r_begin + erow;
     int en;
     const int cnt_next = take(en);
@@ -2049,7 +2052,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    if (lse_only) {
+    if (SCR && lse_only) {
       cnt = cnt_next;
       continue;
     }
@@ -2108,7 +2111,7 @@ void diag_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int 
     cnt = cnt_next;
     if (part + 1 < parts && past_lo) break;
   }
-  if (lse_only || (faint && qt == 0)) return;
+  if ((SCR && lse_only) || (faint && qt == 0)) return;
   store(part);
   }
 }
@@ -2757,21 +2760,28 @@ hipError_t launch_passes(const DiagPlan& pl, const float* X, int64_t ldx, unsign
                              words, sel, pl.KB, pl.KP, pl.nslab_lj, pl.rows_per_slab_lj, ncg, pmu, psq, pnk);
         }
       }
-      constexpr size_t lds = gather_lds_bytes(DP);
-      static_assert(lds <= kMaxLds, "gathering pass 2 exceeds LDS");
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&diag_accum_gather<DP>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (e != hipSuccess) return e;
-      auto gather = [&](int faint_pass) {
-        hipLaunchKernelGGL(diag_accum_gather<DP>, dim3((unsigned)gather_grid(pl.nslab, pl.KB)),
-                           dim3(64 * kGatherWaves), lds, stream, X, ldx, pl.N, (int)pl.D,
-                           reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
-                           reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, pl.KP, rowstat, words,
-                           pl.nslab, pl.rows_per_slab, pmu, psq, pnk, dense ? 1 : 0, sel,
-                           logZ, run1 && !faint_pass ? 1 : 0, run2 ? 0 : 1, alive, faint_pass);
+      // After the screened pass 1 the SCR instance, then the other over the faint pairs; the
+      // choice lets one of them, or both, run.
+      auto gather = [&](auto scr_tag) -> hipError_t {
+        constexpr bool SCR = decltype(scr_tag)::value;
+        constexpr size_t lds = gather_lds_bytes(DP, SCR);
+        static_assert(lds <= kMaxLds, "gathering pass 2 exceeds LDS");
+        auto kern = &diag_accum_gather<DP, SCR>;
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3((unsigned)gather_grid(pl.nslab, pl.KB)), dim3(64 * kGatherWaves), lds, stream, X,
+                           ldx, pl.N, (int)pl.D, reinterpret_cast<const bf16x8*>(ws + pl.off_mu3),
+                           reinterpret_cast<const double*>(ws + pl.off_kcx6), pl.KB, pl.KP, rowstat, words, pl.nslab,
+                           pl.rows_per_slab, pmu, psq, pnk, dense ? 1 : 0, sel, logZ, run1 ? 1 : 0, run2 ? 0 : 1, alive);
+        return hipGetLastError();
       };
-      gather(0);
-      if (screen && run2) gather(1);
+      if (screen) {
+        const hipError_t e = gather(std::true_type{});
+        if (e != hipSuccess || !run2) return e;
+      }
+      const hipError_t e = gather(std::false_type{});
+      if (e != hipSuccess) return e;
       return hipGetLastError();
     }
     if (pl.lj_sparse) {
