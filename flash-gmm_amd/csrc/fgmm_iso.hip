@@ -213,7 +213,7 @@ __host__ __device__ constexpr int bf16_halves(int DP);
 __host__ inline int bf16_blocks_per_group(int DP, int KB);
 
 IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool bf16 = false,
-                  bool auto_lj = false, bool allow_screen = true) {
+                  bool auto_lj = false, bool allow_screen = true, bool lean = false) {
   IsoPlan p{};
   p.N = N; p.K = K; p.D = D;
   p.DP = iso_padded_dim(D);
@@ -278,9 +278,12 @@ IsoPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool b
     // (there, 64 slabs in two rounds took 0.266 ms at N=1M K=1024 D=128, 32 slabs take
     // 0.247 ms; their float32 sums go out in two partials each, so that they are no
     // longer).  The stored branch's pass 2 takes eight blocks per compute unit.
-    p.spp = gather_parts(p.DP);
+    // A lean plan has one partial a slab, of as many slabs as that branch has, so its
+    // workspace is the smallest (whole rounds of slabs with two partials take up to twice as
+    // much of them).
+    p.spp = lean ? 1 : gather_parts(p.DP);
     const int64_t cus = current_device_cus(), full = cdiv(8 * cus, p.KB);
-    const int64_t want = p.DP <= 64 ? gather_slab_count(full, cdiv(N, 32), kGatherWaves)
+    const int64_t want = p.DP <= 64 || lean ? gather_slab_count(full, cdiv(N, 32), kGatherWaves)
                                     : gather_slab_rounds(full, cdiv(N, 32), kGatherWaves, p.KB, cus);
     const size_t row_bytes = p.screen ? std::max(sizeof(double2), screen_word_bytes(p.KB, sizeof(unsigned))) : sizeof(double2);
     p.rows_per_slab = cap_slab_rows(round_up(cdiv(N, want), 32 * p.spp), row_bytes) / (32 * p.spp) * (32 * p.spp);
@@ -1490,12 +1493,12 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
                       int64_t rows_per_slab, float* __restrict__ part_mu, float* __restrict__ part_nk,
                       float* __restrict__ part_sig, int dense, const int* __restrict__ sel,
                       const unsigned* __restrict__ own_words, const double2* __restrict__ kc_blk,
-                      float* __restrict__ logZ, int lse_only, unsigned* __restrict__ alive, int faint) {
+                      float* __restrict__ logZ, int lse_only, unsigned* __restrict__ alive, int faint, int spp) {
   constexpr int NQ = DP / 16;
   constexpr int NJ = DP / 32;
   constexpr int RS = gather_rs(DP);
   constexpr int BLK = NQ * 4 * 64;   // bf16x8 per component block
-  constexpr int PW = gather_parts(DP);
+  const int pw = gather_parts(DP) > 1 ? spp : 1;   // partials of this plan's slabs
   // The stored branch of FGMM_FLAG_STORE_LOGJOINT_AUTO runs instead when selected; after
   // the screened pass 1 this kernel always runs, else with at least dense_min needed rows
   // iso_accum_tiles does (uniform exits).
@@ -1627,7 +1630,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   // issued into the same stage once its registers are free.  Returns that tile's count.
   auto tile = [&](auto par) __attribute__((always_inline)) -> int {
     constexpr int P = decltype(par)::value;
-    if (PW > 1) past_lo = __builtin_amdgcn_ballot_w64(erow[P] >= last_lo) != 0;
+    if (gather_parts(DP) > 1) past_lo = __builtin_amdgcn_ballot_w64(erow[P] >= last_lo) != 0;
     // This tile's rows: bf16 splits in registers, x1 and x2 to LDS, row state to LDS.
     // A row whose one needed block is this one (fused) has no row state yet: its ||x||^2
     // is formed here as pass 1 does, its logZ2 below.
@@ -1735,7 +1738,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   auto store = [&](int p) __attribute__((always_inline)) {
     nk += __shfl_xor(nk, 32);
     sig += __shfl_xor(sig, 32);
-    const int64_t kbase = (int64_t)(slab * PW + p) * KP + (int64_t)kb * 32;
+    const int64_t kbase = (int64_t)(slab * pw + p) * KP + (int64_t)kb * 32;
     float* pm = part_mu + kbase * DP + 4 * g * DP + c;
     if (faint) {
       nk += part_nk[kbase + c];
@@ -1767,7 +1770,7 @@ void iso_accum_gather(const float* __restrict__ X, int64_t ldx, int64_t N, int D
   int cnt1 = cnt0 > 0 ? take(e) : 0;
   if (cnt1 > 0) issue(e, raw[1], rst[1], sgl[1], erow[1]);
   // Above D = 64 the first partial ends with the tile that reaches the slab's second half.
-  const int parts = (lse_only || faint) ? 1 : PW;
+  const int parts = (lse_only || faint) ? 1 : pw;
 #pragma unroll 1
   for (int p = 0; p < parts; ++p) {
     while (cnt0 > 0) {
@@ -3473,7 +3476,7 @@ hipError_t launch_passes(const IsoPlan& pl, const float* X, int64_t ldx, unsigne
                            reinterpret_cast<const double4*>(ws + pl.off_kcgat), pl.KB, pl.KP, rowstat,
                            words, ljcount, dense_min, pl.nslab, pl.rows_per_slab, pmu, pnk, psig,
                            dense ? 1 : 0, sel, faint_pass ? ljmask : run1 ? faint : nullptr, kc_blk, logZ,
-                           run2 ? 0 : 1, alive, faint_pass);
+                           run2 ? 0 : 1, alive, faint_pass, pl.spp);
       };
       gather(ljmask, 0);
       if (!run2) return hipGetLastError();
@@ -4638,14 +4641,14 @@ extern "C" void fgmm_iso_plan_info(int64_t N, int64_t K, int64_t D, unsigned fla
   std::copy(v, v + 6, info);
 }
 
-// The least workspace fgmm_iso_estep_f32 takes for the call (without the screened pass
-// 1); fgmm_iso_workspace_bytes_ex gives what it can use.
+// The least workspace fgmm_iso_estep_f32 takes for the call (a lean plan without the screened
+// pass 1); fgmm_iso_workspace_bytes_ex gives what it can use.
 namespace fgmm {
 size_t iso_min_workspace(int64_t N, int64_t K, int64_t D, unsigned flags);
 }
 size_t fgmm::iso_min_workspace(int64_t N, int64_t K, int64_t D, unsigned flags) {
   const int64_t rows = iso_bw_call(D, flags) ? std::min(N, iso_bw_chunk_rows(K)) : N;
-  return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags), false)
+  return make_plan(rows, K, D, wants_stored_lj(flags), (flags & FGMM_FLAG_BF16) != 0, wants_auto_lj(flags), false, true)
       .total;
 }
 
@@ -4687,10 +4690,13 @@ extern "C" int fgmm_iso_estep_f32(const float* X, int64_t ldx, int64_t N, int64_
   }
   // The stored log-joint path streams X with 32-bit buffer offsets (row stride at
   // most kMaxBufLdx floats); wider strides recompute, which needs less workspace.
-  // A workspace without room for the screened pass 1 runs the call without it.
+  // A workspace without room for the screened pass 1 runs the call without it, one without
+  // room for two partials a slab on a lean plan.
   const bool stored = wants_stored_lj(flags) && ldx <= kMaxBufLdx;
   IsoPlan pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags));
   if (workspace_bytes < pl.total && pl.screen) pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags), false);
+  if (workspace_bytes < pl.total && pl.spp > 1)
+    pl = make_plan(N, K, D, stored, bf16, wants_auto_lj(flags), false, true);
   if (workspace_bytes < pl.total || (pl.total > 0 && workspace == nullptr)) return FGMM_ERR_WORKSPACE;
   if (!want_logz) logZ = nullptr;
   unsigned char* ws = static_cast<unsigned char*>(workspace);

@@ -193,3 +193,37 @@ def test_noalloc_under_graph_capture(gpu_device):
         ref = _run(inp, dev, noalloc=False)
         for u, v in zip(o, ref):
             assert torch.equal(u, v), f"replay {rep}"
+
+
+@pytest.mark.parametrize("N,K,D", [(60_001, 672, 128), (66_000, 1056, 125), (20_000, 1056, 128)])
+def test_noalloc_takes_what_a_lean_plan_fits(N, K, D, gpu_device):
+    """Calls whose plan with two partials a slab is beyond FGMM_NOALLOC_SCRATCH_BYTES, and whose
+    lean plan is not: one call, split in phases too, logZ bit for bit the workspace entry
+    point's and the statistics' float32 sums in other groupings."""
+    dev = gpu_device
+    L = _lib.lib()
+    assert L.fgmm_iso_workspace_bytes(N, K, D) > 64 << 20
+    inp = data.iso_clustered(N, K, -(-D // 4) * 4, seed=37)
+    inp["X"], inp["mu"] = inp["X"][:, :D].contiguous(), inp["mu"][:, :D].contiguous()
+    if D % 4:   # rows the kernels can read in place
+        inp["X"] = torch.nn.functional.pad(inp["X"], (0, 4 - D % 4))
+    print(f"noalloc lean N={N} K={K} D={D}", flush=True)
+    X, mu, lss, lpi = _inputs(inp, dev)
+    ws = torch.empty(L.fgmm_iso_workspace_bytes(N, K, D), dtype=torch.uint8, device=dev)
+
+    def run(fn, o, flags, *extra):
+        ptrs = [t.data_ptr() for t in o]
+        _lib.check(fn(X.data_ptr(), X.shape[1], N, D, mu.data_ptr(), D, K, lss.data_ptr(), lpi.data_ptr(), *ptrs, *extra,
+                      flags, _lib.stream_handle(dev)), "lean")
+        torch.cuda.synchronize()
+        return o
+
+    ref = run(L.fgmm_iso_estep_f32, _outputs(N, K, D, dev), 0, ws.data_ptr(), ws.numel())
+    whole = run(L.fgmm_iso_estep_f32_noalloc, _outputs(N, K, D, dev), 0)
+    split = _outputs(N, K, D, dev)
+    run(L.fgmm_iso_estep_f32_noalloc, split, _lib.FLAG_PHASE1)
+    run(L.fgmm_iso_estep_f32_noalloc, split, _lib.FLAG_PHASE2)
+    for got in (whole, split):
+        assert torch.equal(got[0], ref[0])
+        for u, v in zip(got[1:], ref[1:]):
+            assert float((u - v).abs().max()) <= 1e-5 * float(v.abs().max())
