@@ -9,56 +9,29 @@ import torch
 
 from flash_gmm import _lib, data, diag_estep_into, flash_gmm_estep_diag
 from oracle import gmm_oracle as O
-from parity import assert_close_stats, assert_dense_agrees
+from parity import assert_dense_agrees
+from routes import SCREEN
+from screened import KEYS, call, check, listed, paired, separated
 
 pytestmark = pytest.mark.gpu
-KEYS = ("X", "mu", "log_sigma_sq", "log_pi")
-
-
-def call(inp, dev, **kw):
-    args = [inp[k].to(dev) for k in KEYS]
-    N, D = args[0].shape
-    K = args[1].shape[0]
-    out = [torch.full((N,), math.nan, device=dev), torch.empty(K, device=dev), torch.empty(K, D, device=dev),
-           torch.empty(K, D, device=dev)]
-    diag_estep_into(*args, *out, **kw)
-    torch.cuda.synchronize()
-    return out
-
-
-def check(inp, dev, what):
-    got = call(inp, dev)
-    assert_dense_agrees(got, call(inp, dev, dense=True), bitwise=False)
-    again = call(inp, dev)
-    assert all(torch.equal(u, v) for u, v in zip(got, again)), f"{what}: not deterministic"
-    assert_close_stats(got, O.estep_diag(*[inp[k] for k in KEYS]), what)
-    return got
-
-
-def paired(N, K, D, seed, share):
-    """Clustered rows, a share of the clusters in close pairs half the components apart
-    (so in two blocks): their rows are near both."""
-    inp = data.diag_clustered(N, K, D, seed=seed)
-    g = torch.Generator().manual_seed(seed)
-    n = int(K // 2 * share)
-    inp["mu"][K // 2:K // 2 + n] = inp["mu"][:n] + 0.1 * torch.randn(n, D, generator=g)
-    inp["log_sigma_sq"][K // 2:K // 2 + n] = inp["log_sigma_sq"][:n]
-    return inp
 
 
 # Widths 32 .. 128 (one and two blocks per stage), a last block of 1 and of 32 components, a
 # last tile of 1 row, D that is no multiple of 4, an odd number of blocks.
-@pytest.mark.parametrize("N,K,D", [(42_017, 1024, 96), (33_001, 993, 125), (70_017, 545, 61), (66_001, 2048, 31)])
+@pytest.mark.parametrize("N,K,D", [(42_017, 1024, 96), (40_513, 1025, 90), (33_001, 993, 125), (111_201, 545, 61),
+                                   (66_001, 2048, 31)])
 def test_screened_sizes(N, K, D, gpu_device):
-    print(f"diag screen N={N} K={K} D={D}", flush=True)
-    check(data.diag_clustered(N, K, D, seed=K % 13), gpu_device, f"diag screen N={N} K={K} D={D}")
+    inp = separated("diag", N, K, D, K % 13) if D < 40 else data.diag_clustered(N, K, D, seed=K % 13)
+    check("diag", inp, gpu_device, f"diag screen N={N} K={K} D={D}", O.estep_diag)
 
 
-@pytest.mark.parametrize("share", [0.02, 0.6])
-def test_rows_near_two_blocks(share, gpu_device):
+@pytest.mark.parametrize("share,many", [(0.02, False), (0.4, True)])
+def test_rows_near_two_blocks(share, many, gpu_device):
     """The listed rows: few (one tile per workgroup) and many (128 rows per workgroup)."""
-    print(f"diag screen paired {share}", flush=True)
-    check(paired(45_009, 1024, 96, 3, share), gpu_device, f"diag paired {share}")
+    inp = paired("diag", 45_009, 1024, 96, 3, share)
+    n, few = listed("diag", inp, gpu_device)
+    assert n > 0 and (n > few) == many, f"{n} rows listed, a short list holds {few}"
+    check("diag", inp, gpu_device, f"diag screen paired {share}", O.estep_diag)
 
 
 def test_faint_and_special_components(gpu_device):
@@ -72,7 +45,7 @@ def test_faint_and_special_components(gpu_device):
     inp["log_sigma_sq"][700:740] = ls
     inp["log_pi"][300:310] = -math.inf
     print("diag screen faint", flush=True)
-    got, dense = call(inp, dev), call(inp, dev, dense=True)
+    got, dense = call("diag", inp, dev, expect=SCREEN), call("diag", inp, dev, dense=True)
     assert_dense_agrees(got, dense, bitwise=False)
     assert (got[1][300:310] == 0).all()
     small = (dense[1] > 1e-30) & (dense[1] < 1e-4)
@@ -85,7 +58,7 @@ def test_faint_and_special_components(gpu_device):
     inp["X"][30_000, 95] = math.inf
     inp["X"][44_999] = 1e18
     print("diag screen special rows", flush=True)
-    got, dense = call(inp, dev), call(inp, dev, dense=True)
+    got, dense = call("diag", inp, dev, expect=SCREEN), call("diag", inp, dev, dense=True)
     assert torch.equal(got[0].isnan(), dense[0].isnan())
     fin = ~dense[0].isnan()
     assert torch.equal(got[0][fin], dense[0][fin])
@@ -97,8 +70,8 @@ def test_phase_split_strided_rows_and_lean_workspace(gpu_device):
     results.  A workspace too small for the screening: the exact pass 1, the same logZ."""
     dev = gpu_device
     N, K, D = 70_009, 1024, 60
-    inp = paired(N, K, D, 4, 0.1)
-    one = call(inp, dev)
+    inp = paired("diag", N, K, D, 4, 0.1)
+    one = call("diag", inp, dev, expect=SCREEN)
     L = _lib.lib()
     ws = torch.empty(L.fgmm_diag_workspace_bytes(N, K, D), dtype=torch.uint8, device=dev)
     args = [inp[k].to(dev) for k in KEYS]

@@ -6,28 +6,18 @@ import math
 import pytest
 import torch
 
-from flash_gmm import data, diag_estep_into, iso_estep_into
+from flash_gmm import data
 from parity import assert_dense_agrees
+from routes import SCREEN
+from screened import call
 
 pytestmark = pytest.mark.gpu
 LOG2_E = math.log2(math.e)
-KEYS = ("X", "mu", "log_sigma_sq", "log_pi")
-
-
-def call(model, inp, dev, **kw):
-    args = [inp[k].to(dev) for k in KEYS]
-    N, D = args[0].shape
-    K = args[1].shape[0]
-    out = [torch.full((N,), math.nan, device=dev), torch.empty(K, device=dev), torch.empty(K, D, device=dev),
-           torch.empty(K, device=dev) if model == "iso" else torch.empty(K, D, device=dev)]
-    (iso_estep_into if model == "iso" else diag_estep_into)(*args, *out, **kw)
-    torch.cuda.synchronize()
-    return out
 
 
 def check(model, inp, dev, what):
     print(what, flush=True)
-    got, dense = call(model, inp, dev), call(model, inp, dev, dense=True)
+    got, dense = call(model, inp, dev, expect=SCREEN), call(model, inp, dev, dense=True)
     bad = (got[0] != dense[0]).nonzero().flatten()
     assert bad.numel() == 0, f"{what}: logZ of rows {bad[:8].tolist()}: {got[0][bad[:8]]} not {dense[0][bad[:8]]}"
     assert_dense_agrees(got[:2], dense[:2], bitwise=False)
