@@ -404,18 +404,6 @@ __device__ __forceinline__ double strided_sum(const float* __restrict__ p, int n
   return s;
 }
 
-// The same sum spread over the 64 lanes of a wave (for large n): lane l adds
-// p[l], p[l + 64], ... in order, then a fixed xor butterfly combines the lanes.
-// Deterministic; every lane returns the total.
-__device__ __forceinline__ double wave_strided_sum(const float* __restrict__ p, int n, int64_t stride,
-                                                   int lane) {
-  double s = 0.0;
-  for (int i = lane; i < n; i += 64) s += (double)p[(int64_t)i * stride];
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-  return s;
-}
-
 // ---------------------------------------------------------------------------
 // Stored log-joint.  Pass 1 can keep the fp32 log-joint (log2 units) of every
 // (32-row tile, 32-component block) pair in the workspace, so that pass 2 reads
@@ -778,7 +766,7 @@ constexpr int64_t kMaxBufLdx = (int64_t)1 << 20;
 // must stay within the 2^31 - 1 grid limit.  Larger data sets stream in chunks.
 constexpr int64_t kMaxRows = (int64_t)1 << 37;
 
-// Partial counts from which the reductions use one wave per output element.
+// Partial counts from which the reductions put 16 threads on an output element instead of 4.
 constexpr int kWideReduce = 128;
 
 __host__ __device__ constexpr int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -125,14 +125,17 @@ __host__ __device__ constexpr int full_list_spill(int DP, int K) {
 // accumulators and split operands of one component fit a wave's registers).
 __host__ __device__ constexpr bool flj_applies(int DP) { return DP <= 64; }
 
-// The screened pass 1 (see full_screen): calls with the probe, up to kScreenMaxK
-// components (the probe's estimate is in pairs: fewer than 16 components leave too little
-// to screen out) and at least kScreenMinWork (32-row tile, component, 32-coordinate block)
-// steps, below which its launches cost what it saves.  In the stored branch's log-joint
-// space: the bounds, 2 bytes a pair, then per tile a pool of screen_cap doubles (about a
-// quarter of its pairs) for the needed pairs' fp64 log-joint.
-constexpr int kScreenMinK = 16;
-constexpr int64_t kScreenMinWork = 40000;
+// The screened pass 1 (see full_screen): calls with the probe (D <= 64, K <= kProbeMaxKB) of
+// at least 16 components (with 8 it gains 10% at best) and at least kFullScreenMinWork (32-row
+// tile, component, 32-coordinate block) steps: where the probe leaves them to the others, its
+// kernels that return cost 5 to 10 us, 2 to 7% at 39,000 steps (N(0, I) rows without and with,
+// D=64 K=256 809 and 813 us, K=32 180 and 186, K=16 143 and 150, D=32 K=16 112 and 121).
+// Separated clusters there, without and with: 829 and 396, 171 and 134, 137 and 126, 102 and
+// 104.  In the stored branch's log-joint space: the bounds, 2 bytes a pair, then per tile a
+// pool of screen_cap doubles (about a quarter of its pairs) for the needed pairs' fp64
+// log-joint.
+constexpr int kFullScreenMinK = 16;
+constexpr int64_t kFullScreenMinWork = 40000;
 constexpr int kScreenTpw = 4;      // 32-row tiles per wave
 constexpr int kScreenPieces = 16;  // 1 KB operand pieces per LDS stage
 constexpr int kScreenConsts = 16;  // floats after a component's -b: c (up, down), the error's A, F, B
@@ -215,7 +218,7 @@ FullPlan make_plan(int64_t N, int64_t K, int64_t D, bool allow_lj = false, bool 
   p.autolj = p.need && auto_lj && flj_applies(p.DP) && N > 0 && K <= kProbeMaxKB &&
              full_lj_bytes(N, p.KP) <= kMaxLjBytes;
   p.screen_cap = 0;
-  if (p.autolj && K >= kScreenMinK && cdiv(N, 32) * K * p.NMB >= kScreenMinWork &&
+  if (p.autolj && K >= kFullScreenMinK && cdiv(N, 32) * K * p.NMB >= kFullScreenMinWork &&
       full_lj_bytes(N, p.KP) > screen_ub_bytes(N, p.KP))
     p.screen_cap = (int)std::min<size_t>(
         65535, (full_lj_bytes(N, p.KP) - screen_ub_bytes(N, p.KP)) / sizeof(double) / (size_t)cdiv(N, 32));
@@ -726,7 +729,7 @@ void full_lse_x6(const float* __restrict__ X, int64_t ldx, int64_t N, int D, con
 // kLjNeedGap = 160 margin) into `lls` ([tile][KP][32] floats).  full_probe_count:
 // per row, the components with ll >= M - kLjNeedGap (M the row's largest) are
 // counted, an estimate of the pairs pass 1 marks as needed; the tile's count is
-// written, and the kernels that need the choice sum the counts (probe_selects).
+// written, and the kernels that need the choice sum the counts (probe_mode).
 // ---------------------------------------------------------------------------
 constexpr int kProbeWaves = 16;
 constexpr int kProbeSplit = 4;
@@ -1649,9 +1652,13 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // with the exact pass 1 over all).  Bound: matrix steps and the squares' VALU, about equal.
 // The steps of the blocks above L's diagonal (2 of 8 at D = 64) are left out: a component
 // with a nonzero there has A = infinity, so nothing of it is screened.
-// N=250K K=256 D=64, clustered: the drop-in call 2.641 -> 0.618 ms (0.705 with all eight
-// steps and a log-joint of every pair; exact pass 1 2.45 ms;
-// traced: full_screen 0.565, the gathered log-joint 0.075, full_need_lse 0.020).
+// N=250K K=256 D=64, clustered: the drop-in call 2.641 -> 0.635 ms (0.705 with all eight
+// steps and a log-joint of every pair); traced: full_screen 0.495, the gathered log-joint
+// 0.082, full_need_lse 0.021 (exact pass 1 2.45).  Counters: matrix steps 38% and other VALU
+// 45% of the SIMDs' cycles.
+// The eighth of the sampled pairs up to which the probe selects it, with means pulled
+// together, screened and exact: 0.85 and 3.96 ms, 4.4 and 5.6 (nearer), 10.1 and 7.4 (nearer
+// still; the probe leaves it to the exact pass 1).
 // ---------------------------------------------------------------------------
 template <int DP>
 __global__ __attribute__((amdgpu_flat_work_group_size(kThreads, kThreads), amdgpu_waves_per_eu(2, 2)))

@@ -1093,15 +1093,15 @@ void iso_lse_pipe(const float* __restrict__ X, int64_t ldx, int64_t N, int D,
 }
 
 // ---------------------------------------------------------------------------
-// The probe of FGMM_FLAG_STORE_LOGJOINT_AUTO (up to D = 128): one workgroup per
-// sampled 32-row tile; its waves take the component blocks in turn and form each
+// The probe of FGMM_FLAG_STORE_LOGJOINT_AUTO and of the screened pass 1 (up to D = 128): one
+// workgroup per sampled 32-row tile; its waves take the component blocks in turn and form each
 // row's block maximum R of the log-joint in LDS.  An estimate suffices here, so
 // the contraction keeps two of pass 1's seven steps per 16-dimension chunk (the
 // centring step and x1 mu1: an error of a fraction of a log2 unit against the
 // kLjNeedGap = 160 margin).  Then, per row, the blocks with R >= M - kLjNeedGap (M
 // the row's largest R) are counted: an estimate of the pairs pass 1 will mark as
-// needed, since logZ2 >= M.  The tile's count is written; no atomics: the kernels
-// that need the choice sum the counts themselves (probe_selects).
+// needed, since logZ2 >= M; and the rows the screening would find near several blocks.  The
+// last workgroup makes the call's choice (probe_finish).
 // ---------------------------------------------------------------------------
 constexpr int kProbeWaves = 16;
 template <int DP>

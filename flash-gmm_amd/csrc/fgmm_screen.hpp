@@ -32,11 +32,18 @@ __host__ __device__ constexpr size_t screen_lds_bytes(int DP, bool DIAG, int KB)
   const size_t b = screen_stage_bytes(DP, DIAG) + (size_t)kScreenWaves * 64 * round_up(KB, 8) * 2;
   return screen_stage_bytes(DP, DIAG) + (a > b ? a : b);
 }
-// Calls whose pass 1 is worth screening: at least kScreenMinWork (32-row tile, block,
-// chunk) steps, below which the further launches cost more than the screening saves
-// (about 100 us of exact pass 1), and at least 4 blocks (with one near block a row,
-// screening B blocks leaves 1/B of the exact contraction); two workgroups per compute
-// unit.
+// Calls that may screen: at least 4 blocks (with one near block a row, screening B blocks
+// leaves 1/B of the exact contraction), two workgroups per compute unit (the rows' block
+// bounds in LDS: at most 2816 components at D = 128 and 1792 diagonal ones at D = 96; beyond,
+// the exact pass 1 runs) and at least kScreenMinWork (32-row tile, block, chunk) steps.
+// Calls that the probe then leaves to the exact pass 1 pay for the probe and two kernels that
+// return, 10 to 22 us, where they had no probe before (the default plan without the automatic
+// stored branch); N(0, I) rows, K=1024, without and with: at 500,000 steps 305 and 309 us
+// (D=128), 345 and 360 us (D=96), 324 and 335 us (D=64), at 250,000 steps 201 and 222, 203
+// and 216, 187 and 198 us, at 2,000,000 at most 2% more.  Separated clusters gain at once: at
+// 250,000 steps 136 -> 92 us, 130 -> 84 us and 153 -> 99 us, at 500,000 167 -> 101, 192 ->
+// 126 and 258 -> 113 us.  So the line lies where the first has become small, well above the
+// crossover of the second (between 60,000 and 125,000 steps).
 constexpr int64_t kScreenMinWork = 500000;
 constexpr int64_t kMaxScreenLdx = (int64_t)4 << 20;   // 64 rows within 32-bit buffer offsets
 __host__ inline bool use_screen(int64_t N, int DP, bool DIAG, int KB) {
@@ -56,11 +63,13 @@ __host__ inline int64_t few_rows(int64_t grid) {
 __host__ constexpr size_t screen_word_bytes(int KB, size_t word) { return ((size_t)KB * word + 31) / 32; }
 
 // The screened pass 1 tells near pairs from faint ones.  A pair is near unless its
-// responsibility r provably has r, r ||x||, r ||x||^2 <= 2^-kNearGap; the faint pairs of
-// a component with Nk >= kNearNk then change none of its sums by a rounding (at most
-// N 2^-72 <= 2^-41, against 2^-24 of 2^-10), and a row's terms outside its near blocks
-// change no bit of its fp32 log-sum-exp (at most K 2^-72 of it).  So pass 2 takes the
-// near pairs, and then the faint ones of those blocks that hold a component with less.
+// responsibility r provably has r, r ||x||, r ||x||^2 <= 2^-kNearGap.  Pass 2 takes the near
+// pairs, and then the faint ones of those blocks that hold a component with Nk < kNearNk.
+// What it leaves out, the faint pairs of the other components, changes their Nk by at most
+// N 2^-72 in absolute value, less than a rounding (N 2^-72 <= 2^-41, against 2^-24 of 2^-10),
+// and their other sums by at most N 2^-72 each: an element of mu_acc that is 0 in the near
+// rows, or whose terms cancel, loses terms of that size.  A row's terms outside its near
+// blocks change no bit of its fp32 log-sum-exp (at most K 2^-72 of it).
 constexpr float kNearGap = 72.0f;
 constexpr float kNearNk = 0x1p-10f;
 // Pass 2 marks, in one word per block (`alive`, zeroed by the prologue), the components
@@ -123,7 +132,13 @@ enum CallMode { kModeDefault = 0, kModeStored = 1, kModeScreen = 2 };
 __device__ __forceinline__ int call_mode(const int* __restrict__ sel) { return sel ? *sel : kModeDefault; }
 // What the probe chooses from: up to max_multi sampled rows near several blocks, the
 // screened pass 1 (-1: never); else, from min_pairs needed pairs on, the stored branch if
-// the call has one.
+// the call has one.  The callers' max_multi is half of the rows.  Clustered rows with that
+// share on the list, screened and exact, us: N=1M K=1024 D=128 2744 and 3217 (0.50 listed),
+// N=500K D=96 1013 and 1414 (0.49), N=400K K=300 D=50 399 and 508 (0.53), diagonal N=1M
+// K=1024 D=96 3123 and 5257 (0.58), N=500K D=64 906 and 2032 (0.47); the two cross at 0.6
+// (isotropic D=128) to 0.95 (diagonal D=64).  Not so where, besides, a few components hold
+// many of the rows: the gathering pass 2 takes longer for such a block with logZ formed in it
+// (N=1M K=1024 D=128, half of the clusters without a component of their own: 3756 and 2971).
 struct ProbeRule {
   int64_t max_multi, min_pairs;
   int stored;
@@ -251,13 +266,13 @@ __device__ __forceinline__ void probe_finish(const float* rmax, const float* rer
 // rest go on a list, which the exact pass 1 then runs.
 //
 // Bound: matrix steps and VALU, which mostly add up on a SIMD: at D = 128, 9 matrix
-// steps (288 cycles) and about 25 VALU instructions per (32 rows, block); matrix steps
-// alone 51% of its cycles.  Each operand read from LDS serves two 32-row tiles.  Rows
-// are read in whole lines and transposed through LDS (the exact pass reads 16-byte
-// pieces of 32 rows per instruction, which at this kernel's length would bound it).
-// N=1M K=1024 D=128 clustered: 0.27 ms, and pass 1 and 2 with it 0.55 ms instead of
-// 1.73 ms (drop-in call 1.75 -> 0.55 ms); N=400K K=300 D=50: call 0.51 -> 0.27 ms.
-// Diagonal (13 steps at D = 96): N=1M K=1024 D=96 clustered 0.39 ms, call 2.86 -> 0.72 ms.
+// steps (288 cycles) and 31 VALU instructions per (32 rows, block), 58% and 25% of the SIMDs'
+// cycles (diagonal, D = 96: 13 and 36, 56% and 19%).  Each operand read from LDS serves two
+// 32-row tiles.  Rows are read in whole lines and transposed through LDS (the exact pass
+// reads 16-byte pieces of 32 rows per instruction, which at this kernel's length would bound
+// it).  N=1M K=1024 D=128 clustered: 0.27 ms, drop-in call 1.75 -> 0.57 ms; N=400K K=300
+// D=50: call 0.51 -> 0.28 ms; diagonal N=1M K=1024 D=96 clustered 0.38 ms, call 2.86 ->
+// 0.69 ms.
 // ---------------------------------------------------------------------------
 template <int DP, bool DIAG>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kScreenWaves, 64 * kScreenWaves),

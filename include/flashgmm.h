@@ -165,7 +165,9 @@ int fgmm_iso_estep_f32(const float *X, int64_t ldx, int64_t N, int64_t D,
 /* deferred loading off, HIP_ENABLE_DEFERRED_LOADING=0, every code object is   */
 /* loaded with the library), and it is held until the process ends.  A call   */
 /* whose workspace (fgmm_iso_workspace_bytes_ex with the same flags) exceeds   */
-/* it (above about 1.5M rows at K=1024, D=128) runs as consecutive row chunks  */
+/* it runs on a smaller plan where that fits (logZ the same, the statistics'   */
+/* float32 sums in other groupings).  Beyond (above about 1.5M rows at K=1024, */
+/* D=128) it runs as consecutive row chunks                                    */
 /* on the array, each after the first adding its statistics to the outputs:   */
 /* logZ is the one-call result per row, the statistics round once per chunk.   */
 /* Such a call with FGMM_FLAG_PHASE1 or PHASE2, or one where not even 256 rows */
