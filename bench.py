@@ -61,8 +61,24 @@ WORKLOADS = {
 # --copy-calibration 512: FETCH_SIZE x2.0, WRITE_SIZE x1.0).  Per kernel of one step:
 # (FETCH_SIZE KiB, WRITE_SIZE KiB); the commands and tables are in profiles/.
 TRAFFIC_KIB = {
-    # (workload, plan, precision): {kernel: (fetch KiB, write KiB)}; "phase1" names pass 1's
-    # The screened calls (clustered data, SCREENED) are not listed: their pass 1 is several kernels.
+    # (workload, plan, precision): {kernel: (fetch KiB, write KiB)}; "phase1" names pass 1's, the
+    # screening where the drop-in call takes the screened pass 1 (clustered data, SCREENED: on
+    # these the screening lists no rows; counted over the drop-in call alone, the kernels that
+    # return left out).
+    ("iso_n1m_k1024_d128", "default", "fp32"): {
+        "phase1": "screen_pairs<128, 0>",
+        "iso_prep": (315, 1_394), "iso_store_probe<128>": (2_682, 6), "screen_pairs<128, 0>": (256_900, 7_812),
+        "iso_accum_gather<128>": (266_800, 64_750), "iso_reduce": (16_670, 520)},
+    ("diag_n1m_k1024_d96", "default", "fp32"): {
+        "phase1": "screen_pairs<96, 1>",
+        "diag_x6_prep": (447, 1_962), "diag_store_probe<96>": (3_553, 6), "screen_pairs<96, 1>": (191_200, 7_812),
+        "diag_accum_gather<96, 1>": (202_100, 64_720), "diag_reduce": (25_830, 796)},
+    ("full_n250k_k256_d64", "default", "fp32"): {
+        "phase1": "full_screen<64>",
+        "full_x6_prep": (2_151, 8_400), "full_probe_ll<64>": (5_292, 2_048), "full_probe_count": (1_044, 2),
+        "full_screen<64>": (103_000, 140_800), "full_accum_gather<64, 0, 0, 1>": (74_190, 7_651),
+        "full_need_lse": (5_376, 2_930), "full_accum_gather<64, 0, 0, 0>": (68_270, 25_150),
+        "full_reduce_sig": (12_320, 4_096), "full_reduce": (286, 65)},
     # The reference's N(0, I) data: the probe selects the stored branch (pass 1 writes the
     # log-joint, the X parts and the logZ pairs; iso_accum_ljt reads them back).
     ("iso_ref_n1m_k1024_d128", "default", "fp32"): {
