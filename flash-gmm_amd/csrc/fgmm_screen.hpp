@@ -455,8 +455,7 @@ void screen_pairs(const float* __restrict__ X, int64_t ldx, int64_t N, int D, co
 
   // Need words of the two tiles (each lane reads back the bounds it wrote itself), 32
   // blocks at a time, lane c of half g keeping block kb0 + c of tile g.
-  const bool valid = row < N;
-  if (!valid) L = INFINITY;   // a row past N (zeros: finite bounds) gets no bit
+  const uint64_t valid = __builtin_amdgcn_ballot_w64(row < N);   // a row past N gets no bit
   const float near_gap = fminf(kLjNeedGap, kNearGap + 2.0f * log2f(1.0f + nx));   // kLjNeedGap if nx is NaN
   uint64_t once = 0, twice = 0;   // rows with at least one, two near blocks
   const int64_t tile = (row0 >> 5) + g;
@@ -471,8 +470,8 @@ void screen_pairs(const float* __restrict__ X, int64_t ldx, int64_t N, int D, co
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const float u = ub[j] - L;
-        const uint64_t b = __builtin_amdgcn_ballot_w64(!(u < -near_gap));
-        const uint64_t f = __builtin_amdgcn_ballot_w64(!(u < -kLjNeedGap)) & ~b;
+        const uint64_t b = __builtin_amdgcn_ballot_w64(!(u < -near_gap)) & valid;
+        const uint64_t f = __builtin_amdgcn_ballot_w64(!(u < -kLjNeedGap)) & valid & ~b;
         twice |= once & b;
         once |= b;
         if (c == j0 + j) {
@@ -488,7 +487,7 @@ void screen_pairs(const float* __restrict__ X, int64_t ldx, int64_t N, int D, co
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   const uint64_t one = once & ~twice;
-  const uint64_t many = __builtin_amdgcn_ballot_w64(valid) & ~one;
+  const uint64_t many = valid & ~one;
   const unsigned own = g == 0 ? (unsigned)one : (unsigned)(one >> 32);
   for (int kb0 = 0; kb0 < KB; kb0 += 32) {
     const uint2 w = words_l[kb0 * 16 + lane];
