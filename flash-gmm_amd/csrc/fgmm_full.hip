@@ -1646,7 +1646,7 @@ void full_accum_ljt(const float* __restrict__ X, int64_t ldx, int64_t N, int D, 
 // Upper bounds go to `ub` as bf16 ([workgroup][wave][tile pair][component][64 rows], 128
 // bytes a store); once the row's largest lower bound is final each lane reads its own
 // back, counts the needed pairs and leaves each its place in its tile's pool instead.  A tile
-// with more than the pool holds (nine rows of NaN, of whose pairs none can be left out) sets
+// with more than the pool holds (eight rows of NaN, of whose pairs none can be left out) sets
 // its byte after `any_over`: full_lse_x6 runs the tile groups that hold such a byte, the
 // others keep the screening's results (N=250K K=256 D=64, one such tile: 1.61 ms, 3.25 ms
 // with the exact pass 1 over all).  Bound: matrix steps and the squares' VALU, about equal.
